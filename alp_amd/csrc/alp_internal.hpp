@@ -216,6 +216,9 @@ __host__ __device__ __forceinline__ uint64_t dia_pos(uint64_t e0, unsigned w, un
 	return e0 + (uint64_t)q * kSellRows + lane;
 }
 
+// The slices' flags, offsets and masks of the diagonal form (no values); as below
+alp_rc_t dia_detect(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
+                    size_t entries, const uint64_t *off, const uint32_t *idx);
 // Builds D for a sliced ELL of nslices slices with offsets soff; slice s covers
 // rows [srow[s], srow[s+1]) or, with srow null, [64 s, min(64 s + 64, nrows)).
 // Leaves D empty (and returns SUCCESS) when fewer than half the slices qualify.
@@ -226,6 +229,38 @@ alp_rc_t dia_build(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *s
 alp_rc_t dia_refresh(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
                      const uint64_t *off, int value_type, const void *val, const float *val32);
 void dia_free(DiaSlices &D);
+
+// Constant form of a set of diagonal slices: one template for all of them, at most
+// kDiaSlots (column - row offset, value) pairs in storage order, of which every
+// row's entries are an increasing subsequence with the same value bits (a
+// constant-coefficient stencil with its boundaries cut off). A row then needs
+// only its presence mask: the template travels in the kernel's arguments, so a
+// product streams 4 bytes per row of matrix instead of a value per entry (192^3
+// 27-point FP64: 28 MB instead of 1.6 GB), and its x reads depend on no load.
+// Rows fold in storage order as before, so results stay bit-identical.
+struct ConstDia {
+	unsigned w = 0;  // slots of the template; 0: the slices are not in this form
+	int32_t d[kDiaSlots] = {};
+	int32_t dmin = 0, dmax = 0;
+	double v64[kDiaSlots] = {};  // the values (FP64 matrices) and their FP32 copies,
+	float v32[kDiaSlots] = {};   // or the values of an FP32 matrix
+};
+
+// the template as a kernel argument, with values of type V
+template <typename V>
+struct ConstArg {
+	unsigned w;
+	int32_t dmin, dmax;
+	int32_t d[kDiaSlots];
+	V v[kDiaSlots];
+};
+
+// Detects the constant form over rows [row0, row1) in slices [s0, s1) (slice rows
+// as in dia_build) and writes the slices' presence masks (indexed by slice and
+// lane) to mask; C.w stays 0 when some row does not fit. Blocking.
+alp_rc_t const_detect(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
+                      const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask);
+bool const_dia_enabled();
 
 struct Storage {
 	uint64_t *off = nullptr;  // nmajor + 1
@@ -258,6 +293,10 @@ struct Storage {
 	size_t n_slices = 0;
 	size_t sell_entries = 0;
 	DiaSlices dia;                 // diagonal form of the slices that have it
+	// all rows in constant form (cst.w > 0): the template and the rows' masks; the
+	// sliced-ELL and diagonal forms then keep no values
+	ConstDia cst;
+	uint32_t *cmask = nullptr;
 	// rows longer than kLongRow nonzeros, for the CSR-stream path: split into
 	// chunks of kChunk nonzeros that separate blocks fold into partials, then one
 	// thread per long row folds its partials in chunk order (deterministic)

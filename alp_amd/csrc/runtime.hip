@@ -8,6 +8,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <chrono>
 #include <climits>
 #include <cmath>
@@ -414,12 +415,10 @@ alp_rc_t dia_refresh(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t 
 	return ALP_SUCCESS;
 }
 
-alp_rc_t dia_build(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
-                   size_t entries, const uint64_t *off, const uint32_t *idx, int value_type, const void *val,
-                   const float *val32) {
+alp_rc_t dia_detect(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
+                    size_t entries, const uint64_t *off, const uint32_t *idx) {
 	dia_free(D);
 	if (nslices == 0 || entries == 0) return ALP_SUCCESS;
-	const size_t vs = value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
 	unsigned long long *d_count = nullptr;
 	DiaSlices T;
 	if (hipMalloc(&T.flag, nslices) != hipSuccess || hipMalloc(&T.col, sizeof(int32_t) * kDiaSlots * nslices) != hipSuccess ||
@@ -446,18 +445,218 @@ alp_rc_t dia_build(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *s
 		dia_free(T);
 		return rc;
 	}
-	if ((vs && hipMalloc(&T.val, vs * entries) != hipSuccess) ||
-	    (val32 && hipMalloc(&T.val32, sizeof(float) * entries) != hipSuccess)) {
+	T.n_dia = cnt;
+	D = T;
+	return ALP_SUCCESS;
+}
+
+// value arrays of D (val, and val32 when the matrix has an FP32 copy), allocated
+// where missing, then filled; without memory D is dropped
+static alp_rc_t dia_values(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
+                           size_t entries, const uint64_t *off, int value_type, const void *val, const float *val32) {
+	if (!D.flag) return ALP_SUCCESS;
+	const size_t vs = value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
+	if ((vs && !D.val && hipMalloc(&D.val, vs * entries) != hipSuccess) ||
+	    (val32 && !D.val32 && hipMalloc(&D.val32, sizeof(float) * entries) != hipSuccess)) {
 		(void)hipGetLastError();
-		dia_free(T);
+		dia_free(D);
 		return ALP_SUCCESS;
 	}
-	T.n_dia = cnt;
-	if ((rc = dia_refresh(T, nslices, nrows, srow, soff, off, value_type, val, val32)) != ALP_SUCCESS) {
-		dia_free(T);
-		return rc;
+	const alp_rc_t rc = dia_refresh(D, nslices, nrows, srow, soff, off, value_type, val, val32);
+	if (rc != ALP_SUCCESS) dia_free(D);
+	return rc;
+}
+
+alp_rc_t dia_build(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
+                   size_t entries, const uint64_t *off, const uint32_t *idx, int value_type, const void *val,
+                   const float *val32) {
+	ALP_TRY(dia_detect(D, nslices, nrows, srow, soff, entries, off, idx));
+	return dia_values(D, nslices, nrows, srow, soff, entries, off, value_type, val, val32);
+}
+
+// ---- constant form ----------------------------------------------------------------
+
+// *best = min(*best, first row in [row0, row1) with the most entries of that range):
+// per-block (length, row) maxima, one 64-bit atomic per block (longest first, then
+// the lowest row)
+__global__ __launch_bounds__(kBlock) void k_const_longest(size_t row0, size_t row1, const uint64_t *off,
+                                                         unsigned long long *best) {
+	__shared__ unsigned long long s_best;
+	if (threadIdx.x == 0) s_best = 0;
+	__syncthreads();
+	unsigned long long b = 0;
+	grid_for_each<1>(row1 - row0, [&](size_t i) {
+		const uint64_t len = off[row0 + i + 1] - off[row0 + i];
+		const unsigned long long k = (unsigned long long)(len < 0xFFFFull ? len : 0xFFFFull) << 48 |
+		                             (0xFFFFFFFFFFFFull - (unsigned long long)i);
+		b = k > b ? k : b;
+	});
+	atomicMax(&s_best, b);
+	__syncthreads();
+	if (threadIdx.x == 0) atomicMax(best, s_best);
+}
+
+// the candidate template: the entries of row r (V: the value type; char for patterns)
+struct ConstTemplate {
+	unsigned w, pad;
+	long long d[kDiaSlots];
+	unsigned long long bits[kDiaSlots];
+};
+
+template <typename V>
+__global__ void k_const_template(size_t row0, const uint64_t *off, const uint32_t *idx, const V *val,
+                                 const unsigned long long *best, ConstTemplate *T) {
+	const unsigned q = threadIdx.x;
+	const size_t r = row0 + (size_t)(0xFFFFFFFFFFFFull - (*best & 0xFFFFFFFFFFFFull));
+	const uint64_t b = off[r];
+	const unsigned w = (unsigned)(off[r + 1] - b);
+	if (q == 0) T->w = w;
+	if (q < w && q < kDiaSlots) {
+		T->d[q] = (long long)idx[b + q] - (long long)r;
+		unsigned long long u = 0;
+		const V v = val[b + q];
+		__builtin_memcpy(&u, &v, sizeof(V));
+		T->bits[q] = u;
 	}
-	D = T;
+}
+
+// One wavefront per slice: every row matches its (offset, value) pairs greedily
+// against the template's in order. The template's offsets are distinct (one row
+// stores a column once), so a row that is a subsequence is matched completely.
+// *bad is set when some row is not (it counts the slices seen before the rest left).
+template <typename V>
+__global__ __launch_bounds__(kBlock) void k_const_match(size_t s0, size_t s1, size_t row1, const uint32_t *srow,
+                                                       const uint64_t *off, const uint32_t *idx, const V *val,
+                                                       const ConstTemplate *T, uint32_t *mask, unsigned *bad) {
+	const size_t sl = s0 + (size_t)blockIdx.x * (kBlock / kSellRows) + threadIdx.x / kSellRows;
+	if (sl >= s1 || *bad) return;  // whole wavefronts leave together; a slice that failed decides
+	const unsigned lane = threadIdx.x % kSellRows;
+	size_t r0, r1;
+	dia_rows(sl, row1, srow, &r0, &r1);
+	const size_t r = r0 + lane;
+	const bool act = r < r1;
+	const uint64_t b = act ? off[r] : 0;
+	const uint64_t len = act ? off[r + 1] - b : 0;
+	const unsigned w = T->w;
+	uint32_t bits = 0;
+	unsigned j = 0;
+	for (unsigned q = 0; q < w; ++q) {
+		if (j >= len) break;
+		if ((long long)idx[b + j] - (long long)r != T->d[q]) continue;
+		unsigned long long u = 0;
+		const V v = val[b + j];
+		__builtin_memcpy(&u, &v, sizeof(V));
+		if (u == T->bits[q]) {
+			bits |= 1u << q;
+			++j;
+		}
+	}
+	mask[sl * kSellRows + lane] = bits;
+	if (__ballot(j != len) != 0 && lane == 0) atomicAdd(bad, 1u);
+}
+
+// ALP_HIP_CONST_DIA=0 keeps the diagonal slices' own values (diagnostics, tests)
+bool const_dia_enabled() {
+	const char *e = std::getenv("ALP_HIP_CONST_DIA");
+	return !(e && e[0] == '0');
+}
+
+template <typename V>
+static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
+                               const uint64_t *off, const uint32_t *idx, const V *val, uint32_t *mask) {
+	struct Work {
+		unsigned long long best;
+		unsigned bad, pad;
+		ConstTemplate t;
+	} h{}, *d = nullptr;
+	ALP_HIP_TRY(hipMalloc(&d, sizeof(Work)));
+	struct Free {
+		void *p;
+		~Free() { hipFree(p); }
+	} guard{d};
+	hipStream_t s = stream();
+	ALP_HIP_TRY(hipMemsetAsync(d, 0, sizeof(Work), s));
+	hipLaunchKernelGGL(k_const_longest, dim3(stream_grid(row1 - row0)), dim3(kBlock), 0, s, row0, row1, off, &d->best);
+	hipLaunchKernelGGL(k_const_template<V>, dim3(1), dim3(kDiaSlots), 0, s, row0, off, idx, val,
+	                   (const unsigned long long *)&d->best, &d->t);
+	ALP_LAUNCH_CHECK();
+	ALP_HIP_TRY(copy_sync(&h, d, sizeof(Work), hipMemcpyDeviceToHost));
+	if (h.t.w == 0 || h.t.w > kDiaSlots) return ALP_SUCCESS;
+	for (unsigned q = 0; q < h.t.w; ++q) {
+		if (h.t.d[q] < INT32_MIN || h.t.d[q] > INT32_MAX) return ALP_SUCCESS;
+		for (unsigned p = 0; p < q; ++p)
+			if (h.t.d[p] == h.t.d[q]) return ALP_SUCCESS;  // a column stored twice: the diagonal form keeps it
+	}
+	const size_t per = kBlock / kSellRows;
+	hipLaunchKernelGGL(k_const_match<V>, dim3((s1 - s0 + per - 1) / per), dim3(kBlock), 0, s, s0, s1, row1, srow, off,
+	                   idx, val, (const ConstTemplate *)&d->t, mask, &d->bad);
+	ALP_LAUNCH_CHECK();
+	ALP_HIP_TRY(copy_sync(&h.bad, &d->bad, sizeof(unsigned), hipMemcpyDeviceToHost));
+	if (h.bad) return ALP_SUCCESS;
+	C.w = h.t.w;
+	C.dmin = INT32_MAX;
+	C.dmax = INT32_MIN;
+	for (unsigned q = 0; q < C.w; ++q) {
+		V v;
+		__builtin_memcpy(&v, &h.t.bits[q], sizeof(V));
+		C.d[q] = (int32_t)h.t.d[q];
+		C.v64[q] = (double)v;
+		C.v32[q] = (float)v;
+		C.dmin = std::min(C.dmin, C.d[q]);
+		C.dmax = std::max(C.dmax, C.d[q]);
+	}
+	return ALP_SUCCESS;
+}
+
+alp_rc_t const_detect(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
+                      const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask) {
+	C = ConstDia();
+	if (row1 <= row0 || s1 <= s0 || !val) return ALP_SUCCESS;
+	if (value_type == ALP_VAL_F64)
+		return const_detect_t<double>(C, row0, row1, s0, s1, srow, off, idx, (const double *)val, mask);
+	if (value_type == ALP_VAL_F32)
+		return const_detect_t<float>(C, row0, row1, s0, s1, srow, off, idx, (const float *)val, mask);
+	return ALP_SUCCESS;
+}
+
+static bool keep_sell() {
+	const char *keep = std::getenv("ALP_HIP_KEEP_SELL");  // "1": keep them (tests of the sliced-ELL path)
+	return keep && keep[0] == '1';
+}
+
+// Tries the constant form on S's rows; frees the mask array when it does not hold.
+static alp_rc_t storage_const(Storage &S, int value_type) {
+	S.cst = ConstDia();
+	if (S.max_len == 0 || S.max_len > kDiaSlots || value_type == ALP_VAL_PATTERN || !const_dia_enabled()) return ALP_SUCCESS;
+	const size_t ns = (S.nmajor + kSellRows - 1) / kSellRows;
+	if (!S.cmask && hipMalloc(&S.cmask, sizeof(uint32_t) * ns * kSellRows) != hipSuccess) {
+		(void)hipGetLastError();
+		S.cmask = nullptr;  // no memory for the masks: the other forms
+		return ALP_SUCCESS;
+	}
+	const alp_rc_t rc = const_detect(S.cst, 0, S.nmajor, 0, ns, nullptr, S.off, S.idx, value_type, S.val, S.cmask);
+	if (rc != ALP_SUCCESS || !S.cst.w) {
+		hipFree(S.cmask);
+		S.cmask = nullptr;
+	}
+	return rc;
+}
+
+// S's sliced-ELL arrays (those it has) from the CRS
+static alp_rc_t sell_fill(Storage &S, int value_type) {
+	if (!S.sell_idx) return ALP_SUCCESS;  // diagonal slices only
+	const unsigned g = stream_grid(S.n_slices * kSellRows);
+	if (value_type == ALP_VAL_F32)
+		hipLaunchKernelGGL(k_sell_fill<float>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, S.n_slices,
+		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const float *)S.val,
+		                   (const float *)S.val32, (const uint64_t *)S.sell_off, S.sell_idx, (float *)S.sell_val,
+		                   S.sell_val32);
+	else
+		hipLaunchKernelGGL(k_sell_fill<double>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, S.n_slices,
+		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const double *)S.val,
+		                   (const float *)S.val32, (const uint64_t *)S.sell_off, S.sell_idx, (double *)S.sell_val,
+		                   S.sell_val32);
+	ALP_LAUNCH_CHECK();
 	return ALP_SUCCESS;
 }
 
@@ -492,72 +691,73 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 		hipFree(soff);
 		return ALP_SUCCESS;
 	}
-	const size_t vs = value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
-	uint32_t *sidx = nullptr;
-	void *sval = nullptr;
-	float *sval32 = nullptr;
-	if (hipMalloc(&sidx, sizeof(uint32_t) * total) != hipSuccess ||
-	    (vs && hipMalloc(&sval, vs * total) != hipSuccess) ||
-	    (S.val32 && hipMalloc(&sval32, sizeof(float) * total) != hipSuccess)) {
-		// not enough memory for the copy: keep the CRS kernels only
-		(void)hipGetLastError();
-		if (sidx) hipFree(sidx);
-		if (sval) hipFree(sval);
-		if (sval32) hipFree(sval32);
+	DiaSlices dia;
+	alp_rc_t rc = dia_detect(dia, ns, S.nmajor, nullptr, soff, total, S.off, S.idx);
+	if (rc == ALP_SUCCESS) rc = storage_const(S, value_type);
+	if (rc != ALP_SUCCESS) {
 		hipFree(soff);
-		return ALP_SUCCESS;
+		dia_free(dia);
+		return rc;
 	}
-	const unsigned g = stream_grid(ns * kSellRows);
-	if (value_type == ALP_VAL_F32)
-		hipLaunchKernelGGL(k_sell_fill<float>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, ns,
-		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const float *)S.val,
-		                   (const float *)S.val32, (const uint64_t *)soff, sidx, (float *)sval, sval32);
-	else
-		hipLaunchKernelGGL(k_sell_fill<double>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, ns,
-		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const double *)S.val,
-		                   (const float *)S.val32, (const uint64_t *)soff, sidx, (double *)sval, sval32);
-	ALP_LAUNCH_CHECK();
+	// A matrix in constant form reads no values and, when every slice also has the
+	// diagonal form (which the pattern rings then use), no column indices; a
+	// diagonal-only one no sliced-ELL arrays either: only the slice offsets are kept
+	const bool keep = keep_sell(), all_dia = dia.flag && dia.n_dia == ns;
+	if (!all_dia || keep) {
+		const bool values = !S.cst.w || keep;
+		const size_t vs = !values ? 0 : value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
+		uint32_t *sidx = nullptr;
+		void *sval = nullptr;
+		float *sval32 = nullptr;
+		if (hipMalloc(&sidx, sizeof(uint32_t) * total) != hipSuccess ||
+		    (vs && hipMalloc(&sval, vs * total) != hipSuccess) ||
+		    (values && S.val32 && hipMalloc(&sval32, sizeof(float) * total) != hipSuccess)) {
+			// not enough memory for the copy: keep the CRS kernels only
+			(void)hipGetLastError();
+			if (sidx) hipFree(sidx);
+			if (sval) hipFree(sval);
+			if (sval32) hipFree(sval32);
+			hipFree(soff);
+			dia_free(dia);
+			if (S.cmask) hipFree(S.cmask);
+			S.cmask = nullptr;
+			S.cst = ConstDia();
+			return ALP_SUCCESS;
+		}
+		S.sell_idx = sidx;
+		S.sell_val = sval;
+		S.sell_val32 = sval32;
+	}
 	S.sell_off = soff;
-	S.sell_idx = sidx;
-	S.sell_val = sval;
-	S.sell_val32 = sval32;
 	S.n_slices = ns;
 	S.sell_entries = total;
-	ALP_TRY(dia_build(S.dia, ns, S.nmajor, nullptr, soff, total, S.off, S.idx, value_type, S.val, S.val32));
-	const char *keep = std::getenv("ALP_HIP_KEEP_SELL");  // "1": keep them (tests of the sliced-ELL path)
-	if (S.dia.flag && S.dia.n_dia == ns && !(keep && keep[0] == '1')) {
-		// every slice has the diagonal form, which reads neither the column
-		// indices nor the sliced-ELL values: keep only the slice offsets
-		ALP_HIP_TRY(hipStreamSynchronize(stream()));
-		hipFree(S.sell_idx);
-		if (S.sell_val) hipFree(S.sell_val);
-		if (S.sell_val32) hipFree(S.sell_val32);
-		S.sell_idx = nullptr;
-		S.sell_val = nullptr;
-		S.sell_val32 = nullptr;
-	}
-	return ALP_SUCCESS;
+	S.dia = dia;
+	ALP_TRY(sell_fill(S, value_type));
+	if (S.cst.w) return ALP_SUCCESS;
+	return dia_values(S.dia, ns, S.nmajor, nullptr, S.sell_off, total, S.off, value_type, S.val, S.val32);
 }
 
-// Copies S's current CRS values (and FP32 copy) into its sliced-ELL copy, after a
-// caller rewrote the values in place; the index layout is unchanged.
+// Copies S's current CRS values (and FP32 copy) into its sliced layouts, after a
+// caller rewrote the values in place; the index layout is unchanged. Values that
+// leave the constant form get the arrays it did without.
 alp_rc_t storage_refresh_values(Storage &S, int value_type) {
 	if (!S.sell_off || S.n_slices == 0) return ALP_SUCCESS;
-	const unsigned g = stream_grid(S.n_slices * kSellRows);
-	if (!S.sell_idx) {
-		// diagonal slices only (no sliced-ELL arrays)
-	} else if (value_type == ALP_VAL_F32)
-		hipLaunchKernelGGL(k_sell_fill<float>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, S.n_slices,
-		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const float *)S.val,
-		                   (const float *)S.val32, (const uint64_t *)S.sell_off, S.sell_idx, (float *)S.sell_val,
-		                   S.sell_val32);
-	else if (value_type == ALP_VAL_F64)
-		hipLaunchKernelGGL(k_sell_fill<double>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, S.n_slices,
-		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const double *)S.val,
-		                   (const float *)S.val32, (const uint64_t *)S.sell_off, S.sell_idx, (double *)S.sell_val,
-		                   S.sell_val32);
-	ALP_LAUNCH_CHECK();
-	return dia_refresh(S.dia, S.n_slices, S.nmajor, nullptr, S.sell_off, S.off, value_type, S.val, S.val32);
+	ALP_TRY(storage_const(S, value_type));
+	if (!S.cst.w && S.sell_idx) {
+		const size_t vs = value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
+		if (vs && !S.sell_val && hipMalloc(&S.sell_val, vs * S.sell_entries) != hipSuccess) {
+			(void)hipGetLastError();
+			S.sell_val = nullptr;  // the products then use the CRS kernels
+		}
+		if (S.val32 && !S.sell_val32 && hipMalloc(&S.sell_val32, sizeof(float) * S.sell_entries) != hipSuccess) {
+			(void)hipGetLastError();
+			S.sell_val32 = nullptr;
+		}
+	}
+	ALP_TRY(sell_fill(S, value_type));
+	if (S.cst.w) return ALP_SUCCESS;
+	return dia_values(S.dia, S.n_slices, S.nmajor, nullptr, S.sell_off, S.sell_entries, S.off, value_type, S.val,
+	                  S.val32);
 }
 
 alp_rc_t storage_ensure_f32(Storage &S, size_t nnz) {
@@ -568,18 +768,7 @@ alp_rc_t storage_ensure_f32(Storage &S, size_t nnz) {
 		hipLaunchKernelGGL((k_convert<double, float>), dim3(stream_grid(nnz)), dim3(kBlock), 0, stream(), nnz,
 		                   (const double *)S.val, S.val32);
 	ALP_LAUNCH_CHECK();
-	if (S.sell_off && S.sell_idx && S.sell_entries) {
-		if (hipMalloc(&S.sell_val32, sizeof(float) * S.sell_entries) != hipSuccess) {
-			(void)hipGetLastError();
-			S.sell_val32 = nullptr;  // the FP32 products then use the CRS kernels
-		}
-	}
-	if (S.dia.flag && S.sell_entries) {
-		if (hipMalloc(&S.dia.val32, sizeof(float) * S.sell_entries) != hipSuccess) {
-			(void)hipGetLastError();
-			S.dia.val32 = nullptr;
-		}
-	}
+	if (S.cst.w) return ALP_SUCCESS;  // the template holds both precisions
 	return storage_refresh_values(S, ALP_VAL_F64);
 }
 
@@ -629,6 +818,7 @@ void storage_free(Storage &S) {
 	if (S.sell_val) hipFree(S.sell_val);
 	if (S.sell_val32) hipFree(S.sell_val32);
 	dia_free(S.dia);
+	if (S.cmask) hipFree(S.cmask);
 	void *lr[] = {S.lr_rows, S.lr_c0, S.ch_row, S.ch_beg, S.ch_part};
 	for (void *q : lr)
 		if (q) hipFree(q);
@@ -1045,6 +1235,7 @@ size_t storage_bytes(const Storage &S, int value_type, size_t nnz) {
 	if (S.sell_val) b += vs * S.sell_entries;
 	if (S.sell_val32) b += sizeof(float) * S.sell_entries;
 	if (S.dia.flag) b += S.n_slices + sizeof(int32_t) * kDiaSlots * S.n_slices + sizeof(uint32_t) * S.n_slices * kSellRows;
+	if (S.cmask) b += sizeof(uint32_t) * S.n_slices * kSellRows;
 	if (S.dia.val) b += vs * S.sell_entries;
 	if (S.dia.val32) b += sizeof(float) * S.sell_entries;
 	b += S.n_long * 4 + (S.n_long + 1) * 8 + S.n_chunks * (4 + 8 + 8);

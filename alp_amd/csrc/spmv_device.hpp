@@ -171,6 +171,58 @@ __device__ __forceinline__ void rows_gather(const uint64_t (&beg)[RR], const uin
 	for (int i = 0; i < RR; ++i) acc[i] = group_fold<G, R>(acc[i]);
 }
 
+// ---- constant form ----------------------------------------------------------------
+// The fold of one row of a slice in constant form: r0 is the slice's first row
+// (uniform across the wavefront), the lane's row is r0 + lane with presence mask
+// bits; entry q multiplies x[row + d_q] by v_q, in storage order. Offsets and values
+// come from the kernel's arguments (scalar registers), so no load waits for
+// another: a launch's chain is the arguments, then mask and x together. W: the
+// template's width when known at compile time, else 0.
+//
+// A wavefront whose 64 rows all reach into [0, ncols) with every slot reads x
+// without per-lane conditions (an absent entry's x is in range and dropped by the
+// select below, whatever it holds) and folds without selects when all its rows
+// have every slot; only the slices at the two ends of the matrix mask their loads.
+template <typename R, int W>
+__device__ __forceinline__ typename R::A const_fold(const ConstArg<typename R::V> &T, long long r0, unsigned lane,
+                                                    uint32_t bits, long long ncols,
+                                                    const typename R::X *__restrict__ x) {
+	using A = typename R::A;
+	using X = typename R::X;
+	constexpr unsigned U = W ? W : 8;  // slots in flight
+	const unsigned w = W ? W : T.w;
+	const uint32_t full = w < 32 ? (1u << w) - 1u : 0xFFFFFFFFu;
+	const bool inside = r0 + T.dmin >= 0 && r0 + kSellRows - 1 + T.dmax < ncols;
+	A acc = R::zero();
+	if (inside) {
+#pragma unroll 1
+		for (unsigned q0 = 0; q0 < w; q0 += U) {
+			X xv[U];
+#pragma unroll
+			for (unsigned u = 0; u < U; ++u) {
+				const unsigned q = W ? u : (q0 + u < w ? q0 + u : w - 1);
+				xv[u] = (x + (r0 + T.d[q]))[lane];
+			}
+			if (__builtin_amdgcn_ballot_w64(bits != full) == 0) {
+#pragma unroll
+				for (unsigned u = 0; u < U; ++u)
+					if (W || q0 + u < w) acc = R::add(R::mul(T.v[W ? u : q0 + u], xv[u]), acc);
+			} else {
+#pragma unroll
+				for (unsigned u = 0; u < U; ++u)
+					if (W || q0 + u < w) {
+						const A t = R::add(R::mul(T.v[W ? u : q0 + u], xv[u]), acc);
+						acc = (bits >> (q0 + u)) & 1u ? t : acc;
+					}
+			}
+		}
+	} else {
+		for (unsigned q = 0; q < w; ++q)
+			if ((bits >> q) & 1u) acc = R::add(R::mul(T.v[q], (x + (r0 + T.d[q]))[lane]), acc);
+	}
+	return acc;
+}
+
 // ---- block tile fold (the CSR-stream pattern with a caller epilogue) ----------
 // Rows [r0, r1) of one tile whose nonzeros [base, top) number at most J*kBlock.
 // Every thread issues its J index/value loads, then the x gathers, products go

@@ -1,0 +1,125 @@
+"""The constant form (one template of offsets and values for all rows): every product
+and solve on it must equal the forms that keep values bit for bit, and matrices
+that only nearly fit must keep those forms. ALP_HIP_CONST_DIA=0 builds without it."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def A():
+    import alp_amd
+    alp_amd.init(0)
+    return alp_amd
+
+
+def banded(n, m, offs, vals, drop=None):
+    """Rows r of an n x m matrix with entries (r + d, v) for the offsets in the given
+    order that land in [0, m); drop(r, q) leaves entry q of row r out."""
+    R = np.repeat(np.arange(n, dtype=np.int64), len(offs))
+    C = R + np.tile(np.asarray(offs, np.int64), n)
+    V = np.tile(np.asarray(vals), n)
+    keep = (C >= 0) & (C < m)
+    if drop is not None:
+        keep &= ~drop
+    off = np.zeros(n + 1, np.uint64)
+    np.cumsum(np.bincount(R[keep], minlength=n), out=off[1:])
+    return off, C[keep].astype(np.uint32), V[keep]
+
+
+def both(A, monkeypatch, build):
+    monkeypatch.setenv("ALP_HIP_CONST_DIA", "0")
+    plain = build()
+    monkeypatch.delenv("ALP_HIP_CONST_DIA")
+    return build(), plain
+
+
+def products(A, M, x, y0, ring, mask):
+    out = []
+    for descr, mk in ((0, None), (A.OVERWRITE, None), (0, mask), (A.INVERT_MASK, mask), (A.OVERWRITE, mask)):
+        y = A.Vector.from_numpy(y0)
+        assert A.mxv(y, M, A.Vector.from_numpy(x), ring=ring, descr=descr,
+                     mask=None if mk is None else A.Vector.from_numpy(mk)) == A.SUCCESS
+        out.append(y.numpy())
+    return out
+
+
+# widths around the compile-time ones (7 and 27) and the largest; rows around a slice,
+# wider and narrower than long, with NaN and infinities at entries of x
+@pytest.mark.parametrize("w", [1, 2, 6, 7, 8, 9, 26, 27, 28, 32])
+@pytest.mark.parametrize("n,m", [(64, 64), (65, 130), (1000, 1000), (3001, 2950)])
+def test_const_products_equal_kept_values(A, w, n, m, monkeypatch):
+    rng = np.random.default_rng(1000 * w + n)
+    offs = rng.permutation(rng.choice(np.arange(-45, 46), size=w, replace=False))
+    vals = rng.standard_normal(w)
+    drop = rng.random(n * w) < 0.1
+    drop[np.arange(n // 2) * w + rng.integers(0, w, n // 2)] = False
+    off, idx, val = banded(n, m, offs, vals, drop if n > 64 else None)
+    x, y0 = rng.standard_normal(m), rng.standard_normal(n)
+    if n == 1000:
+        x[17], x[400], x[999] = np.nan, np.inf, -np.inf
+    mask = (rng.random(n) < 0.5).astype(np.uint8)
+    F, P = both(A, monkeypatch, lambda: A.Matrix.from_crs(n, m, off, idx, val, flags=A.MAT_WITH_F32))
+    F32, P32 = both(A, monkeypatch, lambda: A.Matrix.from_crs(n, m, off, idx, val.astype(np.float32)))
+    x32, y32 = x.astype(np.float32), y0.astype(np.float32)
+    for c, p, ring, xv, yv in ((F, P, A.PLUS_TIMES_F64, x, y0), (F, P, A.MIN_PLUS_F64, x, y0),
+                               (F, P, A.PLUS_TIMES_F32, x32, y32), (F32, P32, A.PLUS_TIMES_F32, x32, y32),
+                               (F, P, A.PLUS_PATTERN_F64, x, y0)):
+        # kernel 4 folds each row in storage order whatever the default is
+        for k in (c, p):
+            if k.layout()[0]:
+                k.set_kernel(4)
+        for a, b in zip(products(A, c, xv, yv, ring, mask), products(A, p, xv, yv, ring, mask)):
+            assert np.array_equal(a, b, equal_nan=True), (w, n, ring)
+
+
+@pytest.mark.parametrize("sides", [(4, 4, 4), (8, 8, 8), (65, 3, 5), (33, 17, 9), (64, 12, 10), (130, 20, 3)])
+def test_const_stencil_takes_the_form(A, sides, monkeypatch):
+    """27-point stencils, also where slices straddle lines and planes, hold fewer bytes
+    than with values; products are the same bits through mxv and the transposed vxm."""
+    C, P = both(A, monkeypatch, lambda: A.Matrix.stencil27(*sides, flags=A.MAT_WITH_CCS | A.MAT_WITH_F32))
+    if P.layout()[0]:
+        assert C.device_bytes() < P.device_bytes()
+        P.set_kernel(4)
+        C.set_kernel(4)
+    rng = np.random.default_rng(7)
+    x = A.Vector.from_numpy(rng.standard_normal(C.nrows))
+    for f in (lambda M, y: A.mxv(y, M, x), lambda M, y: A.vxm(y, x, M), lambda M, y: A.mxv(y, M, x, descr=A.TRANSPOSE_MATRIX)):
+        got = []
+        for M in (C, P):
+            y = A.Vector(C.nrows, fill=0.5)
+            assert f(M, y) == A.SUCCESS
+            got.append(y.numpy())
+        assert np.array_equal(got[0], got[1])
+
+
+def test_const_near_misses_keep_their_values(A, monkeypatch):
+    """One value off by an ulp, one row in another order, one column stored twice: not
+    one template, so the bytes held and the results are those without the form."""
+    rng = np.random.default_rng(3)
+    n, offs = 2000, [-40, -1, 0, 1, 40]
+    off, idx, val = banded(n, n, offs, [-1.0, -1.0, 4.0, -1.0, -1.0])
+    x = rng.standard_normal(n)
+
+    def variant(k):
+        i, v = idx.copy(), val.copy()
+        a = int(off[n // 2])
+        if k == 0:
+            v[a + 2] = np.nextafter(4.0, 5.0)
+        elif k == 1:
+            i[a], i[a + 1] = i[a + 1], i[a]
+        else:
+            i[a + 1] = i[a]
+        return A.Matrix.from_crs(n, n, off, i, v)
+
+    for k in range(3):
+        C, P = both(A, monkeypatch, lambda: variant(k))
+        assert C.device_bytes() == P.device_bytes(), k
+        got = []
+        for M in (C, P):
+            M.set_kernel(4)
+            y = A.Vector(n, fill=0.0)
+            assert A.mxv(y, M, A.Vector.from_numpy(x)) == A.SUCCESS
+            got.append(y.numpy())
+        assert np.array_equal(got[0], got[1]), k
