@@ -29,6 +29,7 @@
 
 #include <hipcub/hipcub.hpp>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <type_traits>
@@ -84,6 +85,16 @@ struct HpLevel {
 	std::vector<size_t> colour_slice_off;  // slices of colour c: [cso[c], cso[c+1])
 	size_t sell_entries = 0;
 	DiaSlices dia;                         // diagonal form of the slices that have it
+	// constant form, one template per colour (empty: some row does not fit): the
+	// slices' masks, the templates on the device for products over all colours, and
+	// the diagonal value that every row has. The sliced layouts are then not built.
+	std::vector<ConstDia> cst;
+	uint32_t *cmask = nullptr;
+	ConstArg<double> *ctab = nullptr;
+	ConstArg<float> *ctab32 = nullptr;
+	uint32_t *crow = nullptr;              // first row of each colour (ncolors + 1)
+	uint32_t *cslice = nullptr;            // first slice of each colour (ncolors + 1)
+	double cdiag = 0.0;
 };
 
 // Per-iteration scalars in two slots: iteration j reads slot j % 2 and only its
@@ -499,6 +510,152 @@ __global__ __launch_bounds__(kBlock) void k_sell_rows(size_t s0, size_t s1, cons
 	const int stop = done ? *done : 0;
 	slice_rows<T, U, DIA>(sl, threadIdx.x % kSellRows, stop, srow, soff, sidx, sval, off, x, ep, dflag, dcol, dmask,
 	                      dval);
+}
+
+// ---- constant form ------------------------------------------------------------------
+//
+// On a level whose rows fit one template per colour (ConstDia; any level with even
+// sides) a colour step reads no matrix: a mask per row, r, and z. The template is a
+// kernel argument and a colour's slices are consecutive, so all of a slice's loads
+// go out together: the chain is the arguments, one round of loads, the store. That
+// chain is what the coarse levels' launches cost.
+
+// x at the slots of row r0 + lane (0 where absent at the ends of the vector, and
+// whatever is there where absent inside: sum27 drops it)
+template <typename T>
+__device__ __forceinline__ void gather27(const ConstArg<T> &C, long long r0, unsigned lane, uint32_t bits, long long n,
+                                         const T *__restrict__ x, T (&xv)[kDiaFullWidth]) {
+	if (r0 + C.dmin >= 0 && r0 + kSellRows - 1 + C.dmax < n) {
+#pragma unroll
+		for (unsigned q = 0; q < kDiaFullWidth; ++q) xv[q] = (x + (r0 + C.d[q]))[lane];
+	} else {
+#pragma unroll
+		for (unsigned q = 0; q < kDiaFullWidth; ++q) {
+			xv[q] = T(0);
+			if ((bits >> q) & 1u) xv[q] = (x + (r0 + C.d[q]))[lane];
+		}
+	}
+}
+
+// the row's fold in storage order over accumulator type A; the entry of slot self
+// takes own instead of the gathered value (self = kDiaFullWidth: none)
+template <typename A, typename T>
+__device__ __forceinline__ A sum27(const ConstArg<T> &C, uint32_t bits, const T (&xv)[kDiaFullWidth],
+                                   unsigned self = kDiaFullWidth, T own = T(0)) {
+	A acc = A(0);
+	if (__builtin_amdgcn_ballot_w64(bits != (1u << kDiaFullWidth) - 1u) == 0) {
+#pragma unroll
+		for (unsigned q = 0; q < kDiaFullWidth; ++q) {
+			const A prod = (A)C.v[q] * (A)(q == self ? own : xv[q]);
+			acc = prod + acc;
+		}
+	} else {
+#pragma unroll
+		for (unsigned q = 0; q < kDiaFullWidth; ++q) {
+			const A prod = (A)C.v[q] * (A)(q == self ? own : xv[q]);
+			const A t = prod + acc;
+			acc = (bits >> q) & 1u ? t : acc;
+		}
+	}
+	return acc;
+}
+
+// What a colour step does beside z = ((r - A z) + z d) / d on its rows. A proper
+// colouring's rows read no other row of their colour, so steps that follow each
+// other on one colour run as one, on the row's gathered z with its own entry
+// replaced: the same operations in the same order as separate launches.
+enum : int {
+	kStepPlain = 0,
+	kStepTwice,     // the last forward and first backward step of a sweep
+	kStepRestrict,  // then r_c = (r - A z) and z_c = 0 at the injected rows
+	kStepProlong,   // first z += z_c at the injected rows
+};
+
+template <typename T>
+struct ConstStep {
+	ConstArg<T> C;
+	uint32_t row0, row1;  // the colour's rows
+	uint32_t s0;          // and its first slice
+	unsigned self;        // the diagonal's slot
+	T d;                  // and its value
+	size_t n;
+	const uint32_t *mask, *f2c;
+	const T *r;
+	T *z, *rc, *zc;
+	const int *done;
+};
+
+template <typename T, int MODE>
+__global__ __launch_bounds__(kBlock) void k_const_step(ConstStep<T> a) {
+	const unsigned nw = blockDim.x / kSellRows;
+	const unsigned bl = xcd_logical_block(blockIdx.x, gridDim.x);
+	const unsigned i = __builtin_amdgcn_readfirstlane(bl * nw + threadIdx.x / kSellRows);
+	const unsigned lane = threadIdx.x % kSellRows;
+	const uint32_t r0 = a.row0 + i * kSellRows;
+	if (r0 >= a.row1) return;  // whole wavefronts leave together
+	const int stop = a.done ? *a.done : 0;
+	const uint32_t row = r0 + lane;
+	const bool act = row < a.row1;
+	const uint32_t bits = a.mask[(size_t)(a.s0 + i) * kSellRows + lane];
+	T xv[kDiaFullWidth];
+	gather27<T>(a.C, (long long)r0, lane, bits, (long long)a.n, a.z, xv);
+	T ri = T(0), zi = T(0);
+	uint32_t c = 0;
+	if (act) {
+		ri = a.r[row];
+		zi = a.z[row];
+		if (MODE == kStepRestrict || MODE == kStepProlong) c = a.f2c[row - a.row0];
+		if (MODE == kStepProlong) zi += a.zc[c];
+	}
+	if (stop) return;
+	T acc = MODE == kStepProlong ? sum27<T, T>(a.C, bits, xv, a.self, zi) : sum27<T, T>(a.C, bits, xv);
+	zi = ((ri - acc) + zi * a.d) / a.d;
+	if (MODE == kStepTwice) {
+		acc = sum27<T, T>(a.C, bits, xv, a.self, zi);
+		zi = ((ri - acc) + zi * a.d) / a.d;
+	}
+	if (act) a.z[row] = zi;
+	if (MODE == kStepRestrict) {
+		acc = sum27<T, T>(a.C, bits, xv, a.self, zi);
+		if (act) {
+			a.rc[c] = ri - acc;
+			a.zc[c] = T(0);
+		}
+	}
+}
+
+// Row products over all colours: blockIdx.y is the colour; ep as in k_sell_rows.
+template <typename T, typename Ep>
+__global__ __launch_bounds__(kBlock) void k_const_rows(const ConstArg<T> *__restrict__ tab,
+                                                      const uint32_t *__restrict__ crow,
+                                                      const uint32_t *__restrict__ cslice,
+                                                      const uint32_t *__restrict__ mask, size_t n,
+                                                      const T *__restrict__ x, Ep ep, const int *done) {
+	const unsigned colour = blockIdx.y;
+	const uint32_t row1 = crow[colour + 1];
+	const unsigned bl = xcd_logical_block(blockIdx.x, gridDim.x);
+	const unsigned i = __builtin_amdgcn_readfirstlane(bl * (kBlock / kSellRows) + threadIdx.x / kSellRows);
+	const unsigned lane = threadIdx.x % kSellRows;
+	const uint32_t r0 = crow[colour] + i * kSellRows;
+	if (r0 >= row1) return;
+	const int stop = done ? *done : 0;
+	const uint32_t row = r0 + lane;
+	const bool act = row < row1;
+	const uint32_t bits = mask[(size_t)(cslice[colour] + i) * kSellRows + lane];
+	if (act) ep.prefetch(row);
+	T xv[kDiaFullWidth];
+	gather27<T>(tab[colour], (long long)r0, lane, bits, (long long)n, x, xv);
+	if (stop) return;
+	using A = typename AccOf<Ep, T>::type;
+	const A acc = sum27<A, T>(tab[colour], bits, xv);
+	if (act) ep.finish(row, acc, bits == 0);
+}
+
+// *bad = 1 when some diagonal entry differs from v
+__global__ __launch_bounds__(kBlock) void k_check_diag(size_t n, const double *diag, double v, int *bad) {
+	grid_for_each<4>(n, [&](size_t i) {
+		if (diag[i] != v) atomicOr(bad, 1);
+	});
 }
 
 __global__ __launch_bounds__(kBlock) void k_hs_width(size_t ns, const uint32_t *srow, const uint64_t *off,
@@ -934,7 +1091,8 @@ static void free_level(HpLevel &L) {
 	void *ps[] = {L.off, L.idx, L.val, L.val32, L.diag, L.diag32, L.perm, L.iperm, L.colour,
 	              L.ts[0].rb, L.ts[0].re, L.ts[0].base, L.ts[0].top, L.ts[1].rb, L.ts[1].re,
 	              L.ts[1].base, L.ts[1].top, L.inj, L.z, L.r, L.t,
-	              L.z32, L.r32, L.t32, L.srow, L.soff, L.sidx, L.sval, L.sval32, L.f2c};
+	              L.z32, L.r32, L.t32, L.srow, L.soff, L.sidx, L.sval, L.sval32, L.f2c,
+	              L.cmask, L.ctab, L.ctab32, L.crow, L.cslice};
 	for (void *p : ps)
 		if (p) hipFree(p);
 	dia_free(L.dia);
@@ -944,6 +1102,82 @@ static void free_level(HpLevel &L) {
 template <typename T>
 static alp_rc_t dmalloc(T **p, size_t count) {
 	ALP_HIP_TRY(hipMalloc(p, sizeof(T) * (count ? count : 1)));
+	return ALP_SUCCESS;
+}
+
+template <typename T>
+static ConstArg<T> const_level_arg(const ConstDia &D) {
+	ConstArg<T> a{};
+	a.w = D.w;
+	a.dmin = D.dmin;
+	a.dmax = D.dmax;
+	for (unsigned q = 0; q < kDiaSlots; ++q) {
+		a.d[q] = D.d[q];
+		a.v[q] = sizeof(T) == 8 ? (T)D.v64[q] : (T)D.v32[q];
+	}
+	return a;
+}
+
+// The level's constant form: every colour's rows fit one 27-slot template and all
+// rows have the same diagonal entry. Leaves L.cst empty when they do not.
+static alp_rc_t build_level_const(HpLevel &L) {
+	if (!L.proper || !const_dia_enabled() || L.nslices == 0) return ALP_SUCCESS;
+	ALP_TRY(dmalloc(&L.cmask, L.nslices * kSellRows));
+	std::vector<ConstDia> cst(L.ncolors);
+	std::vector<ConstArg<double>> tab(L.ncolors);
+	std::vector<ConstArg<float>> tab32(L.ncolors);
+	std::vector<uint32_t> crow(L.ncolors + 1), cslice(L.ncolors + 1);
+	bool ok = true;
+	double diag = 0.0;
+	for (int c = 0; c <= L.ncolors; ++c) {
+		crow[c] = (uint32_t)L.color_off[c];
+		cslice[c] = (uint32_t)L.colour_slice_off[c];
+	}
+	for (int c = 0; c < L.ncolors && ok; ++c) {
+		ALP_TRY(const_detect(cst[c], L.color_off[c], L.color_off[c + 1], L.colour_slice_off[c],
+		                     L.colour_slice_off[c + 1], L.srow, L.off, L.idx, ALP_VAL_F64, L.val, L.cmask));
+		ok = cst[c].w == kDiaFullWidth;
+		double v = 0.0;
+		bool self = false;
+		for (unsigned q = 0; ok && q < cst[c].w; ++q)
+			if (cst[c].d[q] == 0) {
+				v = cst[c].v64[q];
+				self = true;
+			}
+		ok = ok && self && (c == 0 || v == diag);
+		diag = v;
+		tab[c] = const_level_arg<double>(cst[c]);
+		tab32[c] = const_level_arg<float>(cst[c]);
+	}
+	if (ok) {
+		int *bad = nullptr, hbad = 1;
+		ALP_TRY(dmalloc(&bad, 1));
+		hipError_t e = hipMemsetAsync(bad, 0, sizeof(int), stream());
+		if (e == hipSuccess) {
+			hipLaunchKernelGGL(k_check_diag, dim3(grid_for(L.n)), dim3(kBlock), 0, stream(), L.n,
+			                   (const double *)L.diag, diag, bad);
+			e = hipGetLastError();
+		}
+		if (e == hipSuccess) e = copy_sync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost);
+		hipFree(bad);
+		ALP_HIP_TRY(e);
+		ok = hbad == 0;
+	}
+	if (!ok) {
+		hipFree(L.cmask);
+		L.cmask = nullptr;
+		return ALP_SUCCESS;
+	}
+	ALP_TRY(dmalloc(&L.ctab, L.ncolors));
+	ALP_TRY(dmalloc(&L.ctab32, L.ncolors));
+	ALP_TRY(dmalloc(&L.crow, L.ncolors + 1));
+	ALP_TRY(dmalloc(&L.cslice, L.ncolors + 1));
+	ALP_HIP_TRY(copy_sync(L.ctab, tab.data(), sizeof(tab[0]) * tab.size(), hipMemcpyHostToDevice));
+	ALP_HIP_TRY(copy_sync(L.ctab32, tab32.data(), sizeof(tab32[0]) * tab32.size(), hipMemcpyHostToDevice));
+	ALP_HIP_TRY(copy_sync(L.crow, crow.data(), 4 * crow.size(), hipMemcpyHostToDevice));
+	ALP_HIP_TRY(copy_sync(L.cslice, cslice.data(), 4 * cslice.size(), hipMemcpyHostToDevice));
+	L.cdiag = diag;
+	L.cst = std::move(cst);
 	return ALP_SUCCESS;
 }
 
@@ -971,6 +1205,7 @@ static alp_rc_t build_level_sell(HpLevel &L) {
 			break;
 		}
 		if (ns == 0) break;
+		if ((rc = build_level_const(L)) || !L.cst.empty()) break;  // the constant form needs no other layout
 		hipLaunchKernelGGL(k_hs_width, dim3(grid_for(ns)), dim3(kBlock), 0, s, ns, (const uint32_t *)L.srow,
 		                   (const uint64_t *)L.off, sizes);
 		size_t tb = 0;
@@ -1167,6 +1402,47 @@ static Tiles all_tiles(const HpLevel &L) {
 	return Tiles{S.rb, S.re, S.base, S.top, 0, S.count, tile_xcd()};
 }
 
+// Row products over all rows of a level in constant form (false: not in it).
+template <typename T, typename Ep>
+static bool const_rows(const HpLevel &L, const T *x, Ep ep, hipStream_t s, const int *done) {
+	if (L.cst.empty()) return false;
+	size_t most = 0;
+	for (int c = 0; c < L.ncolors; ++c) most = std::max(most, L.colour_slice_off[c + 1] - L.colour_slice_off[c]);
+	const size_t per = kBlock / kSellRows;
+	const ConstArg<T> *tab;
+	if constexpr (sizeof(T) == 8) tab = L.ctab; else tab = L.ctab32;
+	hipLaunchKernelGGL((k_const_rows<T, Ep>), dim3((most + per - 1) / per, L.ncolors), dim3(kBlock), 0, s, tab,
+	                   (const uint32_t *)L.crow, (const uint32_t *)L.cslice, (const uint32_t *)L.cmask, L.n, x, ep, done);
+	return true;
+}
+
+// One colour step of a level in constant form; C: the coarse level of a step that
+// restricts to it or prolongs from it.
+template <typename T, int MODE>
+static void const_step(HpLevel &L, int c, HpLevel *C, hipStream_t s, const int *done) {
+	const size_t rows = L.color_off[c + 1] - L.color_off[c];
+	if (rows == 0) return;
+	ConstStep<T> a{const_level_arg<T>(L.cst[c]),
+	               (uint32_t)L.color_off[c],
+	               (uint32_t)L.color_off[c + 1],
+	               (uint32_t)L.colour_slice_off[c],
+	               0,
+	               (T)L.cdiag,
+	               L.n,
+	               L.cmask,
+	               C ? C->f2c : nullptr,
+	               Vec<T>::r(L),
+	               Vec<T>::z(L),
+	               C ? Vec<T>::r(*C) : nullptr,
+	               C ? Vec<T>::z(*C) : nullptr,
+	               done};
+	for (unsigned q = 0; q < a.C.w; ++q)
+		if (a.C.d[q] == 0) a.self = q;
+	const unsigned waves = kBlock / kSellRows;
+	const size_t ns = (rows + kSellRows - 1) / kSellRows;
+	hipLaunchKernelGGL((k_const_step<T, MODE>), dim3((ns + waves - 1) / waves), dim3(waves * kSellRows), 0, s, a);
+}
+
 // Row products over slices [s0, s1) of the level's sliced-ELL copy in precision
 // T; false when the level has no copy in that precision (the tile path runs
 // instead). Diagonal-slice launches map slices to XCDs in contiguous ranges: the
@@ -1176,6 +1452,7 @@ static Tiles all_tiles(const HpLevel &L) {
 template <typename T, typename Ep>
 static bool sell_rows(const HpLevel &L, size_t s0, size_t s1, const T *x, Ep ep, hipStream_t s,
                       const int *done) {
+	if (s0 == 0 && s1 == L.nslices && const_rows<T>(L, x, ep, s, done)) return true;
 	const T *sval = Vec<T>::sval(L);
 	if (!sval || !L.soff) return false;
 	const size_t per = kBlock / kSellRows;
@@ -1235,11 +1512,32 @@ static void colour_step(HpLevel &L, int c, hipStream_t s, const int *done, bool 
 	}
 }
 
-// z_is_zero: z was just set to 0 (the first sweep of a V-cycle level)
+// z_is_zero: z was just set to 0 (the first sweep of a V-cycle level). from / to:
+// the coarse level whose correction is added before the sweep, or that gets the
+// residual after it (levels whose steps can take them: fused_transfers)
 template <typename T>
-static void rbgs(HpLevel &L, hipStream_t s, const int *done, bool z_is_zero = false) {
+static void rbgs(HpLevel &L, hipStream_t s, const int *done, bool z_is_zero = false, HpLevel *from = nullptr,
+                 HpLevel *to = nullptr) {
+	if (!L.cst.empty() && L.ncolors > 1) {
+		const int last = L.ncolors - 1;
+		if (z_is_zero) colour_step<T>(L, 0, s, done, true);
+		else if (from) const_step<T, kStepProlong>(L, 0, from, s, done);
+		else const_step<T, kStepPlain>(L, 0, nullptr, s, done);
+		for (int c = 1; c < last; ++c) const_step<T, kStepPlain>(L, c, nullptr, s, done);
+		const_step<T, kStepTwice>(L, last, nullptr, s, done);
+		for (int c = last - 1; c > 0; --c) const_step<T, kStepPlain>(L, c, nullptr, s, done);
+		if (to) const_step<T, kStepRestrict>(L, 0, to, s, done);
+		else const_step<T, kStepPlain>(L, 0, nullptr, s, done);
+		return;
+	}
 	for (int c = 0; c < L.ncolors; ++c) colour_step<T>(L, c, s, done, z_is_zero && c == 0);
 	for (int c = L.ncolors - 1; c >= 0; --c) colour_step<T>(L, c, s, done);
+}
+
+// the transfers between F and its coarse level C run inside F's sweeps: F is in
+// constant form and C's injected rows are F's colour 0
+static bool fused_transfers(const HpLevel &F, const HpLevel &C) {
+	return !F.cst.empty() && F.ncolors > 1 && C.f2c && C.f2c_colour == 0;
 }
 
 // multi_grid (multigrid_v_cycle.hpp:180-246) from level l; z_l must already be 0
@@ -1250,10 +1548,12 @@ static void vcycle(alp_hip_hpcg_s *H, size_t l, hipStream_t s, const int *done) 
 		rbgs<T>(F, s, done, true);
 		return;
 	}
-	for (size_t i = 0; i < H->presmooth; ++i) rbgs<T>(F, s, done, i == 0);
 	HpLevel &C = H->L[l + 1];
-	bool swept = false;
-	if (C.f2c) {
+	const bool fused = fused_transfers(F, C);
+	bool swept = fused && H->presmooth > 0;
+	for (size_t i = 0; i < H->presmooth; ++i)
+		rbgs<T>(F, s, done, i == 0, nullptr, swept && i + 1 == H->presmooth ? &C : nullptr);
+	if (!swept && C.f2c) {
 		const int c = C.f2c_colour;
 		EpRestrict<T> ep{Vec<T>::r(F), C.f2c, C.f2c_base, Vec<T>::r(C), Vec<T>::z(C), T(0)};
 		swept = sell_rows<T>(F, F.colour_slice_off[c], F.colour_slice_off[c + 1], (const T *)Vec<T>::z(F), ep, s,
@@ -1267,9 +1567,11 @@ static void vcycle(alp_hip_hpcg_s *H, size_t l, hipStream_t s, const int *done) 
 		                   Vec<T>::z(C), done);
 	}
 	vcycle<T>(H, l + 1, s, done);
-	hipLaunchKernelGGL(k_prolong<T>, dim3(grid_for(C.n)), dim3(kBlock), 0, s, C.n, (const uint32_t *)C.inj,
-	                   (const T *)Vec<T>::z(C), Vec<T>::z(F), done);
-	for (size_t i = 0; i < H->postsmooth; ++i) rbgs<T>(F, s, done);
+	const bool added = fused && H->postsmooth > 0;
+	if (!added)
+		hipLaunchKernelGGL(k_prolong<T>, dim3(grid_for(C.n)), dim3(kBlock), 0, s, C.n, (const uint32_t *)C.inj,
+		                   (const T *)Vec<T>::z(C), Vec<T>::z(F), done);
+	for (size_t i = 0; i < H->postsmooth; ++i) rbgs<T>(F, s, done, false, added && i == 0 ? &C : nullptr);
 }
 
 // z = M r (V-cycle) or z = r, in precision T, on the finest level's vectors
@@ -1427,7 +1729,7 @@ static alp_rc_t run_iterations(alp_hip_hpcg_s *H, T *x, T *p, T *Ap, HpState *st
 // onto that colour's row range), the restriction runs as a sweep over that
 // colour's slices (EpRestrict) instead of one gather per coarse row.
 static alp_rc_t build_restrict_map(HpLevel &C, HpLevel &F) {
-	if (C.n == 0 || !F.soff || F.colour_slice_off.empty()) return ALP_SUCCESS;
+	if (C.n == 0 || (!F.soff && F.cst.empty()) || F.colour_slice_off.empty()) return ALP_SUCCESS;
 	uint32_t f0 = 0;
 	ALP_HIP_TRY(copy_sync(&f0, C.inj, sizeof(uint32_t), hipMemcpyDeviceToHost));
 	int c = -1;

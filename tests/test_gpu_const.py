@@ -123,3 +123,26 @@ def test_const_near_misses_keep_their_values(A, monkeypatch):
             assert A.mxv(y, M, A.Vector.from_numpy(x)) == A.SUCCESS
             got.append(y.numpy())
         assert np.array_equal(got[0], got[1]), k
+
+
+@pytest.mark.parametrize("sizes,levels,pre,post", [((16, 16, 16), 2, 1, 1), ((24, 16, 40), 1, 2, 2), ((12, 20, 28), 1, 1, 1),
+                                                  ((32, 16, 16), 2, 0, 1), ((16, 32, 16), 2, 1, 0), ((8, 12, 10), 0, 1, 1),
+                                                  ((9, 11, 7), 0, 1, 1)])
+def test_const_hpcg_equals_kept_values(A, sizes, levels, pre, post, monkeypatch):
+    """V-cycle and solves on levels in constant form (whose steps on one colour, and
+    transfers, run in one launch) equal the sliced layouts' bit for bit; odd sides
+    (whose colours do not share offsets) keep those layouts."""
+    C, P = both(A, monkeypatch, lambda: A.Hpcg(*sizes, max_levels=levels, colours=0, presmooth=pre, postsmooth=post))
+    rng = np.random.default_rng(11)
+    r = A.Vector.from_numpy(rng.standard_normal(C.n))
+    z = [A.Vector(C.n, fill=0.0) for _ in range(2)]
+    C.vcycle(r, z[0])
+    P.vcycle(r, z[1])
+    assert np.array_equal(z[0].numpy(), z[1].numpy())
+    for precision in (0, 1, 2, 3):
+        got = []
+        for H in (C, P):
+            x = A.Vector(C.n, fill=0.0)
+            got.append((H.solve(r, x, 60, 1e-9, precision), x.numpy()))
+        assert got[0][0] == got[1][0], precision
+        assert np.array_equal(got[0][1], got[1][1]), precision
