@@ -242,6 +242,9 @@ struct ConstDia {
 	unsigned w = 0;  // slots of the template; 0: the slices are not in this form
 	int32_t d[kDiaSlots] = {};
 	int32_t dmin = 0, dmax = 0;
+	// 1 / -1: the template is kDiaFullWidth / 3 runs of three offsets going up / down
+	// by one; 0: it is not
+	int run = 0;
 	double v64[kDiaSlots] = {};  // the values (FP64 matrices) and their FP32 copies,
 	float v32[kDiaSlots] = {};   // or the values of an FP32 matrix
 };

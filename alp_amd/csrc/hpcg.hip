@@ -520,19 +520,18 @@ __global__ __launch_bounds__(kBlock) void k_sell_rows(size_t s0, size_t s1, cons
 // go out together: the chain is the arguments, one round of loads, the store. That
 // chain is what the coarse levels' launches cost.
 
-// x at the slots of row r0 + lane (0 where absent at the ends of the vector, and
-// whatever is there where absent inside: sum27 drops it)
+// x at the slots of row r0 + lane, where the row has no entry whatever is there (at the
+// two ends of the vector at a clamped position): sum27 drops it
 template <typename T>
-__device__ __forceinline__ void gather27(const ConstArg<T> &C, long long r0, unsigned lane, uint32_t bits, long long n,
-                                         const T *__restrict__ x, T (&xv)[kDiaFullWidth]) {
+__device__ __forceinline__ void gather27(const ConstArg<T> &C, long long r0, unsigned lane, long long n, const T *__restrict__ x, T (&xv)[kDiaFullWidth]) {
 	if (r0 + C.dmin >= 0 && r0 + kSellRows - 1 + C.dmax < n) {
 #pragma unroll
 		for (unsigned q = 0; q < kDiaFullWidth; ++q) xv[q] = (x + (r0 + C.d[q]))[lane];
 	} else {
 #pragma unroll
 		for (unsigned q = 0; q < kDiaFullWidth; ++q) {
-			xv[q] = T(0);
-			if ((bits >> q) & 1u) xv[q] = (x + (r0 + C.d[q]))[lane];
+			const long long c = r0 + lane + C.d[q];
+			xv[q] = x[c < 0 ? 0 : c < n ? c : n - 1];
 		}
 	}
 }
@@ -552,9 +551,8 @@ __device__ __forceinline__ A sum27(const ConstArg<T> &C, uint32_t bits, const T 
 	} else {
 #pragma unroll
 		for (unsigned q = 0; q < kDiaFullWidth; ++q) {
-			const A prod = (A)C.v[q] * (A)(q == self ? own : xv[q]);
-			const A t = prod + acc;
-			acc = (bits >> q) & 1u ? t : acc;
+			const A prod = (A)C.v[q] * (A)keep_if(bits, q, q == self ? own : xv[q]);
+			acc = prod + acc;
 		}
 	}
 	return acc;
@@ -598,7 +596,7 @@ __global__ __launch_bounds__(kBlock) void k_const_step(ConstStep<T> a) {
 	const bool act = row < a.row1;
 	const uint32_t bits = a.mask[(size_t)(a.s0 + i) * kSellRows + lane];
 	T xv[kDiaFullWidth];
-	gather27<T>(a.C, (long long)r0, lane, bits, (long long)a.n, a.z, xv);
+	gather27<T>(a.C, (long long)r0, lane, (long long)a.n, a.z, xv);
 	T ri = T(0), zi = T(0);
 	uint32_t c = 0;
 	if (act) {
@@ -644,7 +642,7 @@ __global__ __launch_bounds__(kBlock) void k_const_rows(const ConstArg<T> *__rest
 	const uint32_t bits = mask[(size_t)(cslice[colour] + i) * kSellRows + lane];
 	if (act) ep.prefetch(row);
 	T xv[kDiaFullWidth];
-	gather27<T>(tab[colour], (long long)r0, lane, bits, (long long)n, x, xv);
+	gather27<T>(tab[colour], (long long)r0, lane, (long long)n, x, xv);
 	if (stop) return;
 	using A = typename AccOf<Ep, T>::type;
 	const A acc = sum27<A, T>(tab[colour], bits, xv);

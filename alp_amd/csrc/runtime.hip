@@ -583,6 +583,9 @@ static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0,
 	ALP_HIP_TRY(copy_sync(&h, d, sizeof(Work), hipMemcpyDeviceToHost));
 	if (h.t.w == 0 || h.t.w > kDiaSlots) return ALP_SUCCESS;
 	for (unsigned q = 0; q < h.t.w; ++q) {
+		V v;
+		__builtin_memcpy(&v, &h.t.bits[q], sizeof(V));
+		if (!std::isfinite((double)v) || !std::isfinite((float)v)) return ALP_SUCCESS;  // absent entries fold v * 0
 		if (h.t.d[q] < INT32_MIN || h.t.d[q] > INT32_MAX) return ALP_SUCCESS;
 		for (unsigned p = 0; p < q; ++p)
 			if (h.t.d[p] == h.t.d[q]) return ALP_SUCCESS;  // a column stored twice: the diagonal form keeps it
@@ -604,6 +607,14 @@ static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0,
 		C.v32[q] = (float)v;
 		C.dmin = std::min(C.dmin, C.d[q]);
 		C.dmax = std::max(C.dmax, C.d[q]);
+	}
+	if (C.w == kDiaFullWidth) {
+		C.run = C.d[1] > C.d[0] ? 1 : -1;
+		for (unsigned q = 0; q < C.w; q += 3)
+			if ((int64_t)C.d[q + 1] - C.d[q] != C.run || (int64_t)C.d[q + 2] - C.d[q + 1] != C.run) {
+				C.run = 0;
+				break;
+			}
 	}
 	return ALP_SUCCESS;
 }

@@ -558,7 +558,8 @@ __global__ __launch_bounds__(kBlock) void k_sell_dot(
 // wavefront's reads mostly straddle (about 18 cycles each). 192^3, 27 points, y += A x
 // in FP64: 300 -> 93 us; FP32, y = A x: 135 -> 33 us. XCD-contiguous slices (the
 // default) keep the neighbouring planes of x in one L2: 100 -> 93 us against plain
-// block order, where the value stream of k_spmv_sell preferred plain order.
+// block order, where the value stream of k_spmv_sell preferred plain order. Templates
+// in runs of three take k_const_run instead.
 template <typename R, int MASK, bool OVERWRITE, int W, bool XCD>
 __global__ __launch_bounds__(kBlock) void k_spmv_const(size_t nrows, size_t ncols, size_t nslices,
                                                       ConstArg<typename R::V> T, const uint32_t *__restrict__ cmask,
@@ -587,6 +588,117 @@ __global__ __launch_bounds__(kBlock) void k_spmv_const(size_t nrows, size_t ncol
 	} else {
 		y[r] = OVERWRITE ? static_cast<Y>(acc) : static_cast<Y>(R::add(yv, acc));
 	}
+}
+
+// The product with several rows per lane (const_run_fold): RPL * 64 rows per wavefront.
+// 192^3, y += A x in FP64: 93 -> 47 us (4.2 TB/s of its mask, x and y), FP32 y = A x
+// 33 -> 29 us, where the four operations per entry and row bind; staging x in LDS
+// windows instead took 83 and 62 us.
+template <typename R, int MASK, bool OVERWRITE, int DIR>
+__global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols, ConstArg<typename R::V> T,
+                                                     const uint32_t *__restrict__ cmask,
+                                                     const typename R::X *__restrict__ x,
+                                                     typename R::Y *__restrict__ y,
+                                                     const uint8_t *__restrict__ mask, const int *__restrict__ skip) {
+	using A = typename R::A;
+	using Y = typename R::Y;
+	constexpr unsigned N = RowsPerLane<typename R::X>::N;
+	const unsigned bl = xcd_logical_block(blockIdx.x, gridDim.x);
+	const size_t r0 =
+	    (size_t)__builtin_amdgcn_readfirstlane(bl * (kBlock / kWave) + threadIdx.x / kWave) * (kSellRows * N);
+	if (r0 >= nrows) return;  // whole wavefronts leave together
+	const unsigned lane = threadIdx.x % kWave;
+	const size_t r = r0 + (size_t)lane * N;
+	const int stop = skip ? *skip : 0;
+	const bool whole = r + N <= nrows;
+	uint32_t bits[N] = {};
+	Y yv[N] = {};
+	if (whole) {
+		load_run<N>(cmask + r, bits);
+		if (!OVERWRITE) load_run<N>(y + r, yv);
+	} else {
+#pragma unroll
+		for (unsigned i = 0; i < N; ++i)
+			if (r + i < nrows) {
+				bits[i] = cmask[r + i];
+				if (!OVERWRITE) yv[i] = y[r + i];
+			}
+	}
+	if (stop) return;  // a solver loop that has stopped
+	A acc[N];
+	const_run_fold<R, DIR>(T, (long long)r0, lane, bits, (long long)ncols, x, acc);
+#pragma unroll
+	for (unsigned i = 0; i < N; ++i) {
+		if (OVERWRITE) yv[i] = bits[i] == 0 ? static_cast<Y>(R::zero()) : static_cast<Y>(acc[i]);
+		else if (bits[i] != 0) yv[i] = static_cast<Y>(R::add(static_cast<A>(yv[i]), acc[i]));
+	}
+	if (!MASK && whole) {
+		store_run<N>(y + r, yv);
+	} else {
+#pragma unroll
+		for (unsigned i = 0; i < N; ++i) {
+			if (r + i >= nrows || (!OVERWRITE && bits[i] == 0)) continue;
+			if (MASK && (MASK == 1) != (mask[r + i] != 0)) continue;
+			y[r + i] = yv[i];
+		}
+	}
+}
+
+// and with the partials of y.x (overwrite): wavefronts take several groups of rows
+template <typename R, int DIR>
+__global__ __launch_bounds__(kBlock) void k_const_run_dot(size_t nrows, ConstArg<typename R::V> T,
+                                                         const uint32_t *__restrict__ cmask,
+                                                         const typename R::X *__restrict__ x,
+                                                         typename R::Y *__restrict__ y, double *__restrict__ partials,
+                                                         const int *__restrict__ skip) {
+	__shared__ double red[kBlock / kWave];
+	using A = typename R::A;
+	using X = typename R::X;
+	using Y = typename R::Y;
+	constexpr unsigned N = RowsPerLane<X>::N;
+	constexpr size_t kRows = (size_t)kBlock * N;
+	const int stop = skip ? *skip : 0;
+	const unsigned lane = threadIdx.x % kWave;
+	const WorkSplit ws = xcd_split((nrows + kRows - 1) / kRows);
+	double part = 0.0;
+	for (size_t b = ws.first; b < ws.last; b += ws.step) {
+		const size_t r0 = b * kRows + (size_t)__builtin_amdgcn_readfirstlane(threadIdx.x / kWave) * (kSellRows * N);
+		if (r0 >= nrows) continue;  // uniform across the wavefront
+		const size_t r = r0 + (size_t)lane * N;
+		const bool whole = r + N <= nrows;
+		uint32_t bits[N] = {};
+		X xv[N] = {};
+		if (whole) {
+			load_run<N>(cmask + r, bits);
+			load_run<N>(x + r, xv);
+		} else {
+#pragma unroll
+			for (unsigned i = 0; i < N; ++i)
+				if (r + i < nrows) {
+					bits[i] = cmask[r + i];
+					xv[i] = x[r + i];
+				}
+		}
+		if (stop) return;  // uniform over the grid: no wavefront reaches the reduction
+		A acc[N];
+		const_run_fold<R, DIR>(T, (long long)r0, lane, bits, (long long)nrows, x, acc);
+		Y yv[N];
+#pragma unroll
+		for (unsigned i = 0; i < N; ++i) {
+			yv[i] = bits[i] == 0 ? static_cast<Y>(R::zero()) : static_cast<Y>(acc[i]);
+			if (r + i < nrows) part += (double)yv[i] * (double)xv[i];
+		}
+		if (whole) {
+			store_run<N>(y + r, yv);
+		} else {
+#pragma unroll
+			for (unsigned i = 0; i < N; ++i)
+				if (r + i < nrows) y[r + i] = yv[i];
+		}
+	}
+	if (stop) return;
+	part = block_sum(part, red);
+	if (threadIdx.x == 0) partials[blockIdx.x] = part;
 }
 
 // The same product (overwrite) with the partials of y.x: a grid of at most the
@@ -1099,7 +1211,7 @@ static bool const_arg(const Storage &S, const void *val, ConstArg<typename R::V>
 	a.dmax = S.cst.dmax;
 	for (unsigned q = 0; q < kDiaSlots; ++q) {
 		a.d[q] = S.cst.d[q];
-		a.v[q] = sizeof(typename R::V) == 8 ? (typename R::V)S.cst.v64[q] : (typename R::V)S.cst.v32[q];
+		a.v[q] = sizeof(typename R::X) == 8 ? (typename R::V)S.cst.v64[q] : (typename R::V)S.cst.v32[q];
 	}
 	return true;
 }
@@ -1110,6 +1222,17 @@ static void launch_const(int xcd, const Storage &S, const ConstArg<typename R::V
 	const size_t per = kBlock / kSellRows;
 	const size_t grid = (S.n_slices + per - 1) / per;
 	if (grid == 0) return;
+	if (S.cst.run) {  // no slower than a row per lane at any size measured (16^3 to 192^3)
+		const size_t rows = (size_t)kBlock * RowsPerLane<typename R::X>::N;
+#define ALP_CRUN(DD)                                                                                       \
+	hipLaunchKernelGGL((k_const_run<R, MASK, OW, DD>), dim3((S.nmajor + rows - 1) / rows), dim3(kBlock), 0, s, \
+	                   S.nmajor, S.nminor, T, (const uint32_t *)S.cmask, (const typename R::X *)x,             \
+	                   (typename R::Y *)y, mask, skip)
+		if (S.cst.run > 0) ALP_CRUN(1);
+		else ALP_CRUN(-1);
+#undef ALP_CRUN
+		return;
+	}
 #define ALP_CONST(WW, XX)                                                                                      \
 	hipLaunchKernelGGL((k_spmv_const<R, MASK, OW, WW, XX>), dim3(grid), dim3(kBlock), 0, s, S.nmajor, S.nminor,  \
 	                   S.n_slices, T, (const uint32_t *)S.cmask, (const typename R::X *)x, (typename R::Y *)y, mask, skip)
@@ -1155,8 +1278,14 @@ int default_lanes(const Storage &S) {
 }
 
 // the template's value type (patterns have none and never take the form)
+template <typename R, bool P = R::kPattern>
+struct ConstVal {
+	using T = typename ConstRing<R>::T::V;
+};
 template <typename R>
-using ConstV = std::conditional_t<R::kPattern, double, typename R::V>;
+struct ConstVal<R, true> {
+	using T = double;
+};
 
 template <typename R>
 static void dispatch(const Storage &S, const void *val, unsigned descr, void *y, const void *x,
@@ -1170,9 +1299,9 @@ static void dispatch(const Storage &S, const void *val, unsigned descr, void *y,
 	// the constant form where the matrix has it (kernel 5, or 4 when no sliced-ELL
 	// values are kept: the same fold order); it reads neither indices nor values
 	bool cst = false;
-	ConstArg<ConstV<R>> carg;
+	ConstArg<typename ConstVal<R>::T> carg;
 	if constexpr (!R::kPattern) {
-		if (kernel == 5 || (kernel == 4 && !S.sell_val)) cst = const_arg<R>(S, val, carg);
+		if (kernel == 5 || (kernel == 4 && !S.sell_val)) cst = const_arg<typename ConstRing<R>::T>(S, val, carg);
 	}
 	const void *sval = nullptr, *dval = nullptr;
 	bool dia = false;
@@ -1195,7 +1324,7 @@ static void dispatch(const Storage &S, const void *val, unsigned descr, void *y,
 #define ALP_GO(MM, OWV)                                                 \
 	if constexpr (!R::kPattern)                                         \
 		if (cst) {                                                      \
-			launch_const<R, MM, OWV>(S.kernel ? S.lanes : 1, S, carg, x, y, mask, s, skip); \
+			launch_const<typename ConstRing<R>::T, MM, OWV>(S.kernel ? S.lanes : 1, S, carg, x, y, mask, s, skip); \
 			return;                                                     \
 		}                                                               \
 	if (kernel == 4)                                                    \
@@ -1223,13 +1352,27 @@ static bool sell_dot_launch(const Storage &S, const void *val, const void *x, vo
                             unsigned max_partials, unsigned *nparts, const int *skip, hipStream_t s) {
 	const int k = S.kernel ? S.kernel : auto_kernel(S);
 	if (k != 4 && k != 5) return false;
-	ConstArg<typename R::V> carg;
-	if ((k == 5 || !S.sell_val) && const_arg<R>(S, val, carg)) {
+	using RC = typename ConstRing<R>::T;
+	ConstArg<typename RC::V> carg;
+	if ((k == 5 || !S.sell_val) && const_arg<RC>(S, val, carg)) {
 		const size_t nb = (S.n_slices + kBlock / kSellRows - 1) / (kBlock / kSellRows);
 		const unsigned grid = (unsigned)std::min<size_t>(nb, std::min<size_t>(max_partials, fill_blocks(8)));
 		if (grid == 0) return false;
+		if (S.cst.run) {  // no slower than a row per lane at any size measured (16^3 to 192^3)
+			const size_t rows = (size_t)kBlock * RowsPerLane<typename RC::X>::N;
+			const unsigned gr = (unsigned)std::min<size_t>((S.nmajor + rows - 1) / rows,
+			                                               std::min<size_t>(max_partials, fill_blocks(8)));
+#define ALP_CRDOT(DD)                                                                                       \
+	hipLaunchKernelGGL((k_const_run_dot<RC, DD>), dim3(gr), dim3(kBlock), 0, s, S.nmajor, carg,                \
+	                   (const uint32_t *)S.cmask, (const typename R::X *)x, (typename R::Y *)y, partials, skip)
+			if (S.cst.run > 0) ALP_CRDOT(1);
+			else ALP_CRDOT(-1);
+#undef ALP_CRDOT
+			*nparts = gr;
+			return true;
+		}
 #define ALP_CDOT(WW)                                                                                         \
-	hipLaunchKernelGGL((k_const_dot<R, WW>), dim3(grid), dim3(kBlock), 0, s, S.nmajor, S.n_slices, carg,       \
+	hipLaunchKernelGGL((k_const_dot<RC, WW>), dim3(grid), dim3(kBlock), 0, s, S.nmajor, S.n_slices, carg,       \
 	                   (const uint32_t *)S.cmask, (const typename R::X *)x, (typename R::Y *)y, partials, skip)
 		if (carg.w == kDiaFullWidth) ALP_CDOT((int)kDiaFullWidth);
 		else if (carg.w == 7) ALP_CDOT(7);

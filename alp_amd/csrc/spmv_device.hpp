@@ -18,12 +18,15 @@ namespace alp {
 // Each functor gives the additive identity, multiplication of a matrix value
 // (or the pattern's implicit one) with an input element, and the additive
 // fold. V = matrix value type (void for pattern), X = input, Y = output,
-// A = accumulator.
+// A = accumulator. kZeroSkips: folding in the product of a finite matrix value and
+// x = 0 changes no accumulator that started at zero() (a sum from +0 is never -0), so
+// an absent entry can be skipped by clearing its x.
 
 template <typename T>
 struct PlusTimes {
 	using V = T; using X = T; using Y = T; using A = T;
 	static constexpr bool kPattern = false;
+	static constexpr bool kZeroSkips = true;
 	__device__ static A zero() { return A(0); }
 	__device__ static A mul(V a, X x) { return a * x; }
 	__device__ static A add(A a, A b) { return a + b; }
@@ -35,9 +38,31 @@ struct PlusTimes {
 struct PlusTimesF32Acc64 {
 	using V = float; using X = float; using Y = float; using A = double;
 	static constexpr bool kPattern = false;
+	static constexpr bool kZeroSkips = true;
 	__device__ static A zero() { return 0.0; }
 	__device__ static A mul(V a, X x) { return (double)a * (double)x; }
 	__device__ static A add(A a, A b) { return a + b; }
+};
+
+// the same with the matrix value already widened (uniform template values: one
+// conversion on the host instead of one per use)
+struct PlusTimesF32Acc64Wide {
+	using V = double; using X = float; using Y = float; using A = double;
+	static constexpr bool kPattern = false;
+	static constexpr bool kZeroSkips = true;
+	__device__ static A zero() { return 0.0; }
+	__device__ static A mul(V a, X x) { return a * (double)x; }
+	__device__ static A add(A a, A b) { return a + b; }
+};
+
+// the ring that the constant-form kernels run for R
+template <typename R>
+struct ConstRing {
+	using T = R;
+};
+template <>
+struct ConstRing<PlusTimesF32Acc64> {
+	using T = PlusTimesF32Acc64Wide;
 };
 
 // lor-land over a pattern matrix: bytes 0/1 (monoid.hpp:139-147: lor has
@@ -63,6 +88,7 @@ struct PlusPattern {
 struct MinPlus {
 	using V = double; using X = double; using Y = double; using A = double;
 	static constexpr bool kPattern = false;
+	static constexpr bool kZeroSkips = false;
 	__device__ static A zero() { return __builtin_inf(); }
 	__device__ static A mul(V a, X x) { return a + x; }
 	__device__ static A add(A a, A b) { return a < b ? a : b; }
@@ -172,6 +198,31 @@ __device__ __forceinline__ void rows_gather(const uint64_t (&beg)[RR], const uin
 }
 
 // ---- constant form ----------------------------------------------------------------
+// x when bit q of bits is set, else +0: a sign-extended bit field and an AND per word
+// (a compare and a select per word of the accumulator otherwise)
+__device__ __forceinline__ float keep_if(uint32_t bits, unsigned q, float x) {
+	const uint32_t k = (uint32_t)__builtin_amdgcn_sbfe((int)bits, q, 1);
+	return __uint_as_float(__float_as_uint(x) & k);
+}
+__device__ __forceinline__ double keep_if(uint32_t bits, unsigned q, double x) {
+	const uint32_t k = (uint32_t)__builtin_amdgcn_sbfe((int)bits, q, 1);
+	const unsigned long long u = (unsigned long long)__double_as_longlong(x);
+	const uint32_t lo = (uint32_t)u & k, hi = (uint32_t)(u >> 32) & k;
+	return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// entry q of a row with mask bits folded into acc (nothing when bit q is clear)
+template <typename R>
+__device__ __forceinline__ typename R::A const_term(typename R::V v, uint32_t bits, unsigned q, typename R::X x,
+                                                    typename R::A acc) {
+	if constexpr (R::kZeroSkips) {
+		return R::add(R::mul(v, keep_if(bits, q, x)), acc);
+	} else {
+		const typename R::A t = R::add(R::mul(v, x), acc);
+		return (bits >> q) & 1u ? t : acc;
+	}
+}
+
 // The fold of one row of a slice in constant form: r0 is the slice's first row
 // (uniform across the wavefront), the lane's row is r0 + lane with presence mask
 // bits; entry q multiplies x[row + d_q] by v_q, in storage order. Offsets and values
@@ -180,9 +231,10 @@ __device__ __forceinline__ void rows_gather(const uint64_t (&beg)[RR], const uin
 // template's width when known at compile time, else 0.
 //
 // A wavefront whose 64 rows all reach into [0, ncols) with every slot reads x
-// without per-lane conditions (an absent entry's x is in range and dropped by the
-// select below, whatever it holds) and folds without selects when all its rows
-// have every slot; only the slices at the two ends of the matrix mask their loads.
+// without per-lane conditions (an absent entry's x is in range and
+// skipped by const_term, whatever it holds); the slices at the two ends of the matrix clamp
+// the positions, so that their loads are in flight together too. Rows that all have
+// every slot fold without masking x.
 template <typename R, int W>
 __device__ __forceinline__ typename R::A const_fold(const ConstArg<typename R::V> &T, long long r0, unsigned lane,
                                                     uint32_t bits, long long ncols,
@@ -194,33 +246,124 @@ __device__ __forceinline__ typename R::A const_fold(const ConstArg<typename R::V
 	const uint32_t full = w < 32 ? (1u << w) - 1u : 0xFFFFFFFFu;
 	const bool inside = r0 + T.dmin >= 0 && r0 + kSellRows - 1 + T.dmax < ncols;
 	A acc = R::zero();
-	if (inside) {
 #pragma unroll 1
-		for (unsigned q0 = 0; q0 < w; q0 += U) {
-			X xv[U];
+	for (unsigned q0 = 0; q0 < w; q0 += U) {
+		X xv[U];
+		if (inside) {
+#pragma unroll
+			for (unsigned u = 0; u < U; ++u) xv[u] = (x + (r0 + T.d[W ? u : (q0 + u < w ? q0 + u : w - 1)]))[lane];
+		} else {
 #pragma unroll
 			for (unsigned u = 0; u < U; ++u) {
-				const unsigned q = W ? u : (q0 + u < w ? q0 + u : w - 1);
-				xv[u] = (x + (r0 + T.d[q]))[lane];
-			}
-			if (__builtin_amdgcn_ballot_w64(bits != full) == 0) {
-#pragma unroll
-				for (unsigned u = 0; u < U; ++u)
-					if (W || q0 + u < w) acc = R::add(R::mul(T.v[W ? u : q0 + u], xv[u]), acc);
-			} else {
-#pragma unroll
-				for (unsigned u = 0; u < U; ++u)
-					if (W || q0 + u < w) {
-						const A t = R::add(R::mul(T.v[W ? u : q0 + u], xv[u]), acc);
-						acc = (bits >> (q0 + u)) & 1u ? t : acc;
-					}
+				const long long c = r0 + lane + T.d[W ? u : (q0 + u < w ? q0 + u : w - 1)];
+				xv[u] = x[c < 0 ? 0 : c < ncols ? c : ncols - 1];
 			}
 		}
-	} else {
-		for (unsigned q = 0; q < w; ++q)
-			if ((bits >> q) & 1u) acc = R::add(R::mul(T.v[q], (x + (r0 + T.d[q]))[lane]), acc);
+		if (__builtin_amdgcn_ballot_w64(bits != full) == 0) {
+#pragma unroll
+			for (unsigned u = 0; u < U; ++u)
+				if (W || q0 + u < w) acc = R::add(R::mul(T.v[W ? u : q0 + u], xv[u]), acc);
+		} else {
+#pragma unroll
+			for (unsigned u = 0; u < U; ++u)
+				if (W || q0 + u < w) acc = const_term<R>(T.v[W ? u : q0 + u], bits, q0 + u, xv[u], acc);
+		}
 	}
 	return acc;
+}
+
+// Several rows per lane for templates that are nine runs of three consecutive
+// offsets (ConstDia::run; the 27-point stencil's order): a lane owns RPL = 16 /
+// sizeof(x) consecutive rows, whose slots of one run lie in RPL + 2 consecutive
+// elements of x, read by one 16-byte load and one of the rest. A wavefront's reads
+// then move 1.5 to 2 elements per row and run through L1 instead of 3, in a third
+// (FP64) or a sixth (FP32) of the load instructions. Each row's fold keeps its order.
+template <typename X>
+struct RowsPerLane {
+	static constexpr unsigned N = 16 / sizeof(X);
+};
+
+// n consecutive elements, whatever their alignment (global loads need only 4 bytes)
+template <unsigned N, typename X>
+__device__ __forceinline__ void load_run(const X *p, X *out) {
+	typedef X V __attribute__((ext_vector_type(N), aligned(sizeof(X))));
+	const V v = *reinterpret_cast<const V *>(p);
+#pragma unroll
+	for (unsigned i = 0; i < N; ++i) out[i] = v[i];
+}
+
+template <unsigned N, typename X>
+__device__ __forceinline__ void store_run(X *p, const X *in) {
+	typedef X V __attribute__((ext_vector_type(N), aligned(sizeof(X))));
+	V v;
+#pragma unroll
+	for (unsigned i = 0; i < N; ++i) v[i] = in[i];
+	*reinterpret_cast<V *>(p) = v;
+}
+
+// rows r0 + lane * RPL + i, i < RPL (r0 uniform), with masks bits[i]; DIR = the sign of
+// the runs
+template <typename R, int DIR>
+__device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T, long long r0, unsigned lane,
+                                               const uint32_t (&bits)[RowsPerLane<typename R::X>::N], long long ncols,
+                                               const typename R::X *__restrict__ x,
+                                               typename R::A (&acc)[RowsPerLane<typename R::X>::N]) {
+	using A = typename R::A;
+	using X = typename R::X;
+	constexpr unsigned N = RowsPerLane<X>::N, kGroup = 3;  // runs in flight
+	constexpr uint32_t full = (1u << kDiaFullWidth) - 1u;
+	const bool inside = r0 + T.dmin >= 0 && r0 + (long long)(kSellRows * N) - 1 + T.dmax < ncols;
+	bool some = false;
+	uint32_t m[N];
+#pragma unroll
+	for (unsigned i = 0; i < N; ++i) {
+		acc[i] = R::zero();
+		m[i] = bits[i];
+		some |= bits[i] != full;
+	}
+	const bool select = __builtin_amdgcn_ballot_w64(some) != 0;
+	// three runs at a time: unrolled whole, the loads and the template's values of all
+	// nine take 120-190 registers and the occupancy with them
+#pragma unroll 1
+	for (unsigned q0 = 0; q0 < kDiaFullWidth; q0 += 3 * kGroup) {
+		X e[kGroup][N + 2];
+		if (inside) {
+#pragma unroll
+			for (unsigned k = 0; k < kGroup; ++k) {
+				const X *p = (x + (r0 + T.d[q0 + 3 * k + 1] - 1)) + lane * N;
+				load_run<N>(p, e[k]);
+				load_run<2>(p + N, e[k] + N);
+			}
+		} else {  // the two ends of the matrix: clamped positions
+#pragma unroll
+			for (unsigned k = 0; k < kGroup; ++k)
+#pragma unroll
+				for (unsigned i = 0; i < N + 2; ++i) {
+					const long long c = r0 + T.d[q0 + 3 * k + 1] - 1 + lane * N + i;
+					e[k][i] = x[c < 0 ? 0 : c < ncols ? c : ncols - 1];
+				}
+		}
+		if (!select) {
+#pragma unroll
+			for (unsigned k = 0; k < kGroup; ++k)
+#pragma unroll
+				for (unsigned j = 0; j < 3; ++j)
+#pragma unroll
+					for (unsigned i = 0; i < N; ++i)
+						acc[i] = R::add(R::mul(T.v[q0 + 3 * k + j], e[k][i + (DIR > 0 ? j : 2 - j)]), acc[i]);
+		} else {
+#pragma unroll
+			for (unsigned k = 0; k < kGroup; ++k)
+#pragma unroll
+				for (unsigned j = 0; j < 3; ++j)
+#pragma unroll
+					for (unsigned i = 0; i < N; ++i)
+						acc[i] = const_term<R>(T.v[q0 + 3 * k + j], m[i], 3 * k + j, e[k][i + (DIR > 0 ? j : 2 - j)],
+						                       acc[i]);
+#pragma unroll
+			for (unsigned i = 0; i < N; ++i) m[i] >>= 3 * kGroup;
+		}
+	}
 }
 
 // ---- block tile fold (the CSR-stream pattern with a caller epilogue) ----------
