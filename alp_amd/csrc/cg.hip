@@ -8,9 +8,10 @@
 //   k_cg_spmv_dot  temp = A u and one partial sum of temp.u per block, in one pass
 //                  (CSR-vector matrices; on a sliced layout k_sell_dot does the same)
 //   k_cg_update    every block folds the temp.u partials into alpha = sigma / (temp.u);
-//                  x += alpha u, r -= alpha temp and one partial of r.r per block
+//                  r -= alpha temp and one partial of r.r per block
 //   k_cg_dir       every block folds r.r, applies the stopping test (||r|| < tol ||b||,
-//                  :378,437) and, unless done, u = r + (r.r / sigma) u
+//                  :378,437) and, unless done, u' = r + (r.r / sigma) u; every fourth
+//                  iteration, and the last, x += alpha u for the directions since
 // Every reduction has a fixed tree (fixed grid, fixed per-thread strides, the
 // partials folded in index order), so results are run-to-run deterministic.
 // Iterations are enqueued in batches replayed from one captured hipGraph; the
@@ -49,7 +50,11 @@ struct CgState {
 	double r0norm;     // sqrt of the first r.r (inner solves)
 	double tol_true;   // reliable updates: tol * ||b|| for the FP64 residual
 	unsigned long long max_iter;
+	double alpha[4];   // the step lengths of the current group of iterations
 };
+
+// directions kept before the solution takes them (k_cg_dir)
+constexpr int kDirs = 4;
 
 template <typename T>
 struct CgArgs {
@@ -57,13 +62,20 @@ struct CgArgs {
 	const uint64_t *off;
 	const uint32_t *idx;
 	const T *val;
-	T *x, *r, *u, *temp;
+	T *x, *r, *u[kDirs], *temp;  // u: the directions of a group of iterations (k_cg_dir)
 	const T *b;
 	double *partials;  // kMaxPartials doubles: [0, half) p.Ap, [half, 2 half) r.r (or r.z)
 	unsigned *ticket;
 	CgState *st;
 	double *x64 = nullptr;  // set: the solution is FP64 (x unused), x64 += alpha u in FP64
+	int dirs = 1;           // directions u holds: kDirs or 1
 };
+
+template <typename T>
+static void set_dirs(CgArgs<T> &a, void *const *buf, int dirs) {
+	for (int g = 0; g < dirs; ++g) a.u[g] = (T *)buf[g];
+	a.dirs = dirs;
+}
 
 constexpr unsigned kHalfPartials = kMaxPartials / 2;
 
@@ -79,7 +91,7 @@ __device__ __forceinline__ double fold_partials(const double *p, unsigned n, dou
 // ---- kernels ------------------------------------------------------------------
 
 template <int G, int RR, typename T>
-__global__ __launch_bounds__(kBlock) void k_cg_spmv_dot(CgArgs<T> a, const CgScal *in) {
+__global__ __launch_bounds__(kBlock) void k_cg_spmv_dot(CgArgs<T> a, const T *__restrict__ u, const CgScal *in) {
 	__shared__ double lds[kBlock / kWave];
 	if (in->done) return;
 	constexpr unsigned kGroups = kBlock / G;
@@ -101,11 +113,11 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dot(CgArgs<T> a, const CgSca
 			if (row[i] < a.n) {
 				beg[i] = a.off[row[i]];
 				end[i] = a.off[row[i] + 1];
-				if (lane == 0) ur[i] = a.u[row[i]];
+				if (lane == 0) ur[i] = u[row[i]];
 			}
 		}
 		T acc[RR];
-		rows_gather<G, RR, PlusTimes<T>>(beg, end, lane, a.idx, a.val, a.u, acc);
+		rows_gather<G, RR, PlusTimes<T>>(beg, end, lane, a.idx, a.val, u, acc);
 #pragma unroll
 		for (int i = 0; i < RR; ++i) {
 			if (lane == 0 && row[i] < a.n) {
@@ -120,61 +132,158 @@ __global__ __launch_bounds__(kBlock) void k_cg_spmv_dot(CgArgs<T> a, const CgSca
 
 // generic-SpMV path: the partials of temp.u
 template <typename T>
-__global__ __launch_bounds__(kBlock) void k_cg_dot(CgArgs<T> a, const CgScal *in) {
+__global__ __launch_bounds__(kBlock) void k_cg_dot(CgArgs<T> a, const T *u, const CgScal *in) {
 	__shared__ double lds[kBlock / kWave];
 	if (in->done) return;
 	double part = 0.0;
-	grid_for_each<4>(a.n, [&](size_t i) { part += (double)a.temp[i] * (double)a.u[i]; });
+	grid_for_each<4>(a.n, [&](size_t i) { part += (double)a.temp[i] * (double)u[i]; });
 	part = block_sum(part, lds);
 	if (threadIdx.x == 0) a.partials[blockIdx.x] = part;
 }
 
-// alpha = sigma / p.Ap (folded from npap partials); x += alpha u, r -= alpha temp,
-// and the partials of r.r
-template <typename T>
+// Vectors in 16-byte pieces: use(i, V elements) for the whole pieces, U of them per
+// step, whose loads go out before any is used (through pointers that may alias, a
+// loop of load, use and store keeps one piece in flight); the last n % V elements one
+// per thread.
+template <int V, int U, typename Load, typename Use, typename Tail>
+__device__ __forceinline__ void grid_for_pieces(size_t n, Load &&load, Use &&use, Tail &&tail) {
+	const size_t np = n / V, stride = (size_t)gridDim.x * kBlock;
+	const size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
+	for (size_t i = t; i < np; i += U * stride) {
+#pragma unroll
+		for (int u = 0; u < U; ++u)
+			if (i + u * stride < np) load(u, (i + u * stride) * V);
+#pragma unroll
+		for (int u = 0; u < U; ++u)
+			if (i + u * stride < np) use(u, (i + u * stride) * V);
+	}
+	if (t < n - np * V) tail(np * V + t);
+}
+
+// alpha = sigma / p.Ap (folded from npap partials), r -= alpha temp and the partials
+// of r.r. X: also x += alpha u (the preconditioned loop); otherwise k_cg_dir adds it.
+template <typename T, bool X>
 __global__ __launch_bounds__(kBlock) void k_cg_update(CgArgs<T> a, const CgScal *in, unsigned npap) {
 	__shared__ double lds[kBlock / kWave];
 	if (in->done) return;
 	const double pAp = fold_partials(a.partials, npap, lds);
-	const double alpha64 = in->sigma / pAp;
-	const T alpha = (T)alpha64;
+	const T alpha = (T)(in->sigma / pAp);
 	double part = 0.0;
-	if (a.x64) {
+	if (X) {
 		grid_for_each<4>(a.n, [&](size_t i) {
-			a.x64[i] = alpha64 * (double)a.u[i] + a.x64[i];
+			a.x[i] = alpha * a.u[0][i] + a.x[i];
 			const T ri = a.r[i] - alpha * a.temp[i];
 			a.r[i] = ri;
 			part += (double)ri * (double)ri;
 		});
 	} else {
-		grid_for_each<4>(a.n, [&](size_t i) {
-			a.x[i] = alpha * a.u[i] + a.x[i];
-			const T ri = a.r[i] - alpha * a.temp[i];
-			a.r[i] = ri;
-			part += (double)ri * (double)ri;
-		});
+		constexpr int V = 16 / (int)sizeof(T), U = 4;
+		T r[U][V], t[U][V];
+		grid_for_pieces<V, U>(
+		    a.n,
+		    [&](int u, size_t i) {
+			    load_run<V>(a.r + i, r[u]);
+			    load_run<V>(a.temp + i, t[u]);
+		    },
+		    [&](int u, size_t i) {
+#pragma unroll
+			    for (int v = 0; v < V; ++v) {
+				    r[u][v] = r[u][v] - alpha * t[u][v];
+				    part += (double)r[u][v] * (double)r[u][v];
+			    }
+			    store_run<V>(a.r + i, r[u]);
+		    },
+		    [&](size_t i) {
+			    const T ri = a.r[i] - alpha * a.temp[i];
+			    a.r[i] = ri;
+			    part += (double)ri * (double)ri;
+		    });
 	}
 	part = block_sum(part, lds);
 	if (threadIdx.x == 0) a.partials[kHalfPartials + blockIdx.x] = part;
 }
 
 // r.r, the stopping test (sqrt(r.r) < tol ||b||, or the iteration limit;
-// conjugate_gradient.hpp:378,437) and, unless done, u = r + (r.r / sigma) u;
-// block 0 writes the next slot
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in, CgScal *out, unsigned nrr) {
+// conjugate_gradient.hpp:378,437) and, unless done, the next direction
+// u[G + 1] = r + (r.r / sigma) u[G]; block 0 writes the next slot.
+//
+// The solution is updated once in kDirs iterations: iteration G of a group writes its
+// direction beside the previous ones, and the group's last iteration (or the one that
+// stops) adds alpha_0 u[0], ..., alpha_G u[G] to x one after the other, the sums of
+// an update per iteration bit for bit. x costs 16 bytes of traffic per row and
+// iteration otherwise (FP64; the update and direction kernels run at the card's
+// rate): with 4 directions they move 31 instead of 44 bytes per row in mixed
+// precision, 58 instead of 72 in FP64 (dirs_for has the times).
+// K: the group's size, kDirs or 1 (no room for more directions). XT: the solution's type
+// (double with T = float when CgArgs::x64 is set).
+template <typename T, typename XT, int G, int K>
+__global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in, CgScal *out, unsigned npap,
+                                                  unsigned nrr) {
 	__shared__ double lds[kBlock / kWave];
 	if (in->done) {
 		if (blockIdx.x == 0 && threadIdx.x == 0) *out = *in;
 		return;
 	}
+	XT *x;
+	if constexpr (std::is_same<XT, T>::value) x = a.x; else x = a.x64;
+	const double pAp = fold_partials(a.partials, npap, lds);
 	const double rr = fold_partials(a.partials + kHalfPartials, nrr, lds);
+	const double alpha64 = in->sigma / pAp;
 	const unsigned long long iter = in->iter + 1;
 	const bool conv = std::sqrt(rr) < a.st->tol_abs;
 	const bool done = conv || iter >= a.st->max_iter;
-	if (!done) {
-		const T ratio = (T)(rr / in->sigma);
-		grid_for_each<4>(a.n, [&](size_t i) { a.u[i] = ratio * a.u[i] + a.r[i]; });
+	const T ratio = (T)(rr / in->sigma);
+	constexpr int V = 16 / (int)sizeof(T), H = (G + 1) % K;
+	if (done || G == K - 1) {
+		XT alpha[G + 1];
+#pragma unroll
+		for (int g = 0; g < G; ++g) alpha[g] = (XT)a.st->alpha[g];
+		alpha[G] = (XT)alpha64;
+		constexpr int U = sizeof(T) == 8 ? 2 : 1;
+		T w[U][G + 1][V], r[U][V];
+		XT xv[U][V];
+		grid_for_pieces<V, U>(
+		    a.n,
+		    [&](int k, size_t i) {
+#pragma unroll
+			    for (int g = 0; g <= G; ++g) load_run<V>(a.u[g] + i, w[k][g]);
+			    load_run<V>(x + i, xv[k]);
+			    if (!done) load_run<V>(a.r + i, r[k]);
+		    },
+		    [&](int k, size_t i) {
+#pragma unroll
+			    for (int g = 0; g <= G; ++g)
+#pragma unroll
+				    for (int v = 0; v < V; ++v) xv[k][v] = alpha[g] * (XT)w[k][g][v] + xv[k][v];
+			    store_run<V>(x + i, xv[k]);
+			    if (!done) {
+#pragma unroll
+				    for (int v = 0; v < V; ++v) w[k][G][v] = ratio * w[k][G][v] + r[k][v];
+				    store_run<V>(a.u[H] + i, w[k][G]);
+			    }
+		    },
+		    [&](size_t i) {
+			    XT v = x[i];
+#pragma unroll
+			    for (int g = 0; g <= G; ++g) v = alpha[g] * (XT)a.u[g][i] + v;
+			    x[i] = v;
+			    if (!done) a.u[H][i] = ratio * a.u[G][i] + a.r[i];
+		    });
+	} else {
+		constexpr int U = 4;
+		T w[U][V], r[U][V];
+		grid_for_pieces<V, U>(
+		    a.n,
+		    [&](int k, size_t i) {
+			    load_run<V>(a.u[G] + i, w[k]);
+			    load_run<V>(a.r + i, r[k]);
+		    },
+		    [&](int k, size_t i) {
+#pragma unroll
+			    for (int v = 0; v < V; ++v) w[k][v] = ratio * w[k][v] + r[k][v];
+			    store_run<V>(a.u[H] + i, w[k]);
+		    },
+		    [&](size_t i) { a.u[H][i] = ratio * a.u[G][i] + a.r[i]; });
 	}
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		CgScal o;
@@ -184,6 +293,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in
 		o.done = done ? 1 : 0;
 		o.converged = conv ? 1 : 0;
 		*out = o;
+		a.st->alpha[G] = alpha64;  // read by the group's later iterations only
 	}
 }
 
@@ -196,7 +306,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_init(CgArgs<T> a, const double *b
 	grid_for_each<4>(a.n, [&](size_t i) {
 		const T ri = a.b[i] - a.temp[i];
 		a.r[i] = ri;
-		a.u[i] = ri;
+		a.u[0][i] = ri;
 		prr += (double)ri * (double)ri;
 		const double bi = bb_f64 ? bb_f64[i] : (double)bb_t[i];
 		pbb += bi * bi;
@@ -266,9 +376,9 @@ __global__ __launch_bounds__(kBlock) void k_pcg_dir(CgArgs<T> a, const T *z, con
 	const double rz = fold_partials(a.partials + kHalfPartials, nrz, lds);
 	const T ratio = first ? T(0) : (T)(rz / in->sigma);
 	if (first)
-		grid_for_each<4>(a.n, [&](size_t i) { a.u[i] = z[i]; });
+		grid_for_each<4>(a.n, [&](size_t i) { a.u[0][i] = z[i]; });
 	else
-		grid_for_each<4>(a.n, [&](size_t i) { a.u[i] = ratio * a.u[i] + z[i]; });
+		grid_for_each<4>(a.n, [&](size_t i) { a.u[0][i] = ratio * a.u[0][i] + z[i]; });
 	if (blockIdx.x == 0 && threadIdx.x == 0) {
 		CgScal o = *in;
 		o.sigma = rz;
@@ -322,8 +432,10 @@ __global__ __launch_bounds__(kBlock) void k_ru_resid(size_t n, const double *b, 
 	}
 }
 
-// p = r32 + (r32.r32 / sigma) p, or p = r32 on the first call (sigma from slot 0)
-__global__ __launch_bounds__(kBlock) void k_ru_dir(size_t n, const float *r32, float *p, const double *partials,
+// p = r32 + (r32.r32 / sigma) last, or p = r32 on the first call (sigma from slot 0); last,
+// the direction of the segment's last iteration, may be p
+__global__ __launch_bounds__(kBlock) void k_ru_dir(size_t n, const float *r32, const float *last, float *p,
+                                                  const double *partials,
                                                   unsigned np, const CgState *st, int first) {
 	__shared__ double lds[kBlock / kWave];
 	const double rr = block_sum_partials(partials + kQuarterPartials, np, lds);
@@ -332,7 +444,7 @@ __global__ __launch_bounds__(kBlock) void k_ru_dir(size_t n, const float *r32, f
 		return;
 	}
 	const float beta = (float)(rr / st->s[0].sigma);
-	grid_for_each<4>(n, [&](size_t i) { p[i] = beta * p[i] + r32[i]; });
+	grid_for_each<4>(n, [&](size_t i) { p[i] = beta * last[i] + r32[i]; });
 }
 
 // one block: the state after a reliable update (both slots), the FP64 stopping
@@ -453,8 +565,7 @@ struct CgSlot {
 		for (void *p : bufs) hipFree(p);
 	}
 	// buffers of the given byte sizes; reallocated (and the graph dropped) when they change
-	alp_rc_t buffers(std::initializer_list<size_t> want, void **out) {
-		const std::vector<size_t> w(want);
+	alp_rc_t buffers(const std::vector<size_t> &w, void **out) {
 		if (w != sizes) {
 			drop_graph();
 			for (void *p : bufs) hipFree(p);
@@ -471,6 +582,32 @@ struct CgSlot {
 		return ALP_SUCCESS;
 	}
 };
+
+// How many directions an iteration's group keeps: kDirs, except where the vectors of
+// an iteration (n rows of `others` bytes for x, r and A u, 4 for the masks of a
+// constant form, and the directions of dir bytes) stay in the 256 MB Infinity Cache
+// with one direction but not with kDirs: the older directions then cost more than x.
+// FP64 at 176^3 and 192^3: 98 and 130 us per iteration with one, 100 and 135 with
+// four; 128^3 and 256^3: 50 and 360 with one, 48 and 336 with four. Mixed precision
+// at 128^3, 192^3, 256^3: 41.6, 102, 228 with one, 39.1, 94.3, 208 with four.
+static int dirs_for(size_t n, size_t others, size_t dir) {
+	constexpr size_t kCache = size_t(256) << 20;
+	const size_t one = n * (others + 4 + dir), all = n * (others + 4 + kDirs * dir);
+	return one <= kCache && all > kCache ? 1 : kDirs;
+}
+
+// the buffers of sizes `fixed` and after them `dirs` direction vectors of dir bytes, or
+// one where memory does not suffice (dirs then says so); out: all of them in that order
+static alp_rc_t cg_buffers(CgSlot &slot, std::initializer_list<size_t> fixed, size_t dir, void **out, int &dirs) {
+	for (;;) {
+		std::vector<size_t> want(fixed);
+		want.insert(want.end(), (size_t)dirs, dir);
+		const alp_rc_t rc = slot.buffers(want, out);
+		if (rc != ALP_OUTOFMEM || dirs == 1) return rc;
+		(void)hipGetLastError();
+		dirs = 1;
+	}
+}
 
 enum CgSlotId {
 	kSlotFp64 = 0,
@@ -542,21 +679,23 @@ struct CgRunner {
 	const CgScal *slot_in(int p) const { return &a.st->s[p]; }
 	CgScal *slot_out(int p) const { return &a.st->s[1 - p]; }
 
-	// the part of an iteration up to the stopping test, reading slot p: temp = A u,
-	// the partials of p.Ap, alpha, x, r and the partials of r.r
-	alp_rc_t step(hipStream_t s, int p) {
+	// the part of an iteration up to the stopping test, reading slot p: temp = A u[g],
+	// the partials of p.Ap (*np_out of them), alpha, r and the partials of r.r; with_x
+	// also x (then g = 0)
+	alp_rc_t step(hipStream_t s, int p, int g, bool with_x, unsigned *np_out = nullptr) {
 		const CgScal *in = slot_in(p);
+		const T *u = a.u[g];
 		unsigned npap = gvec;
 		if (fused) {
 			npap = gspmv;
 #define ALP_CG_CASE(GG)                                                                               \
 	case GG:                                                                                          \
 		if (RR == 4)                                                                                  \
-			hipLaunchKernelGGL((k_cg_spmv_dot<GG, 4, T>), dim3(gspmv), dim3(kBlock), 0, s, a, in);    \
+			hipLaunchKernelGGL((k_cg_spmv_dot<GG, 4, T>), dim3(gspmv), dim3(kBlock), 0, s, a, u, in); \
 		else if (RR == 2)                                                                             \
-			hipLaunchKernelGGL((k_cg_spmv_dot<GG, 2, T>), dim3(gspmv), dim3(kBlock), 0, s, a, in);    \
+			hipLaunchKernelGGL((k_cg_spmv_dot<GG, 2, T>), dim3(gspmv), dim3(kBlock), 0, s, a, u, in); \
 		else                                                                                          \
-			hipLaunchKernelGGL((k_cg_spmv_dot<GG, 1, T>), dim3(gspmv), dim3(kBlock), 0, s, a, in);    \
+			hipLaunchKernelGGL((k_cg_spmv_dot<GG, 1, T>), dim3(gspmv), dim3(kBlock), 0, s, a, u, in); \
 		break;
 			switch (G) {
 				ALP_CG_CASE(2)
@@ -573,28 +712,61 @@ struct CgRunner {
 			// on a sliced layout the p.Ap partials come out of the product itself
 			const int kind = std::is_same<T, double>::value ? 0 : (acc64 ? 2 : 1);
 			unsigned np = 0;
-			if (spmv_dot(S, vt, kind, a.u, a.temp, a.partials, kHalfPartials, &np, &in->done, s)) {
+			if (spmv_dot(S, vt, kind, u, a.temp, a.partials, kHalfPartials, &np, &in->done, s)) {
 				npap = np;
 			} else {
 				// for an FP64 matrix the FP32 semiring selects its FP32 value copy
 				if (acc64 && std::is_same<T, float>::value)
-					ALP_TRY(spmv_f32_acc64(S, (float *)a.temp, (const float *)a.u, s, &in->done));
+					ALP_TRY(spmv_f32_acc64(S, (float *)a.temp, (const float *)u, s, &in->done));
 				else
 					ALP_TRY(spmv(S, vt,
 					             std::is_same<T, float>::value ? ALP_PLUS_TIMES_F32 : ALP_PLUS_TIMES_F64,
-					             ALP_DESC_OVERWRITE, a.temp, a.u, nullptr, s, &in->done));
-				hipLaunchKernelGGL(k_cg_dot<T>, dim3(gvec), dim3(kBlock), 0, s, a, in);
+					             ALP_DESC_OVERWRITE, a.temp, u, nullptr, s, &in->done));
+				hipLaunchKernelGGL(k_cg_dot<T>, dim3(gvec), dim3(kBlock), 0, s, a, u, in);
 			}
 		}
-		hipLaunchKernelGGL(k_cg_update<T>, dim3(gvec), dim3(kBlock), 0, s, a, in, npap);
+		if (with_x)
+			hipLaunchKernelGGL((k_cg_update<T, true>), dim3(gvec), dim3(kBlock), 0, s, a, in, npap);
+		else
+			hipLaunchKernelGGL((k_cg_update<T, false>), dim3(gvec), dim3(kBlock), 0, s, a, in, npap);
 		ALP_LAUNCH_CHECK();
+		if (np_out) *np_out = npap;
 		return ALP_SUCCESS;
 	}
 
-	// one whole iteration from slot p into slot 1 - p
-	alp_rc_t iteration(hipStream_t s, int p) {
-		ALP_TRY(step(s, p));
-		hipLaunchKernelGGL(k_cg_dir<T>, dim3(gvec), dim3(kBlock), 0, s, a, slot_in(p), slot_out(p), gvec);
+	template <typename XT>
+	void launch_dir(hipStream_t s, int p, int g, unsigned npap) {
+#define ALP_CG_DIR_K(GG, KK)                                                                                   \
+	hipLaunchKernelGGL((k_cg_dir<T, XT, GG, KK>), dim3(gvec), dim3(kBlock), 0, s, a, slot_in(p), slot_out(p), npap, \
+	                   gvec)
+#define ALP_CG_DIR(GG)               \
+	case GG:                         \
+		ALP_CG_DIR_K(GG, kDirs);     \
+		break;
+		if (a.dirs == 1) {
+			ALP_CG_DIR_K(0, 1);
+			return;
+		}
+		switch (g) {
+			ALP_CG_DIR(0)
+			ALP_CG_DIR(1)
+			ALP_CG_DIR(2)
+			ALP_CG_DIR(3)
+			default: break;
+		}
+#undef ALP_CG_DIR
+#undef ALP_CG_DIR_K
+		static_assert(kDirs == 4, "one case per direction");
+	}
+
+	// iteration number i of a batch (whole): from slot i % 2 into the other one, with
+	// direction i % a.dirs
+	alp_rc_t iteration(hipStream_t s, int i) {
+		unsigned npap = 0;
+		const int g = i % a.dirs;
+		ALP_TRY(step(s, i % 2, g, false, &npap));
+		if (a.x64) launch_dir<double>(s, i % 2, g, npap);
+		else launch_dir<T>(s, i % 2, g, npap);
 		ALP_LAUNCH_CHECK();
 		return ALP_SUCCESS;
 	}
@@ -607,7 +779,7 @@ struct CgRunner {
 	// instantiated, so the run allocates nothing)
 	alp_rc_t run(hipStream_t s, CgState *h_state, CgSlot *slot = nullptr, bool capture = true) {
 		const int batch = 16;
-		static_assert(batch % 2 == 0, "batches start and end in slot 0");
+		static_assert(batch % 2 == 0 && batch % kDirs == 0, "batches start and end in slot 0 with no direction pending");
 		hipGraphExec_t exec = nullptr;
 		hipGraph_t graph = nullptr;
 		bool use_graph = false;
@@ -622,7 +794,7 @@ struct CgRunner {
 			if (slot) slot->drop_graph();
 			if (s != nullptr && hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) == hipSuccess) {
 				alp_rc_t rc = ALP_SUCCESS;
-				for (int i = 0; i < batch && rc == ALP_SUCCESS; ++i) rc = iteration(s, i % 2);
+				for (int i = 0; i < batch && rc == ALP_SUCCESS; ++i) rc = iteration(s, i);
 				if (hipStreamEndCapture(s, &graph) == hipSuccess && rc == ALP_SUCCESS &&
 				    hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess)
 					use_graph = true;
@@ -637,14 +809,14 @@ struct CgRunner {
 		}
 		auto launch = [&]() -> alp_rc_t {
 			if (use_graph) return hipGraphLaunch(exec, s) == hipSuccess ? ALP_SUCCESS : ALP_PANIC;
-			for (int i = 0; i < batch; ++i) ALP_TRY(iteration(s, i % 2));
+			for (int i = 0; i < batch; ++i) ALP_TRY(iteration(s, i));
 			return ALP_SUCCESS;
 		};
 		alp_rc_t rc = ALP_SUCCESS;
 		int tail = 0;  // iterations to launch directly instead of the next batch
 		for (;;) {
 			if (tail > 0) {
-				for (int i = 0; i < tail && rc == ALP_SUCCESS; ++i) rc = iteration(s, i % 2);
+				for (int i = 0; i < tail && rc == ALP_SUCCESS; ++i) rc = iteration(s, i);
 				if (rc != ALP_SUCCESS) break;
 			} else if ((rc = launch()) != ALP_SUCCESS) {
 				break;
@@ -675,12 +847,14 @@ static alp_rc_t cg_fp64(alp_hip_matrix_t A, Storage &S, const double *b, double 
 	const size_t n = A->nrows;
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, &S == &A->ccs ? kSlotTransposed : kSlotFp64);
-	void *bp[4];
-	ALP_TRY(slot.buffers({8 * n, 8 * n, 8 * n, sizeof(CgState)}, bp));
-	double *r = (double *)bp[0], *u = (double *)bp[1], *temp = (double *)bp[2];
-	CgState *st = (CgState *)bp[3];
-	CgArgs<double> a{n, S.off, S.idx, (const double *)S.val, x, r, u, temp, b,
+	void *bp[3 + kDirs];
+	int dirs = dirs_for(n, 24, 8);
+	ALP_TRY(cg_buffers(slot, {8 * n, 8 * n, sizeof(CgState)}, 8 * n, bp, dirs));
+	double *r = (double *)bp[0], *temp = (double *)bp[1];
+	CgState *st = (CgState *)bp[2];
+	CgArgs<double> a{n, S.off, S.idx, (const double *)S.val, x, r, {}, temp, b,
 	                 ctx().d_partials, ctx().d_tickets, st};
+	set_dirs(a, bp + 3, dirs);
 	// temp = A x; r = b - temp; u = r; sigma = r.r; tol *= sqrt(b.b) (:332-378)
 	ALP_TRY(spmv(S, ALP_VAL_F64, ALP_PLUS_TIMES_F64, ALP_DESC_OVERWRITE, temp, x, nullptr, s));
 	ALP_TRY(cg_prelude(a, (const double *)b, (const double *)nullptr, tol, max_iter, s));
@@ -698,15 +872,17 @@ static alp_rc_t cg_mixed(alp_hip_matrix_t A, Storage &S, const double *b, double
 	ALP_TRY(storage_ensure_f32(S, A->nnz));
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, &S == &A->ccs ? kSlotMixedInnerT : kSlotMixedInner);
-	void *bp[9];
-	ALP_TRY(slot.buffers({8 * n, 8 * n, 4 * n, 4 * n, 4 * n, 4 * n, 4 * n, sizeof(CgState), sizeof(IrState)}, bp));
+	void *bp[8 + kDirs];
+	int dirs = dirs_for(n, 12, 4);
+	ALP_TRY(cg_buffers(slot, {8 * n, 8 * n, 4 * n, 4 * n, 4 * n, 4 * n, sizeof(CgState), sizeof(IrState)}, 4 * n, bp,
+	                   dirs));
 	double *r64 = (double *)bp[0], *t64 = (double *)bp[1];
-	float *x32 = (float *)bp[2], *r32 = (float *)bp[3], *u32 = (float *)bp[4], *temp32 = (float *)bp[5],
-	      *b32 = (float *)bp[6];
-	CgState *st = (CgState *)bp[7];
-	IrState *ir = (IrState *)bp[8];
-	CgArgs<float> a{n, S.off, S.idx, S.val32, x32, r32, u32, temp32, b32,
+	float *x32 = (float *)bp[2], *r32 = (float *)bp[3], *temp32 = (float *)bp[4], *b32 = (float *)bp[5];
+	CgState *st = (CgState *)bp[6];
+	IrState *ir = (IrState *)bp[7];
+	CgArgs<float> a{n, S.off, S.idx, S.val32, x32, r32, {}, temp32, b32,
 	                ctx().d_partials, ctx().d_tickets, st};
+	set_dirs(a, bp + 8, dirs);
 	CgRunner<float> runner(S, a);
 	const double inner_tol = 1e-5;
 	size_t total = 0;
@@ -755,14 +931,16 @@ static alp_rc_t cg_reliable(alp_hip_matrix_t A, Storage &S, const double *b, dou
 	ALP_TRY(storage_ensure_f32(S, A->nnz));
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, &S == &A->ccs ? kSlotReliableT : kSlotReliable);
-	void *bp[6];
-	ALP_TRY(slot.buffers({8 * n, 4 * n, 4 * n, 4 * n, sizeof(CgState), 4 * n}, bp));
+	void *bp[5 + kDirs];
+	int dirs = dirs_for(n, x_fp64 ? 16 : 12, 4);
+	ALP_TRY(cg_buffers(slot, {8 * n, 4 * n, 4 * n, 4 * n, sizeof(CgState)}, 4 * n, bp, dirs));
 	double *t64 = (double *)bp[0];
-	float *r32 = (float *)bp[1], *p32 = (float *)bp[2], *ap32 = (float *)bp[3], *x32 = (float *)bp[5];
+	float *r32 = (float *)bp[1], *ap32 = (float *)bp[2], *x32 = (float *)bp[3];
 	CgState *st = (CgState *)bp[4];
 	// a segment's iterations accumulate their update of x in FP32 (x32); it is
 	// folded into the FP64 x before each FP64 residual (group-wise update)
-	CgArgs<float> a{n, S.off, S.idx, S.val32, x32, r32, p32, ap32, nullptr, ctx().d_partials, ctx().d_tickets, st};
+	CgArgs<float> a{n, S.off, S.idx, S.val32, x32, r32, {}, ap32, nullptr, ctx().d_partials, ctx().d_tickets, st};
+	set_dirs(a, bp + 5, dirs);
 	if (x_fp64) a.x64 = x;  // x32 then stays zero and the fold below adds nothing
 	CgRunner<float> runner(S, a, ALP_VAL_F64, true);
 	unsigned g = vec_grid(n);
@@ -770,6 +948,7 @@ static alp_rc_t cg_reliable(alp_hip_matrix_t A, Storage &S, const double *b, dou
 	double *part = ctx().d_partials;
 	CgState h{};
 	const unsigned gf = (unsigned)std::min<size_t>(fill_blocks(8), (n + kBlock - 1) / kBlock);
+	int last = 0;  // the direction of the segment's last iteration: the next one starts from it
 	for (int first = 1;; first = 0) {
 		// x += x32 (the last segment's update), x32 = 0; then r = b - A x in FP64;
 		// r32, p and the state from it
@@ -777,8 +956,8 @@ static alp_rc_t cg_reliable(alp_hip_matrix_t A, Storage &S, const double *b, dou
 			hipLaunchKernelGGL(k_ru_fold, dim3(gf ? gf : 1), dim3(kBlock), 0, s, n, x, x32, first);
 		ALP_TRY(spmv(S, ALP_VAL_F64, ALP_PLUS_TIMES_F64, ALP_DESC_OVERWRITE, t64, x, nullptr, s));
 		hipLaunchKernelGGL(k_ru_resid, dim3(g), dim3(kBlock), 0, s, n, b, (const double *)t64, r32, part, first);
-		hipLaunchKernelGGL(k_ru_dir, dim3(g), dim3(kBlock), 0, s, n, (const float *)r32, p32, (const double *)part, g,
-		                   (const CgState *)st, first);
+		hipLaunchKernelGGL(k_ru_dir, dim3(g), dim3(kBlock), 0, s, n, (const float *)r32, (const float *)a.u[last],
+		                   a.u[0], (const double *)part, g, (const CgState *)st, first);
 		hipLaunchKernelGGL(k_ru_fin, dim3(1), dim3(kBlock), 0, s, (const double *)part, g, st, tol, delta,
 		                   (unsigned long long)max_iter, first);
 		ALP_LAUNCH_CHECK();
@@ -787,7 +966,9 @@ static alp_rc_t cg_reliable(alp_hip_matrix_t A, Storage &S, const double *b, dou
 		if (h.s[0].done) break;
 		// FP32 iterations (the update of x accumulated in x32) until the recurrence
 		// residual reaches the segment's threshold
+		const unsigned long long before = h.s[0].iter;
 		ALP_TRY(runner.run(s, &h, &slot));
+		last = (int)((h.s[0].iter - before + a.dirs - 1) % a.dirs);
 	}
 	*iters = h.s[0].iter;
 	*residual = h.s[0].rr;
@@ -809,11 +990,13 @@ alp_rc_t cg_native(alp_hip_matrix_s *A, const T *b, T *x, size_t max_iter, doubl
 	Storage &S = A->crs;
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, std::is_same<T, float>::value ? kSlotNativeF32 : kSlotNativeF64);
-	void *bp[5];
-	ALP_TRY(slot.buffers({sizeof(T) * n, sizeof(T) * n, sizeof(T) * n, sizeof(CgState), sizeof(T) * n}, bp));
-	T *r = (T *)bp[0], *u = (T *)bp[1], *temp = (T *)bp[2], *z = (T *)bp[4];
-	CgState *st = (CgState *)bp[3];
-	CgArgs<T> a{n, S.off, S.idx, (const T *)S.val, x, r, u, temp, b, ctx().d_partials, ctx().d_tickets, st};
+	void *bp[4 + kDirs];
+	int dirs = pc.fn ? 1 : dirs_for(n, 3 * sizeof(T), sizeof(T));
+	ALP_TRY(cg_buffers(slot, {sizeof(T) * n, sizeof(T) * n, sizeof(CgState), sizeof(T) * n}, sizeof(T) * n, bp, dirs));
+	T *r = (T *)bp[0], *temp = (T *)bp[1], *z = (T *)bp[3];
+	CgState *st = (CgState *)bp[2];
+	CgArgs<T> a{n, S.off, S.idx, (const T *)S.val, x, r, {}, temp, b, ctx().d_partials, ctx().d_tickets, st};
+	set_dirs(a, bp + 4, dirs);
 	const alp_semiring_t ring = vt == ALP_VAL_F32 ? ALP_PLUS_TIMES_F32 : ALP_PLUS_TIMES_F64;
 	ALP_TRY(spmv(S, vt, ring, ALP_DESC_OVERWRITE, temp, x, nullptr, s));
 	const double *bb64 = std::is_same<T, double>::value ? (const double *)b : nullptr;
@@ -837,7 +1020,7 @@ alp_rc_t cg_native(alp_hip_matrix_s *A, const T *b, T *x, size_t max_iter, doubl
 		const unsigned g = vec_grid(n);
 		for (size_t it = 0;; ++it) {
 			if (it > 0) {
-				ALP_TRY(runner.step(s, 1));
+				ALP_TRY(runner.step(s, 1, 0, true));
 				hipLaunchKernelGGL(k_cg_check<T>, dim3(1), dim3(kBlock), 0, s, a, runner.slot_in(1),
 				                   runner.slot_out(1), g);
 				ALP_LAUNCH_CHECK();
@@ -924,7 +1107,7 @@ ALP_EXPORT alp_rc_t alp_hip_cg_noalloc(alp_hip_matrix_t A, const double *b, doub
 	double *partials = reinterpret_cast<double *>(base + 256);
 	double *r = partials + kMaxPartials, *u = r + n, *temp = u + n;
 	static_assert(sizeof(CgState) <= 256, "the state block fits its 256 bytes");
-	CgArgs<double> a{n, S.off, S.idx, (const double *)S.val, x, r, u, temp, b, partials, nullptr, st};
+	CgArgs<double> a{n, S.off, S.idx, (const double *)S.val, x, r, {u}, temp, b, partials, nullptr, st};
 	ALP_TRY(spmv(S, ALP_VAL_F64, ALP_PLUS_TIMES_F64, ALP_DESC_OVERWRITE, temp, x, nullptr, s));
 	ALP_TRY(cg_prelude(a, (const double *)b, (const double *)nullptr, tol, max_iter, s));
 	CgRunner<double> runner(S, a);
