@@ -245,9 +245,20 @@ struct ConstDia {
 	// 1 / -1: the template is kDiaFullWidth / 3 runs of three offsets going up / down
 	// by one; 0: it is not
 	int run = 0;
+	// the template gives the values too; else (run form) only the offsets, and the
+	// rows' values are kept in slot order (run_pos)
+	bool uniform = false;
 	double v64[kDiaSlots] = {};  // the values (FP64 matrices) and their FP32 copies,
 	float v32[kDiaSlots] = {};   // or the values of an FP32 matrix
 };
+
+// Where slot q of row r sits among the values of a matrix in run form whose template
+// has offsets only: blocks of kRunRows rows, slot by slot, so that the 16 bytes of a
+// lane's consecutive rows are one load (0 where a row lacks the slot).
+constexpr unsigned kRunRows = 256;
+__host__ __device__ __forceinline__ size_t run_pos(size_t r, unsigned q) {
+	return r / kRunRows * (kRunRows * (size_t)kDiaFullWidth) + (size_t)q * kRunRows + r % kRunRows;
+}
 
 // the template as a kernel argument, with values of type V
 template <typename V>
@@ -260,9 +271,12 @@ struct ConstArg {
 
 // Detects the constant form over rows [row0, row1) in slices [s0, s1) (slice rows
 // as in dia_build) and writes the slices' presence masks (indexed by slice and
-// lane) to mask; C.w stays 0 when some row does not fit. Blocking.
+// lane) to mask; C.w stays 0 when some row does not fit. With offsets_only, rows that
+// fit in their offsets but not their values give a template that is not uniform,
+// provided it is in runs. Blocking.
 alp_rc_t const_detect(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
-                      const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask);
+                      const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask,
+                      bool offsets_only = false);
 bool const_dia_enabled();
 
 struct Storage {
@@ -296,10 +310,12 @@ struct Storage {
 	size_t n_slices = 0;
 	size_t sell_entries = 0;
 	DiaSlices dia;                 // diagonal form of the slices that have it
-	// all rows in constant form (cst.w > 0): the template and the rows' masks; the
+	// all rows fit one template (cst.w > 0): the template and the rows' masks; the
 	// sliced-ELL and diagonal forms then keep no values
 	ConstDia cst;
 	uint32_t *cmask = nullptr;
+	void *rval = nullptr;          // values at run_pos of a template that is not uniform
+	float *rval32 = nullptr;       // and their FP32 copy when the matrix has one
 	// rows longer than kLongRow nonzeros, for the CSR-stream path: split into
 	// chunks of kChunk nonzeros that separate blocks fold into partials, then one
 	// thread per long row folds its partials in chunk order (deterministic)

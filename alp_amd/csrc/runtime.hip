@@ -524,7 +524,7 @@ __global__ void k_const_template(size_t row0, const uint64_t *off, const uint32_
 // against the template's in order. The template's offsets are distinct (one row
 // stores a column once), so a row that is a subsequence is matched completely.
 // *bad is set when some row is not (it counts the slices seen before the rest left).
-template <typename V>
+template <typename V, bool VALUES>
 __global__ __launch_bounds__(kBlock) void k_const_match(size_t s0, size_t s1, size_t row1, const uint32_t *srow,
                                                        const uint64_t *off, const uint32_t *idx, const V *val,
                                                        const ConstTemplate *T, uint32_t *mask, unsigned *bad) {
@@ -544,9 +544,11 @@ __global__ __launch_bounds__(kBlock) void k_const_match(size_t s0, size_t s1, si
 		if (j >= len) break;
 		if ((long long)idx[b + j] - (long long)r != T->d[q]) continue;
 		unsigned long long u = 0;
-		const V v = val[b + j];
-		__builtin_memcpy(&u, &v, sizeof(V));
-		if (u == T->bits[q]) {
+		if (VALUES) {
+			const V v = val[b + j];
+			__builtin_memcpy(&u, &v, sizeof(V));
+		}
+		if (!VALUES || u == T->bits[q]) {
 			bits |= 1u << q;
 			++j;
 		}
@@ -563,7 +565,8 @@ bool const_dia_enabled() {
 
 template <typename V>
 static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
-                               const uint64_t *off, const uint32_t *idx, const V *val, uint32_t *mask) {
+                               const uint64_t *off, const uint32_t *idx, const V *val, uint32_t *mask,
+                               bool offsets_only) {
 	struct Work {
 		unsigned long long best;
 		unsigned bad, pad;
@@ -582,52 +585,81 @@ static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0,
 	ALP_LAUNCH_CHECK();
 	ALP_HIP_TRY(copy_sync(&h, d, sizeof(Work), hipMemcpyDeviceToHost));
 	if (h.t.w == 0 || h.t.w > kDiaSlots) return ALP_SUCCESS;
-	for (unsigned q = 0; q < h.t.w; ++q) {
-		V v;
-		__builtin_memcpy(&v, &h.t.bits[q], sizeof(V));
-		if (!std::isfinite((double)v) || !std::isfinite((float)v)) return ALP_SUCCESS;  // absent entries fold v * 0
+	ConstDia N;
+	N.w = h.t.w;
+	N.uniform = true;
+	N.dmin = INT32_MAX;
+	N.dmax = INT32_MIN;
+	for (unsigned q = 0; q < N.w; ++q) {
 		if (h.t.d[q] < INT32_MIN || h.t.d[q] > INT32_MAX) return ALP_SUCCESS;
 		for (unsigned p = 0; p < q; ++p)
 			if (h.t.d[p] == h.t.d[q]) return ALP_SUCCESS;  // a column stored twice: the diagonal form keeps it
-	}
-	const size_t per = kBlock / kSellRows;
-	hipLaunchKernelGGL(k_const_match<V>, dim3((s1 - s0 + per - 1) / per), dim3(kBlock), 0, s, s0, s1, row1, srow, off,
-	                   idx, val, (const ConstTemplate *)&d->t, mask, &d->bad);
-	ALP_LAUNCH_CHECK();
-	ALP_HIP_TRY(copy_sync(&h.bad, &d->bad, sizeof(unsigned), hipMemcpyDeviceToHost));
-	if (h.bad) return ALP_SUCCESS;
-	C.w = h.t.w;
-	C.dmin = INT32_MAX;
-	C.dmax = INT32_MIN;
-	for (unsigned q = 0; q < C.w; ++q) {
 		V v;
 		__builtin_memcpy(&v, &h.t.bits[q], sizeof(V));
-		C.d[q] = (int32_t)h.t.d[q];
-		C.v64[q] = (double)v;
-		C.v32[q] = (float)v;
-		C.dmin = std::min(C.dmin, C.d[q]);
-		C.dmax = std::max(C.dmax, C.d[q]);
+		N.d[q] = (int32_t)h.t.d[q];
+		N.v64[q] = (double)v;
+		N.v32[q] = (float)v;
+		// absent entries fold v * 0
+		if (!std::isfinite(N.v64[q]) || !std::isfinite(N.v32[q])) N.uniform = false;
+		N.dmin = std::min(N.dmin, N.d[q]);
+		N.dmax = std::max(N.dmax, N.d[q]);
 	}
-	if (C.w == kDiaFullWidth) {
-		C.run = C.d[1] > C.d[0] ? 1 : -1;
-		for (unsigned q = 0; q < C.w; q += 3)
-			if ((int64_t)C.d[q + 1] - C.d[q] != C.run || (int64_t)C.d[q + 2] - C.d[q + 1] != C.run) {
-				C.run = 0;
+	if (N.w == kDiaFullWidth) {
+		N.run = N.d[1] > N.d[0] ? 1 : -1;
+		for (unsigned q = 0; q < N.w; q += 3)
+			if ((int64_t)N.d[q + 1] - N.d[q] != N.run || (int64_t)N.d[q + 2] - N.d[q + 1] != N.run) {
+				N.run = 0;
 				break;
 			}
+	}
+	const unsigned blocks = (unsigned)((s1 - s0 + kBlock / kSellRows - 1) / (kBlock / kSellRows));
+	for (int values : {1, 0}) {
+		if (values ? !N.uniform : !offsets_only || N.run == 0) continue;
+		if (!values) ALP_HIP_TRY(hipMemsetAsync(&d->bad, 0, sizeof(unsigned), s));
+		if (values)
+			hipLaunchKernelGGL((k_const_match<V, true>), dim3(blocks), dim3(kBlock), 0, s, s0, s1, row1, srow, off, idx,
+			                   val, (const ConstTemplate *)&d->t, mask, &d->bad);
+		else
+			hipLaunchKernelGGL((k_const_match<V, false>), dim3(blocks), dim3(kBlock), 0, s, s0, s1, row1, srow, off, idx,
+			                   val, (const ConstTemplate *)&d->t, mask, &d->bad);
+		ALP_LAUNCH_CHECK();
+		ALP_HIP_TRY(copy_sync(&h.bad, &d->bad, sizeof(unsigned), hipMemcpyDeviceToHost));
+		if (h.bad) continue;
+		N.uniform = values != 0;
+		C = N;
+		break;
 	}
 	return ALP_SUCCESS;
 }
 
 alp_rc_t const_detect(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
-                      const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask) {
+                      const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask,
+                      bool offsets_only) {
 	C = ConstDia();
 	if (row1 <= row0 || s1 <= s0 || !val) return ALP_SUCCESS;
 	if (value_type == ALP_VAL_F64)
-		return const_detect_t<double>(C, row0, row1, s0, s1, srow, off, idx, (const double *)val, mask);
+		return const_detect_t<double>(C, row0, row1, s0, s1, srow, off, idx, (const double *)val, mask, offsets_only);
 	if (value_type == ALP_VAL_F32)
-		return const_detect_t<float>(C, row0, row1, s0, s1, srow, off, idx, (const float *)val, mask);
+		return const_detect_t<float>(C, row0, row1, s0, s1, srow, off, idx, (const float *)val, mask, offsets_only);
 	return ALP_SUCCESS;
+}
+
+// values at run_pos from the CRS values: row r's entry popcount(mask below q) at slot
+// q, zeros where the mask has none and after the last row
+template <typename V>
+__global__ __launch_bounds__(kBlock) void k_run_fill(size_t nrows, size_t padded, const uint64_t *off,
+                                                    const uint32_t *mask, const V *val, const float *val32, V *rval,
+                                                    float *rval32) {
+	grid_for_each<1>(padded, [&](size_t r) {
+		const uint32_t bits = r < nrows ? mask[r] : 0u;
+		uint64_t k = r < nrows ? off[r] : 0;
+		for (unsigned q = 0; q < kDiaFullWidth; ++q) {
+			const bool in = (bits >> q) & 1u;
+			if (rval) rval[run_pos(r, q)] = in ? val[k] : V(0);
+			if (rval32) rval32[run_pos(r, q)] = in ? val32[k] : 0.0f;
+			k += in ? 1 : 0;
+		}
+	});
 }
 
 static bool keep_sell() {
@@ -635,22 +667,52 @@ static bool keep_sell() {
 	return keep && keep[0] == '1';
 }
 
-// Tries the constant form on S's rows; frees the mask array when it does not hold.
+static void const_free(Storage &S) {
+	if (S.cmask) hipFree(S.cmask);
+	if (S.rval) hipFree(S.rval);
+	if (S.rval32) hipFree(S.rval32);
+	S.cmask = nullptr;
+	S.rval = nullptr;
+	S.rval32 = nullptr;
+	S.cst = ConstDia();
+}
+
+// Tries one template for all of S's rows, with the values or (in runs) without; then
+// fills the values that a template without them needs. Without memory, or when the
+// rows do not fit, S keeps its other forms.
 static alp_rc_t storage_const(Storage &S, int value_type) {
 	S.cst = ConstDia();
 	if (S.max_len == 0 || S.max_len > kDiaSlots || value_type == ALP_VAL_PATTERN || !const_dia_enabled()) return ALP_SUCCESS;
 	const size_t ns = (S.nmajor + kSellRows - 1) / kSellRows;
 	if (!S.cmask && hipMalloc(&S.cmask, sizeof(uint32_t) * ns * kSellRows) != hipSuccess) {
 		(void)hipGetLastError();
-		S.cmask = nullptr;  // no memory for the masks: the other forms
+		S.cmask = nullptr;
 		return ALP_SUCCESS;
 	}
-	const alp_rc_t rc = const_detect(S.cst, 0, S.nmajor, 0, ns, nullptr, S.off, S.idx, value_type, S.val, S.cmask);
+	const alp_rc_t rc = const_detect(S.cst, 0, S.nmajor, 0, ns, nullptr, S.off, S.idx, value_type, S.val, S.cmask, true);
 	if (rc != ALP_SUCCESS || !S.cst.w) {
-		hipFree(S.cmask);
-		S.cmask = nullptr;
+		const_free(S);
+		return rc;
 	}
-	return rc;
+	if (S.cst.uniform) return ALP_SUCCESS;
+	const size_t padded = (S.nmajor + kRunRows - 1) / kRunRows * kRunRows;
+	const size_t vs = value_type == ALP_VAL_F64 ? 8 : 4;
+	if ((!S.rval && hipMalloc(&S.rval, vs * kDiaFullWidth * padded) != hipSuccess) ||
+	    (S.val32 && !S.rval32 && hipMalloc(&S.rval32, sizeof(float) * kDiaFullWidth * padded) != hipSuccess)) {
+		(void)hipGetLastError();
+		const_free(S);
+		return ALP_SUCCESS;
+	}
+	if (value_type == ALP_VAL_F64)
+		hipLaunchKernelGGL(k_run_fill<double>, dim3(stream_grid(padded)), dim3(kBlock), 0, stream(), S.nmajor, padded,
+		                   (const uint64_t *)S.off, (const uint32_t *)S.cmask, (const double *)S.val,
+		                   (const float *)S.val32, (double *)S.rval, S.rval32);
+	else
+		hipLaunchKernelGGL(k_run_fill<float>, dim3(stream_grid(padded)), dim3(kBlock), 0, stream(), S.nmajor, padded,
+		                   (const uint64_t *)S.off, (const uint32_t *)S.cmask, (const float *)S.val,
+		                   (const float *)S.val32, (float *)S.rval, S.rval32);
+	ALP_LAUNCH_CHECK();
+	return ALP_SUCCESS;
 }
 
 // S's sliced-ELL arrays (those it has) from the CRS
@@ -710,7 +772,7 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 		dia_free(dia);
 		return rc;
 	}
-	// A matrix in constant form reads no values and, when every slice also has the
+	// A matrix with one template for its rows reads no other values and, when every slice also has the
 	// diagonal form (which the pattern rings then use), no column indices; a
 	// diagonal-only one no sliced-ELL arrays either: only the slice offsets are kept
 	const bool keep = keep_sell(), all_dia = dia.flag && dia.n_dia == ns;
@@ -730,9 +792,7 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 			if (sval32) hipFree(sval32);
 			hipFree(soff);
 			dia_free(dia);
-			if (S.cmask) hipFree(S.cmask);
-			S.cmask = nullptr;
-			S.cst = ConstDia();
+			const_free(S);
 			return ALP_SUCCESS;
 		}
 		S.sell_idx = sidx;
@@ -779,7 +839,7 @@ alp_rc_t storage_ensure_f32(Storage &S, size_t nnz) {
 		hipLaunchKernelGGL((k_convert<double, float>), dim3(stream_grid(nnz)), dim3(kBlock), 0, stream(), nnz,
 		                   (const double *)S.val, S.val32);
 	ALP_LAUNCH_CHECK();
-	if (S.cst.w) return ALP_SUCCESS;  // the template holds both precisions
+	if (S.cst.uniform) return ALP_SUCCESS;  // the template holds both precisions
 	return storage_refresh_values(S, ALP_VAL_F64);
 }
 
@@ -829,7 +889,7 @@ void storage_free(Storage &S) {
 	if (S.sell_val) hipFree(S.sell_val);
 	if (S.sell_val32) hipFree(S.sell_val32);
 	dia_free(S.dia);
-	if (S.cmask) hipFree(S.cmask);
+	const_free(S);
 	void *lr[] = {S.lr_rows, S.lr_c0, S.ch_row, S.ch_beg, S.ch_part};
 	for (void *q : lr)
 		if (q) hipFree(q);
@@ -1247,6 +1307,9 @@ size_t storage_bytes(const Storage &S, int value_type, size_t nnz) {
 	if (S.sell_val32) b += sizeof(float) * S.sell_entries;
 	if (S.dia.flag) b += S.n_slices + sizeof(int32_t) * kDiaSlots * S.n_slices + sizeof(uint32_t) * S.n_slices * kSellRows;
 	if (S.cmask) b += sizeof(uint32_t) * S.n_slices * kSellRows;
+	const size_t padded = (S.nmajor + kRunRows - 1) / kRunRows * kRunRows;
+	if (S.rval) b += vs * kDiaFullWidth * padded;
+	if (S.rval32) b += sizeof(float) * kDiaFullWidth * padded;
 	if (S.dia.val) b += vs * S.sell_entries;
 	if (S.dia.val32) b += sizeof(float) * S.sell_entries;
 	b += S.n_long * 4 + (S.n_long + 1) * 8 + S.n_chunks * (4 + 8 + 8);

@@ -593,16 +593,20 @@ __global__ __launch_bounds__(kBlock) void k_spmv_const(size_t nrows, size_t ncol
 // The product with several rows per lane (const_run_fold): RPL * 64 rows per wavefront.
 // 192^3, y += A x in FP64: 93 -> 47 us (4.2 TB/s of its mask, x and y), FP32 y = A x
 // 33 -> 29 us, where the four operations per entry and row bind; staging x in LDS
-// windows instead took 83 and 62 us.
-template <typename R, int MASK, bool OVERWRITE, int DIR>
+// windows instead took 83 and 62 us. VALUES: the rows' values are streamed 16 bytes per
+// lane from run_pos; against the diagonal slices' loads of one row per lane
+// (k_spmv_sell), FP64 accumulate at 64^3, 101x75x61, 128^3: 11.4, 22.4, 92.6 -> 9.3, 17.9,
+// 84 us; FP32 overwrite 7.5, 11.1, 45.9 -> 7.4, 10.3, 40.7 us (5.4 TB/s at 128^3).
+template <typename R, int MASK, bool OVERWRITE, int DIR, bool VALUES>
 __global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols, ConstArg<typename R::V> T,
+                                                     const typename R::V *__restrict__ rval,
                                                      const uint32_t *__restrict__ cmask,
                                                      const typename R::X *__restrict__ x,
                                                      typename R::Y *__restrict__ y,
                                                      const uint8_t *__restrict__ mask, const int *__restrict__ skip) {
 	using A = typename R::A;
 	using Y = typename R::Y;
-	constexpr unsigned N = RowsPerLane<typename R::X>::N;
+	constexpr unsigned N = RowsPerLane<R>::N;
 	const unsigned bl = xcd_logical_block(blockIdx.x, gridDim.x);
 	const size_t r0 =
 	    (size_t)__builtin_amdgcn_readfirstlane(bl * (kBlock / kWave) + threadIdx.x / kWave) * (kSellRows * N);
@@ -626,7 +630,7 @@ __global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols
 	}
 	if (stop) return;  // a solver loop that has stopped
 	A acc[N];
-	const_run_fold<R, DIR>(T, (long long)r0, lane, bits, (long long)ncols, x, acc);
+	const_run_fold<R, DIR, VALUES>(T, rval, (long long)r0, lane, bits, (long long)ncols, x, acc);
 #pragma unroll
 	for (unsigned i = 0; i < N; ++i) {
 		if (OVERWRITE) yv[i] = bits[i] == 0 ? static_cast<Y>(R::zero()) : static_cast<Y>(acc[i]);
@@ -645,8 +649,9 @@ __global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols
 }
 
 // and with the partials of y.x (overwrite): wavefronts take several groups of rows
-template <typename R, int DIR>
+template <typename R, int DIR, bool VALUES>
 __global__ __launch_bounds__(kBlock) void k_const_run_dot(size_t nrows, ConstArg<typename R::V> T,
+                                                         const typename R::V *__restrict__ rval,
                                                          const uint32_t *__restrict__ cmask,
                                                          const typename R::X *__restrict__ x,
                                                          typename R::Y *__restrict__ y, double *__restrict__ partials,
@@ -655,7 +660,7 @@ __global__ __launch_bounds__(kBlock) void k_const_run_dot(size_t nrows, ConstArg
 	using A = typename R::A;
 	using X = typename R::X;
 	using Y = typename R::Y;
-	constexpr unsigned N = RowsPerLane<X>::N;
+	constexpr unsigned N = RowsPerLane<R>::N;
 	constexpr size_t kRows = (size_t)kBlock * N;
 	const int stop = skip ? *skip : 0;
 	const unsigned lane = threadIdx.x % kWave;
@@ -681,7 +686,7 @@ __global__ __launch_bounds__(kBlock) void k_const_run_dot(size_t nrows, ConstArg
 		}
 		if (stop) return;  // uniform over the grid: no wavefront reaches the reduction
 		A acc[N];
-		const_run_fold<R, DIR>(T, (long long)r0, lane, bits, (long long)nrows, x, acc);
+		const_run_fold<R, DIR, VALUES>(T, rval, (long long)r0, lane, bits, (long long)nrows, x, acc);
 		Y yv[N];
 #pragma unroll
 		for (unsigned i = 0; i < N; ++i) {
@@ -1201,11 +1206,12 @@ static bool dia_values(const Storage &S, const void *val, const void **dval) {
 	return false;
 }
 
-// the constant form's template with the values that `val` names (false: not in that
-// form, or values it does not hold)
-template <typename R>
+// the template for the values that `val` names, which it holds itself (UNIFORM) or
+// which are kept beside it (false: not in that form, or not these values)
+template <typename R, bool UNIFORM>
 static bool const_arg(const Storage &S, const void *val, ConstArg<typename R::V> &a) {
-	if (!S.cst.w || !val || (val != S.val && val != S.val32)) return false;
+	if (!S.cst.w || S.cst.uniform != UNIFORM || !val || (val != S.val && val != S.val32)) return false;
+	if (!UNIFORM && (val == S.val ? S.rval == nullptr : S.rval32 == nullptr)) return false;
 	a.w = S.cst.w;
 	a.dmin = S.cst.dmin;
 	a.dmax = S.cst.dmax;
@@ -1216,6 +1222,19 @@ static bool const_arg(const Storage &S, const void *val, ConstArg<typename R::V>
 	return true;
 }
 
+template <typename R, int MASK, bool OW, bool VALUES>
+static void launch_runs(const Storage &S, const ConstArg<typename R::V> &T, const void *rval, const void *x, void *y,
+                        const uint8_t *mask, hipStream_t s, const int *skip) {
+	const size_t rows = (size_t)kBlock * RowsPerLane<R>::N;
+#define ALP_CRUN(DD)                                                                                            \
+	hipLaunchKernelGGL((k_const_run<R, MASK, OW, DD, VALUES>), dim3((S.nmajor + rows - 1) / rows), dim3(kBlock), 0, \
+	                   s, S.nmajor, S.nminor, T, (const typename R::V *)rval, (const uint32_t *)S.cmask,            \
+	                   (const typename R::X *)x, (typename R::Y *)y, mask, skip)
+	if (S.cst.run > 0) ALP_CRUN(1);
+	else ALP_CRUN(-1);
+#undef ALP_CRUN
+}
+
 template <typename R, int MASK, bool OW>
 static void launch_const(int xcd, const Storage &S, const ConstArg<typename R::V> &T, const void *x, void *y,
                          const uint8_t *mask, hipStream_t s, const int *skip) {
@@ -1223,14 +1242,7 @@ static void launch_const(int xcd, const Storage &S, const ConstArg<typename R::V
 	const size_t grid = (S.n_slices + per - 1) / per;
 	if (grid == 0) return;
 	if (S.cst.run) {  // no slower than a row per lane at any size measured (16^3 to 192^3)
-		const size_t rows = (size_t)kBlock * RowsPerLane<typename R::X>::N;
-#define ALP_CRUN(DD)                                                                                       \
-	hipLaunchKernelGGL((k_const_run<R, MASK, OW, DD>), dim3((S.nmajor + rows - 1) / rows), dim3(kBlock), 0, s, \
-	                   S.nmajor, S.nminor, T, (const uint32_t *)S.cmask, (const typename R::X *)x,             \
-	                   (typename R::Y *)y, mask, skip)
-		if (S.cst.run > 0) ALP_CRUN(1);
-		else ALP_CRUN(-1);
-#undef ALP_CRUN
+		launch_runs<R, MASK, OW, false>(S, T, nullptr, x, y, mask, s, skip);
 		return;
 	}
 #define ALP_CONST(WW, XX)                                                                                      \
@@ -1278,12 +1290,16 @@ int default_lanes(const Storage &S) {
 }
 
 // the template's value type (patterns have none and never take the form)
-template <typename R, bool P = R::kPattern>
+template <typename R, bool P = R::kPattern, bool UNIFORM = true>
 struct ConstVal {
 	using T = typename ConstRing<R>::T::V;
 };
 template <typename R>
-struct ConstVal<R, true> {
+struct ConstVal<R, false, false> {
+	using T = typename R::V;
+};
+template <typename R, bool UNIFORM>
+struct ConstVal<R, true, UNIFORM> {
 	using T = double;
 };
 
@@ -1298,10 +1314,14 @@ static void dispatch(const Storage &S, const void *val, unsigned descr, void *y,
 	if (kernel == 0) kernel = auto_kernel(S);
 	// the constant form where the matrix has it (kernel 5, or 4 when no sliced-ELL
 	// values are kept: the same fold order); it reads neither indices nor values
-	bool cst = false;
+	bool cst = false, runs = false;
 	ConstArg<typename ConstVal<R>::T> carg;
+	ConstArg<typename ConstVal<R, R::kPattern, false>::T> rarg;
 	if constexpr (!R::kPattern) {
-		if (kernel == 5 || (kernel == 4 && !S.sell_val)) cst = const_arg<typename ConstRing<R>::T>(S, val, carg);
+		if (kernel == 5 || (kernel == 4 && !S.sell_val)) {
+			cst = const_arg<typename ConstRing<R>::T, true>(S, val, carg);
+			runs = !cst && const_arg<R, false>(S, val, rarg);
+		}
 	}
 	const void *sval = nullptr, *dval = nullptr;
 	bool dia = false;
@@ -1325,6 +1345,10 @@ static void dispatch(const Storage &S, const void *val, unsigned descr, void *y,
 	if constexpr (!R::kPattern)                                         \
 		if (cst) {                                                      \
 			launch_const<typename ConstRing<R>::T, MM, OWV>(S.kernel ? S.lanes : 1, S, carg, x, y, mask, s, skip); \
+			return;                                                     \
+		} else if (runs) {                                              \
+			launch_runs<R, MM, OWV, true>(S, rarg, val == S.val ? S.rval : (const void *)S.rval32, x, y, mask, s, \
+			                              skip);                        \
 			return;                                                     \
 		}                                                               \
 	if (kernel == 4)                                                    \
@@ -1354,17 +1378,17 @@ static bool sell_dot_launch(const Storage &S, const void *val, const void *x, vo
 	if (k != 4 && k != 5) return false;
 	using RC = typename ConstRing<R>::T;
 	ConstArg<typename RC::V> carg;
-	if ((k == 5 || !S.sell_val) && const_arg<RC>(S, val, carg)) {
+	if ((k == 5 || !S.sell_val) && const_arg<RC, true>(S, val, carg)) {
 		const size_t nb = (S.n_slices + kBlock / kSellRows - 1) / (kBlock / kSellRows);
 		const unsigned grid = (unsigned)std::min<size_t>(nb, std::min<size_t>(max_partials, fill_blocks(8)));
 		if (grid == 0) return false;
 		if (S.cst.run) {  // no slower than a row per lane at any size measured (16^3 to 192^3)
-			const size_t rows = (size_t)kBlock * RowsPerLane<typename RC::X>::N;
+			const size_t rows = (size_t)kBlock * RowsPerLane<RC>::N;
 			const unsigned gr = (unsigned)std::min<size_t>((S.nmajor + rows - 1) / rows,
 			                                               std::min<size_t>(max_partials, fill_blocks(8)));
 #define ALP_CRDOT(DD)                                                                                       \
-	hipLaunchKernelGGL((k_const_run_dot<RC, DD>), dim3(gr), dim3(kBlock), 0, s, S.nmajor, carg,                \
-	                   (const uint32_t *)S.cmask, (const typename R::X *)x, (typename R::Y *)y, partials, skip)
+	hipLaunchKernelGGL((k_const_run_dot<RC, DD, false>), dim3(gr), dim3(kBlock), 0, s, S.nmajor, carg,         \
+	                   (const typename RC::V *)nullptr, (const uint32_t *)S.cmask, (const typename R::X *)x, (typename R::Y *)y, partials, skip)
 			if (S.cst.run > 0) ALP_CRDOT(1);
 			else ALP_CRDOT(-1);
 #undef ALP_CRDOT
@@ -1379,6 +1403,22 @@ static bool sell_dot_launch(const Storage &S, const void *val, const void *x, vo
 		else ALP_CDOT(0);
 #undef ALP_CDOT
 		*nparts = grid;
+		return true;
+	}
+	ConstArg<typename R::V> rarg;
+	if ((k == 5 || !S.sell_val) && const_arg<R, false>(S, val, rarg)) {
+		const size_t rows = (size_t)kBlock * RowsPerLane<R>::N, nb = (S.nmajor + rows - 1) / rows;
+		if (nb > max_partials) return false;  // as below: larger matrices keep the separate dot
+		const unsigned gr = (unsigned)std::min<size_t>(nb, std::min<size_t>(max_partials, fill_blocks(8)));
+		const void *rv = val == S.val ? S.rval : (const void *)S.rval32;
+#define ALP_RDOT(DD)                                                                                        \
+	hipLaunchKernelGGL((k_const_run_dot<R, DD, true>), dim3(gr), dim3(kBlock), 0, s, S.nmajor, rarg,           \
+	                   (const typename R::V *)rv, (const uint32_t *)S.cmask, (const typename R::X *)x,          \
+	                   (typename R::Y *)y, partials, skip)
+		if (S.cst.run > 0) ALP_RDOT(1);
+		else ALP_RDOT(-1);
+#undef ALP_RDOT
+		*nparts = gr;
 		return true;
 	}
 	const void *sval = nullptr, *dval = nullptr;

@@ -275,12 +275,12 @@ __device__ __forceinline__ typename R::A const_fold(const ConstArg<typename R::V
 // Several rows per lane for templates that are nine runs of three consecutive
 // offsets (ConstDia::run; the 27-point stencil's order): a lane owns RPL = 16 /
 // sizeof(x) consecutive rows, whose slots of one run lie in RPL + 2 consecutive
-// elements of x, read by one 16-byte load and one of the rest. A wavefront's reads
+// elements of x, read by one 16-byte load and one of the rest; so are its values. A wavefront's reads
 // then move 1.5 to 2 elements per row and run through L1 instead of 3, in a third
 // (FP64) or a sixth (FP32) of the load instructions. Each row's fold keeps its order.
-template <typename X>
+template <typename R>
 struct RowsPerLane {
-	static constexpr unsigned N = 16 / sizeof(X);
+	static constexpr unsigned N = 16 / sizeof(typename R::X);
 };
 
 // n consecutive elements, whatever their alignment (global loads need only 4 bytes)
@@ -288,6 +288,15 @@ template <unsigned N, typename X>
 __device__ __forceinline__ void load_run(const X *p, X *out) {
 	typedef X V __attribute__((ext_vector_type(N), aligned(sizeof(X))));
 	const V v = *reinterpret_cast<const V *>(p);
+#pragma unroll
+	for (unsigned i = 0; i < N; ++i) out[i] = v[i];
+}
+
+// the same for a stream read once (p a multiple of N elements)
+template <unsigned N, typename X>
+__device__ __forceinline__ void load_run_nt(const X *p, X *out) {
+	typedef X V __attribute__((ext_vector_type(N)));
+	const V v = __builtin_nontemporal_load(reinterpret_cast<const V *>(p));
 #pragma unroll
 	for (unsigned i = 0; i < N; ++i) out[i] = v[i];
 }
@@ -302,15 +311,17 @@ __device__ __forceinline__ void store_run(X *p, const X *in) {
 }
 
 // rows r0 + lane * RPL + i, i < RPL (r0 uniform), with masks bits[i]; DIR = the sign of
-// the runs
-template <typename R, int DIR>
-__device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T, long long r0, unsigned lane,
-                                               const uint32_t (&bits)[RowsPerLane<typename R::X>::N], long long ncols,
+// the runs. With VALUES the rows' values come from rval (run_pos), streamed once, not
+// from the template.
+template <typename R, int DIR, bool VALUES>
+__device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T,
+                                               const typename R::V *__restrict__ rval, long long r0, unsigned lane,
+                                               const uint32_t (&bits)[RowsPerLane<R>::N], long long ncols,
                                                const typename R::X *__restrict__ x,
-                                               typename R::A (&acc)[RowsPerLane<typename R::X>::N]) {
+                                               typename R::A (&acc)[RowsPerLane<R>::N]) {
 	using A = typename R::A;
 	using X = typename R::X;
-	constexpr unsigned N = RowsPerLane<X>::N, kGroup = 3;  // runs in flight
+	constexpr unsigned N = RowsPerLane<R>::N, kGroup = 3;  // runs in flight
 	constexpr uint32_t full = (1u << kDiaFullWidth) - 1u;
 	const bool inside = r0 + T.dmin >= 0 && r0 + (long long)(kSellRows * N) - 1 + T.dmax < ncols;
 	bool some = false;
@@ -326,6 +337,12 @@ __device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T,
 	// nine take 120-190 registers and the occupancy with them
 #pragma unroll 1
 	for (unsigned q0 = 0; q0 < kDiaFullWidth; q0 += 3 * kGroup) {
+		typename R::V v[VALUES ? 3 * kGroup : 1][N];
+		if (VALUES) {
+			const typename R::V *vp = rval + run_pos((size_t)r0, q0) + lane * N;
+#pragma unroll
+			for (unsigned j = 0; j < 3 * kGroup; ++j) load_run_nt<N>(vp + j * kRunRows, v[VALUES ? j : 0]);
+		}
 		X e[kGroup][N + 2];
 		if (inside) {
 #pragma unroll
@@ -350,7 +367,9 @@ __device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T,
 				for (unsigned j = 0; j < 3; ++j)
 #pragma unroll
 					for (unsigned i = 0; i < N; ++i)
-						acc[i] = R::add(R::mul(T.v[q0 + 3 * k + j], e[k][i + (DIR > 0 ? j : 2 - j)]), acc[i]);
+						acc[i] = R::add(R::mul(VALUES ? v[VALUES ? 3 * k + j : 0][i] : T.v[q0 + 3 * k + j],
+						                       e[k][i + (DIR > 0 ? j : 2 - j)]),
+						                acc[i]);
 		} else {
 #pragma unroll
 			for (unsigned k = 0; k < kGroup; ++k)
@@ -358,8 +377,8 @@ __device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T,
 				for (unsigned j = 0; j < 3; ++j)
 #pragma unroll
 					for (unsigned i = 0; i < N; ++i)
-						acc[i] = const_term<R>(T.v[q0 + 3 * k + j], m[i], 3 * k + j, e[k][i + (DIR > 0 ? j : 2 - j)],
-						                       acc[i]);
+						acc[i] = const_term<R>(VALUES ? v[VALUES ? 3 * k + j : 0][i] : T.v[q0 + 3 * k + j], m[i],
+						                       3 * k + j, e[k][i + (DIR > 0 ? j : 2 - j)], acc[i]);
 #pragma unroll
 			for (unsigned i = 0; i < N; ++i) m[i] >>= 3 * kGroup;
 		}

@@ -94,6 +94,46 @@ def test_const_stencil_takes_the_form(A, sides, monkeypatch):
         assert np.array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("flip", [False, True])
+@pytest.mark.parametrize("sides", [(4, 4, 4), (16, 5, 4), (65, 3, 5), (33, 17, 9), (64, 12, 10), (130, 20, 3)])
+def test_run_values_equal_kept_values(A, sides, flip, monkeypatch):
+    """27-point patterns with a value per entry take the template's offsets and keep their
+    values slot by slot: the same bits as the sliced ELL's fold in every ring and mask
+    mode, rows in descending and ascending order, with NaN and infinities in the matrix
+    and in x (also where a row lacks the neighbour), and after a change of precision."""
+    rng = np.random.default_rng(sum(sides))
+    off, idx, _ = A.Matrix.stencil27(*sides).download(0)
+    n = off.size - 1
+    val = rng.standard_normal(idx.size)
+    x, y0 = rng.standard_normal(n), rng.standard_normal(n)
+    if flip:  # rows in ascending order
+        order = np.concatenate([np.arange(int(off[r + 1]) - 1, int(off[r]) - 1, -1) for r in range(n)])
+        idx, val = idx[order], val[order]
+    else:
+        val[rng.integers(0, val.size, 3)] = [np.nan, np.inf, -np.inf]
+        x[rng.integers(0, n, 3)] = [np.nan, np.inf, -np.inf]
+    mask = (rng.random(n) < 0.5).astype(np.uint8)
+    F, P = both(A, monkeypatch, lambda: A.Matrix.from_crs(n, n, off, idx, val, flags=A.MAT_WITH_F32))
+    F32, P32 = both(A, monkeypatch, lambda: A.Matrix.from_crs(n, n, off, idx, val.astype(np.float32)))
+    x32, y32 = x.astype(np.float32), y0.astype(np.float32)
+    for c, p, ring, xv, yv in ((F, P, A.PLUS_TIMES_F64, x, y0), (F, P, A.MIN_PLUS_F64, x, y0),
+                               (F, P, A.PLUS_TIMES_F32, x32, y32), (F32, P32, A.PLUS_TIMES_F32, x32, y32),
+                               (F, P, A.PLUS_PATTERN_F64, x, y0)):
+        for k in (c, p):
+            if k.layout()[0]:
+                k.set_kernel(4)
+        for a, b in zip(products(A, c, xv, yv, ring, mask), products(A, p, xv, yv, ring, mask)):
+            assert np.array_equal(a, b, equal_nan=True), ring
+    # the FP32 copy made by a mixed solve instead of at build time
+    if not flip:
+        return
+    D = A.Matrix.from_crs(n, n, off, idx, val)
+    b, s = A.Vector.from_numpy(y0), A.Vector(n, fill=0.0)
+    A.cg(D, b, s, 1, 1e-10, 1)
+    for a, b in zip(products(A, D, x32, y32, A.PLUS_TIMES_F32, mask), products(A, F, x32, y32, A.PLUS_TIMES_F32, mask)):
+        assert np.array_equal(a, b)
+
+
 def test_const_near_misses_keep_their_values(A, monkeypatch):
     """One value off by an ulp, one row in another order, one column stored twice: not
     one template, so the bytes held and the results are those without the form."""
