@@ -540,7 +540,7 @@ static unsigned vec_grid(size_t n) {
 }
 
 int default_lanes(const Storage &S);
-int auto_kernel(const Storage &S);
+int auto_kernel_dot(const Storage &S);
 
 // Work vectors and the captured iteration batch of one solver configuration,
 // kept on the matrix between calls: a repeated solve with the same storage,
@@ -664,7 +664,7 @@ struct CgRunner {
 		RR = S.rows ? S.rows : 1;
 		// the fused SpMV + dot kernel is the CSR-vector gather; the other
 		// kernels run as a generic SpMV followed by the dot
-		const int k = S.kernel ? S.kernel : auto_kernel(S);
+		const int k = S.kernel ? S.kernel : auto_kernel_dot(S);
 		fused = k == 1 && G >= 2 && !acc64;
 		const size_t rows_per = (size_t)(kBlock / G) * RR;
 		const size_t nchunks = (a.n + rows_per - 1) / rows_per;

@@ -69,6 +69,45 @@ __global__ __launch_bounds__(kBlock) void k_spmv_vector(
 	}
 }
 
+// Rows of a tile longer than kRowSteps entries for each of their tpr threads go to a
+// whole wavefront instead, after the others: the thread groups push them to a list in
+// LDS, and each wavefront takes its rows in turn, lanes striding the row's entries, a
+// tree at the end. One thread per row folds up to a tile's 2048 entries in a serial
+// chain that the block waits for: 60001 rows of 6 +- 10 entries (lognormal, sigma
+// 1.1) took 21 us where evenly long rows take 5.
+constexpr unsigned kRowSteps = 32;
+struct TileLong {
+	unsigned n;
+	uint16_t row[4096 / kRowSteps];
+};
+
+// the rows of the list: product(k) is entry k's product, row r's entries [off[r], off[r + 1])
+template <typename R, int MASK, bool OVERWRITE, typename Product>
+__device__ __forceinline__ void fold_long_rows(const TileLong &ll, uint32_t r0, const uint64_t *__restrict__ off,
+                                               typename R::Y *__restrict__ y, Product &&product) {
+	using A = typename R::A;
+	using Y = typename R::Y;
+	const unsigned lane = threadIdx.x % kWave;
+	for (unsigned i = threadIdx.x / kWave; i < ll.n; i += kBlock / kWave) {
+		const uint32_t r = r0 + ll.row[i];
+		const uint64_t rk = off[r], re = off[r + 1];
+		A yv = R::zero();
+		if (!OVERWRITE && lane == 0) yv = static_cast<A>(y[r]);
+		A acc = R::zero();
+		uint64_t q = rk + lane;
+		for (; q + 3 * kWave < re; q += 4 * kWave) {
+			A p[4];
+#pragma unroll
+			for (int u = 0; u < 4; ++u) p[u] = product(q + u * kWave);
+#pragma unroll
+			for (int u = 0; u < 4; ++u) acc = R::add(acc, p[u]);
+		}
+		for (; q < re; q += kWave) acc = R::add(acc, product(q));
+		acc = group_fold<kWave, R>(acc);
+		if (lane == 0) y[r] = OVERWRITE ? static_cast<Y>(acc) : static_cast<Y>(R::add(yv, acc));
+	}
+}
+
 template <typename R, int MASK, bool OVERWRITE, int J, bool XCD>
 __global__ __launch_bounds__(kBlock) void k_spmv_stream(
     size_t nrb, const uint32_t *__restrict__ rb, const uint64_t *__restrict__ rbase,
@@ -83,6 +122,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream(
 	constexpr int kTile = J * kBlock;
 	__shared__ A tile[kTile];
 	__shared__ A red[kBlock / kWave];
+	__shared__ TileLong ll;
 	const auto *val = static_cast<const typename R::V *>(vval);
 	const WorkSplit w = XCD ? xcd_split(nrb) : WorkSplit{blockIdx.x, nrb, gridDim.x};
 	// tile metadata (row bounds and nonzero bounds) is one independent load
@@ -139,18 +179,26 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream(
 				const uint64_t k = base + threadIdx.x + (uint64_t)q * kBlock;
 				if (k < top) tile[k - base] = Val<R>::mul(vv[q], x[jj[q]]);
 			}
+			if (threadIdx.x == 0) ll.n = 0;
 			__syncthreads();
+			const bool lng = re - rk > (uint64_t)kRowSteps * tpr;
 			A acc = R::zero();
-			for (uint64_t q = rk + sub; q < re; q += tpr) acc = R::add(acc, tile[q - base]);
+			if (!lng)
+				for (uint64_t q = rk + sub; q < re; q += tpr) acc = R::add(acc, tile[q - base]);
 			for (unsigned s = tpr / 2; s > 0; s >>= 1) acc = R::add(acc, shfl_xor(acc, s));
-			if (active && sub == 0 && !(skip_long && re - rk > kLongRow)) {
+			const bool mine = active && sub == 0 && !(skip_long && re - rk > kLongRow);
+			if (lng && mine) ll.row[atomicAdd(&ll.n, 1u)] = (uint16_t)(r - r0);
+			if (mine && !lng) {
 				if (rk == re) {
 					if (OVERWRITE) y[r] = static_cast<Y>(R::zero());
 				} else {
 					y[r] = OVERWRITE ? static_cast<Y>(acc) : static_cast<Y>(R::add(yv, acc));
 				}
 			}
-			__syncthreads();
+			if (__syncthreads_or(lng ? 1 : 0)) {
+				fold_long_rows<R, MASK, OVERWRITE>(ll, r0, off, y, [&](uint64_t k) { return tile[k - base]; });
+				__syncthreads();
+			}
 		} else if (!skip_long) {
 			// a single row longer than a tile: the whole block folds it
 			A acc = R::zero();
@@ -199,6 +247,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_seg(
 	__shared__ uint32_t sidx[kTile];
 	__shared__ VT sval[R::kPattern ? 1 : kTile];
 	__shared__ A red[kBlock / kWave];
+	__shared__ TileLong ll;
 	const auto *val = static_cast<const typename R::V *>(vval);
 	for (size_t b = blockIdx.x; b < nrb; b += gridDim.x) {
 		const uint32_t r0 = rb[b], r1 = rb[b + 1];
@@ -238,9 +287,11 @@ __global__ __launch_bounds__(kBlock) void k_spmv_seg(
 					if (!R::kPattern) sval[k - base] = vv[q];
 				}
 			}
+			if (threadIdx.x == 0) ll.n = 0;
 			__syncthreads();
+			const bool lng = re - rk > (uint64_t)kRowSteps * tpr;
 			A acc = R::zero();
-			uint64_t q = rk + sub;
+			uint64_t q = lng ? re : rk + sub;
 			for (; q + (uint64_t)(U - 1) * tpr < re; q += (uint64_t)U * tpr) {
 				X xv[U];
 				VT av[U];
@@ -258,14 +309,19 @@ __global__ __launch_bounds__(kBlock) void k_spmv_seg(
 				acc = R::add(acc, Val<R>::mul(R::kPattern ? VT(0) : sval[R::kPattern ? 0 : t], x[sidx[t]]));
 			}
 			for (unsigned sh = tpr / 2; sh > 0; sh >>= 1) acc = R::add(acc, shfl_xor(acc, sh));
-			if (active && sub == 0 && !(skip_long && re - rk > kLongRow)) {
+			const bool mine = active && sub == 0 && !(skip_long && re - rk > kLongRow);
+			if (lng && mine) ll.row[atomicAdd(&ll.n, 1u)] = (uint16_t)(r - r0);
+			if (mine && !lng) {
 				if (rk == re) {
 					if (OVERWRITE) y[r] = static_cast<Y>(R::zero());
 				} else {
 					y[r] = OVERWRITE ? static_cast<Y>(acc) : static_cast<Y>(R::add(yv, acc));
 				}
 			}
-			__syncthreads();
+			if (__syncthreads_or(lng ? 1 : 0)) {
+				fold_long_rows<R, MASK, OVERWRITE>(ll, r0, off, y, [&](uint64_t k) { return Val<R>::mul(R::kPattern ? VT(0) : sval[R::kPattern ? 0 : (unsigned)(k - base)], x[sidx[(unsigned)(k - base)]]); });
+				__syncthreads();
+			}
 		} else if (!skip_long) {
 			// a single row longer than a tile: the whole block folds it
 			A acc = R::zero();
@@ -782,6 +838,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream_pipe(
 	constexpr int kTile = J * kBlock;
 	__shared__ A tile[kTile];
 	__shared__ A red[kBlock / kWave];
+	__shared__ TileLong ll;
 	const auto *val = static_cast<const typename R::V *>(vval);
 	const size_t step = gridDim.x;
 	size_t b = blockIdx.x;
@@ -832,18 +889,26 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream_pipe(
 				const uint64_t k = cb + threadIdx.x + (uint64_t)q * kBlock;
 				if (k < ct) tile[k - cb] = Val<R>::mul(cur.v[q], xg[q]);
 			}
+			if (threadIdx.x == 0) ll.n = 0;
 			__syncthreads();
+			const bool lng = re - rk > (uint64_t)kRowSteps * tpr;
 			A acc = R::zero();
-			for (uint64_t q = rk + sub; q < re; q += tpr) acc = R::add(acc, tile[q - cb]);
+			if (!lng)
+				for (uint64_t q = rk + sub; q < re; q += tpr) acc = R::add(acc, tile[q - cb]);
 			for (unsigned s = tpr / 2; s > 0; s >>= 1) acc = R::add(acc, shfl_xor(acc, s));
-			if (active && sub == 0) {
+			const bool mine = active && sub == 0;
+			if (lng && mine) ll.row[atomicAdd(&ll.n, 1u)] = (uint16_t)(r - c0);
+			if (mine && !lng) {
 				if (rk == re) {
 					if (OVERWRITE) y[r] = static_cast<Y>(R::zero());
 				} else {
 					y[r] = OVERWRITE ? static_cast<Y>(acc) : static_cast<Y>(R::add(yv, acc));
 				}
 			}
-			__syncthreads();
+			if (__syncthreads_or(lng ? 1 : 0)) {
+				fold_long_rows<R, MASK, OVERWRITE>(ll, c0, off, y, [&](uint64_t k) { return tile[k - cb]; });
+				__syncthreads();
+			}
 		} else {
 			if (n_short) tile_issue<R, J>(nxt, nb, nt, idx, val);
 			A acc = R::zero();
@@ -1272,12 +1337,30 @@ static void launch_wave(const Storage &S, const void *val, const void *x, void *
 	                   (const typename R::X *)x, (typename R::Y *)y, mask, skip);
 }
 
-// without autotuning: sliced ELL where it was built (regular rows), CSR-stream
-// (whole-block folds of long rows) for skewed row lengths, CSR-vector otherwise
+// Nonzeros from which CSR-stream with row segments in LDS is the default where no sliced
+// form was built: with 20 entries per row at random columns in FP64, CSR-vector takes
+// 5.1, 10.8, 33.8 and 193 us at 0.4, 1.2, 4 and 20 M nonzeros, row segments 5.6, 8.6, 25.2
+// and 153 us; on skewed rows (sigma 1.1) the storage-order variant takes 7.8, 10.9, 33.3
+// and 174 us, row segments 8.7, 10.5, 29.8 and 165 us.
+static bool many_nonzeros(const Storage &S) { return S.avg_len * (double)S.nmajor >= (double)(1u << 20); }
+
+static bool skewed(const Storage &S) { return S.max_len > 64 && (double)S.max_len > 8.0 * S.avg_len; }
+
+// without autotuning: sliced ELL where it was built (regular rows), CSR-stream for
+// skewed row lengths (long rows folded by wavefronts) or many nonzeros, CSR-vector
+// otherwise
 int auto_kernel(const Storage &S) {
 	if (S.dia.flag) return 5;
 	if (S.sell_off) return 4;
-	return (S.max_len > 64 && (double)S.max_len > 8.0 * S.avg_len) ? 2 : 1;
+	return skewed(S) || many_nonzeros(S) ? 2 : 1;
+}
+
+// the same for a product whose dot with its input is wanted too: CSR-vector's kernel
+// folds it in, a launch and two vector reads less, which the faster product makes up
+// for from about 4 M nonzeros
+int auto_kernel_dot(const Storage &S) {
+	const int k = auto_kernel(S);
+	return k == 2 && !skewed(S) && S.avg_len * (double)S.nmajor < (double)(4u << 20) ? 1 : k;
 }
 
 int default_lanes(const Storage &S) {
@@ -1340,7 +1423,7 @@ static void dispatch(const Storage &S, const void *val, unsigned descr, void *y,
 		}
 	}
 	if (kernel != 4) dia = false;
-	if (RR == 0) RR = kernel == 2 ? 8 : kernel == 4 ? 8 : 1;
+	if (RR == 0) RR = kernel == 2 ? (S.kernel == 0 && many_nonzeros(S) ? 64 : 8) : kernel == 4 ? 8 : 1;
 #define ALP_GO(MM, OWV)                                                 \
 	if constexpr (!R::kPattern)                                         \
 		if (cst) {                                                      \
@@ -1580,7 +1663,10 @@ ALP_EXPORT alp_rc_t alp_hip_matrix_get_kernel(alp_hip_matrix_t A, int *kernel, i
 	int l = k >= 4 ? A->crs.lanes : (A->crs.lanes ? A->crs.lanes : default_lanes(A->crs));
 	if (kernel) *kernel = k;
 	if (lanes) *lanes = l;
-	if (rows) *rows = A->crs.rows ? A->crs.rows : (k == 2 || k >= 4 ? 8 : 1);
+	if (rows)
+		*rows = A->crs.rows ? A->crs.rows
+		        : k == 2    ? (A->crs.kernel == 0 && many_nonzeros(A->crs) ? 64 : 8)
+		                    : (k >= 4 ? 8 : 1);
 	return ALP_SUCCESS;
 }
 
