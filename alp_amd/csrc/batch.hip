@@ -33,6 +33,25 @@ namespace alp {
 constexpr int kRowsPerTile = 256;
 constexpr int kMaxRhs = 16;
 
+// Directions kept per solve: iteration i works on the direction in slot i % D and
+// writes the next one to the slot after it, and X takes the D steps together
+// (see k_b_dir). FP32 data: four, the three extra ones in the FP64 direction and
+// product, which those solves do not use. FP64: two, the second one in the FP32
+// direction and product. No memory is added for either.
+constexpr int kBatchDirs = 4;
+template <typename T>
+constexpr int batch_dirs() {
+	return sizeof(T) == 4 ? kBatchDirs : 2;
+}
+template <typename T>
+struct Dirs {
+	T *p[batch_dirs<T>()];
+};
+
+// sys_active: a system whose right-hand sides have all stopped is frozen. It passes
+// one k_b_dir in kFreezing, which brings its X up to date.
+constexpr int kFrozen = 0, kRunning = 1, kFreezing = 2;
+
 struct BatchInst {
 	double rz, alpha, beta, rr, tol, bnorm, scale;
 	int active, converged;
@@ -147,7 +166,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm(size_t ntiles, const uint32_t *
 	for (size_t t = ws.first; t < ws.last; t += ws.step) {
 		// a system whose right-hand sides have all converged is frozen: skip its rows
 		// (the residual product RES always runs: the outer loop reads it for every system)
-		if (!RES && sys_active && !sys_active[tile_sys[t]]) continue;
+		if (!RES && sys_active && sys_active[tile_sys[t]] != kRunning) continue;
 		const uint32_t r0 = tile_row0[t], r1 = tile_row1[t];
 		double acc_dot[RPL];
 #pragma unroll
@@ -241,7 +260,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_dia(size_t ntiles, const uint32
 	const unsigned wave_row = (threadIdx.x / kWave) * kWaveRows;
 	const WorkSplit ws = XCD ? xcd_split(ntiles) : WorkSplit{blockIdx.x, ntiles, gridDim.x};
 	for (size_t t = ws.first; t < ws.last; t += ws.step) {
-		if (sys_active && !sys_active[tile_sys[t]]) continue;
+		if (sys_active && sys_active[tile_sys[t]] != kRunning) continue;
 		const uint32_t r0 = tile_row0[t], r1 = tile_row1[t], sl0 = tile_sl0[t];
 		double acc_dot[RPL];
 #pragma unroll
@@ -405,68 +424,113 @@ __device__ __forceinline__ void system_sums(const double *part, const uint32_t *
 	__syncthreads();
 }
 
+// The scalars of the vector kernels, in the vectors' type T: D step lengths (one
+// per direction slot), beta, and 1 for instances that go on, each ninst long.
+template <typename T>
+__device__ __forceinline__ T *coef_alpha(T *c, size_t ninst, int slot) {
+	return c + (size_t)slot * ninst;
+}
+template <typename T>
+__device__ __forceinline__ T *coef_beta(T *c, size_t ninst) {
+	return c + (size_t)batch_dirs<T>() * ninst;
+}
+template <typename T>
+__device__ __forceinline__ T *coef_go(T *c, size_t ninst) {
+	return c + (size_t)(batch_dirs<T>() + 1) * ninst;
+}
+
 // alpha = rz / pAp for active instances (one block per system)
+template <typename T>
 __global__ __launch_bounds__(kBlock) void k_b_alpha(int nrhs, const double *part, const uint32_t *tile0,
-                                                    BatchInst *in) {
+                                                    BatchInst *in, T *coef, size_t ninst, int slot,
+                                                    int *sys_active) {
 	__shared__ double sums[kMaxRhs];
 	const int s = blockIdx.x;
+	if (sys_active[s] != kRunning) {  // uniform per block; X of a freezing system is up to date by now
+		__syncthreads();
+		if (threadIdx.x == 0) sys_active[s] = kFrozen;
+		return;
+	}
 	system_sums(part, tile0, s, nrhs, sums);
 	if (threadIdx.x < nrhs) {
-		BatchInst &I = in[s * nrhs + threadIdx.x];
+		const int i = s * nrhs + threadIdx.x;
+		BatchInst &I = in[i];
 		I.alpha = I.active ? I.rz / sums[threadIdx.x] : 0.0;
+		coef_alpha(coef, ninst, slot)[i] = (T)I.alpha;
 	}
 }
 
-// X += alpha P; R -= alpha AP, with the partials of R.R
-template <typename T>
+// The vector kernels of an iteration move V consecutive entries per lane: 16
+// bytes where the right-hand sides of a row fill them (the tiles then start at
+// multiples of V), else one entry. Threads k, k + kBlock, ... of a tile keep their
+// right-hand sides, since kBlock * V % nrhs == 0. Both are bound by memory:
+// 72 M FP32 entries (64 systems, 8 right-hand sides) at 4.9 TB/s.
+
+// R -= alpha AP, with the partials of R.R
+template <typename T, int V>
 __global__ __launch_bounds__(kBlock) void k_b_update(size_t ntiles, const uint32_t *tile_row0,
                                                      const uint32_t *tile_row1, const uint32_t *tile_sys, int nrhs,
-                                                     T *X, T *R, const T *P, const T *AP, const BatchInst *in,
-                                                     double *part, const int *sys_active) {
-	__shared__ double red[kBlock];
+                                                     T *R, const T *AP, const T *alphas, double *part,
+                                                     const int *sys_active) {
+	__shared__ double red[2][kBlock / kWave][kMaxRhs];
+	const int j0 = threadIdx.x * V % nrhs;
+	const int lanes = nrhs / V;  // lanes that share a row
+	int turn = 0;
 	for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-		if (!sys_active[tile_sys[t]]) continue;  // uniform per block: the barriers below stay matched
-		const size_t base = (size_t)tile_row0[t] * nrhs;
-		const size_t cnt = (size_t)(tile_row1[t] - tile_row0[t]) * nrhs;
 		const int sys = tile_sys[t];
-		// thread k handles entries k, k + kBlock, ... of the tile; kBlock % nrhs == 0,
-		// so each thread keeps one right-hand side
-		const int r = threadIdx.x % nrhs;
-		const BatchInst &I = in[sys * nrhs + r];
-		const T alpha = (T)I.alpha;
-		double acc = 0.0;
-		for (size_t k = threadIdx.x; k < cnt; k += kBlock) {
-			const size_t e = base + k;
-			X[e] = alpha * P[e] + X[e];
-			const T rv = R[e] - alpha * AP[e];
-			R[e] = rv;
-			acc += (double)rv * (double)rv;
+		if (sys_active[sys] != kRunning) continue;  // uniform per block: the barriers below stay matched
+		const size_t base = (size_t)tile_row0[t] * nrhs;
+		const unsigned cnt = (tile_row1[t] - tile_row0[t]) * (unsigned)nrhs;
+		T alpha[V];
+		RowChunk<T, V>::load(alphas + (size_t)sys * nrhs + j0, alpha);
+		double acc[V];
+#pragma unroll
+		for (int j = 0; j < V; ++j) acc[j] = 0.0;
+		for (unsigned k = threadIdx.x * V; k < cnt; k += kBlock * V) {
+			T r[V], ap[V];
+			RowChunk<T, V>::load(R + base + k, r);
+			RowChunk<T, V>::load(AP + base + k, ap);
+#pragma unroll
+			for (int j = 0; j < V; ++j) {
+				r[j] -= alpha[j] * ap[j];
+				acc[j] += (double)r[j] * (double)r[j];
+			}
+			RowChunk<T, V>::store(R + base + k, r);
 		}
-		red[threadIdx.x] = acc;
+#pragma unroll
+		for (int j = 0; j < V; ++j)
+			for (int o = kWave / 2; o >= lanes; o >>= 1) acc[j] += __shfl_xor(acc[j], o, kWave);
+		if ((int)(threadIdx.x % kWave) < lanes)
+#pragma unroll
+			for (int j = 0; j < V; ++j) red[turn][threadIdx.x / kWave][j0 + j] = acc[j];
 		__syncthreads();
 		if (threadIdx.x < nrhs) {
 			double s = 0.0;
-			for (int k = threadIdx.x; k < kBlock; k += nrhs) s += red[k];
+			for (int w = 0; w < kBlock / kWave; ++w) s += red[turn][w][threadIdx.x];
 			part[t * nrhs + threadIdx.x] = s;
 		}
-		__syncthreads();
+		turn ^= 1;  // the next tile writes the other half: one barrier per tile
 	}
 }
 
 // beta = rr / rz; stop tests (||r|| < tol * ||b||, conjugate_gradient.hpp:437)
+template <typename T>
 __global__ __launch_bounds__(kBlock) void k_b_beta(int nrhs, const double *part, const uint32_t *tile0,
                                                    BatchInst *in, unsigned long long max_iter, unsigned *nactive,
-                                                   int *sys_active) {
+                                                   T *coef, size_t ninst, int slot, int *sys_active, int *sys_slot) {
 	__shared__ double sums[kMaxRhs];
 	__shared__ int any;
 	const int s = blockIdx.x;
+	if (sys_active[s] != kRunning) return;  // uniform per block
 	if (threadIdx.x == 0) any = 0;
 	system_sums(part, tile0, s, nrhs, sums);
 	if (threadIdx.x < nrhs) {
-		BatchInst &I = in[s * nrhs + threadIdx.x];
-		if (!I.active) {
-			I.beta = 0.0;
-		} else {
+		const int i = s * nrhs + threadIdx.x;
+		BatchInst &I = in[i];
+		// an instance that has stopped keeps its direction: beta 1, no residual
+		I.beta = 1.0;
+		T go = T(0);
+		if (I.active) {
 			const double rr = sums[threadIdx.x];
 			I.rr = rr;
 			I.iter += 1;
@@ -474,34 +538,106 @@ __global__ __launch_bounds__(kBlock) void k_b_beta(int nrhs, const double *part,
 			if (conv || I.iter >= max_iter) {
 				I.active = 0;
 				I.converged = conv ? 1 : 0;
-				I.beta = 0.0;
 			} else {
 				I.beta = rr / I.rz;
 				I.rz = rr;
+				go = T(1);
 				atomicAdd(nactive, 1u);
 				atomicOr(&any, 1);
 			}
 		}
+		coef_beta(coef, ninst)[i] = (T)I.beta;
+		coef_go(coef, ninst)[i] = go;
 	}
 	__syncthreads();
-	if (threadIdx.x == 0) sys_active[s] = any;
+	if (threadIdx.x == 0) {
+		sys_active[s] = any ? kRunning : kFreezing;
+		sys_slot[s] = slot;
+	}
 }
 
-// P = R + beta P for active instances
-template <typename T>
+// The next direction, P' = R + beta P (P' = P for an instance that has stopped). X
+// is not read by the iteration, so it takes the steps of the last D directions at
+// once, in the order of the iterations, where slot SLOT is the last one or the
+// system freezes: per entry and iteration 3 + 1 + (D + 1) / D accesses with those
+// of k_b_update in place of 9 (64 systems x 8 right-hand sides, 72 M FP32 entries:
+// both kernels 537 us before, see the rate above).
+template <typename T, int V, int SLOT>
 __global__ __launch_bounds__(kBlock) void k_b_dir(size_t ntiles, const uint32_t *tile_row0, const uint32_t *tile_row1,
-                                                  const uint32_t *tile_sys, int nrhs, T *P, const T *R,
-                                                  const BatchInst *in, const int *sys_active) {
+                                                  const uint32_t *tile_sys, int nrhs, T *X, Dirs<T> P, const T *R,
+                                                  T *coef, size_t ninst, const int *sys_active) {
+	constexpr int D = batch_dirs<T>();
+	const T *p0 = P.p[SLOT];
+	T *p1 = P.p[(SLOT + 1) % D];
+	const int j0 = threadIdx.x * V % nrhs;
 	for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-		if (!sys_active[tile_sys[t]]) continue;
+		const int sys = tile_sys[t];
+		const int state = sys_active[sys];
+		if (state == kFrozen) continue;
+		const size_t base = (size_t)tile_row0[t] * nrhs;
+		const unsigned cnt = (tile_row1[t] - tile_row0[t]) * (unsigned)nrhs;
+		const size_t inst = (size_t)sys * nrhs + j0;
+		if (SLOT == D - 1 || state == kFreezing) {
+			T alpha[SLOT + 1][V];
+#pragma unroll
+			for (int d = 0; d <= SLOT; ++d) RowChunk<T, V>::load(coef_alpha(coef, ninst, d) + inst, alpha[d]);
+			T beta[V], go[V];
+			RowChunk<T, V>::load(coef_beta(coef, ninst) + inst, beta);
+			RowChunk<T, V>::load(coef_go(coef, ninst) + inst, go);
+			for (unsigned k = threadIdx.x * V; k < cnt; k += kBlock * V) {
+				const size_t e = base + k;
+				T x[V], p[SLOT + 1][V], r[V];
+				RowChunk<T, V>::load(X + e, x);
+#pragma unroll
+				for (int d = 0; d < SLOT; ++d) RowChunk<T, V>::load(P.p[d] + e, p[d]);
+				RowChunk<T, V>::load(p0 + e, p[SLOT]);
+				RowChunk<T, V>::load(R + e, r);
+#pragma unroll
+				for (int j = 0; j < V; ++j) {
+#pragma unroll
+					for (int d = 0; d <= SLOT; ++d) x[j] = alpha[d][j] * p[d][j] + x[j];
+					r[j] = beta[j] * p[SLOT][j] + (go[j] != T(0) ? r[j] : T(0));
+				}
+				RowChunk<T, V>::store(X + e, x);
+				if (state == kRunning) RowChunk<T, V>::store(p1 + e, r);
+			}
+		} else {
+			T beta[V], go[V];
+			RowChunk<T, V>::load(coef_beta(coef, ninst) + inst, beta);
+			RowChunk<T, V>::load(coef_go(coef, ninst) + inst, go);
+			for (unsigned k = threadIdx.x * V; k < cnt; k += kBlock * V) {
+				T p[V], r[V];
+				RowChunk<T, V>::load(p0 + base + k, p);
+				RowChunk<T, V>::load(R + base + k, r);
+#pragma unroll
+				for (int j = 0; j < V; ++j) r[j] = beta[j] * p[j] + (go[j] != T(0) ? r[j] : T(0));
+				RowChunk<T, V>::store(p1 + base + k, r);
+			}
+		}
+	}
+}
+
+// The first direction after a reliable update, in slot 0: P = R + beta P of the
+// active instances, from the slot that each system stopped at.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void k_b_restart(size_t ntiles, const uint32_t *tile_row0,
+                                                      const uint32_t *tile_row1, const uint32_t *tile_sys, int nrhs,
+                                                      Dirs<T> P, const T *R, const BatchInst *in,
+                                                      const int *sys_active, const int *sys_slot) {
+	for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
+		const int sys = tile_sys[t];
+		if (sys_active[sys] != kRunning) continue;
 		const size_t base = (size_t)tile_row0[t] * nrhs;
 		const size_t cnt = (size_t)(tile_row1[t] - tile_row0[t]) * nrhs;
-		const int sys = tile_sys[t];
-		const int r = threadIdx.x % nrhs;
-		const BatchInst &I = in[sys * nrhs + r];
-		if (!I.active) continue;
-		const T beta = (T)I.beta;
-		for (size_t k = threadIdx.x; k < cnt; k += kBlock) P[base + k] = beta * P[base + k] + R[base + k];
+		const T *p0 = P.p[0];
+#pragma unroll
+		for (int d = 1; d < batch_dirs<T>(); ++d)
+			if (sys_slot[sys] == d) p0 = P.p[d];
+		const BatchInst &I = in[sys * nrhs + threadIdx.x % nrhs];
+		const T beta = I.active ? (T)I.beta : T(1);
+		const bool go = I.active != 0;
+		for (size_t k = threadIdx.x; k < cnt; k += kBlock)
+			P.p[0][base + k] = beta * p0[base + k] + (go ? R[base + k] : T(0));
 	}
 }
 
@@ -730,9 +866,12 @@ struct alp_hip_batch_s {
 	unsigned *nactive = nullptr;
 	double *rnorm = nullptr, *bnorm = nullptr;
 	int *outer_active = nullptr;
-	int *sys_active = nullptr;        // 1 while any right-hand side of the system is active
+	int *sys_active = nullptr;        // kRunning while any right-hand side of the system is active
+	int *sys_slot = nullptr;          // slot of the system's last direction
+	double *coef = nullptr;           // scalars of the vector kernels, in their type
 	double *R = nullptr, *P = nullptr, *AP = nullptr;
-	float *R32 = nullptr, *P32 = nullptr, *AP32 = nullptr, *X32 = nullptr;
+	float *R32 = nullptr, *P32 = nullptr, *AP32 = nullptr, *X32 = nullptr;  // AP32 is the second half of P32's
+	size_t pad = 0;                   // entries of a block vector, rounded up to 16-byte pieces
 };
 
 namespace alp {
@@ -804,8 +943,8 @@ static void free_batch(alp_hip_batch_s *B) {
 	dia_free(B->dia);
 	void *ps[] = {B->srow, B->soff, B->tile_sl0,
 	              B->off, B->idx, B->val, B->val32, B->row_sys, B->sys, B->tile_row0, B->tile_row1, B->tile_sys,
-	              B->tile0, B->part, B->inst, B->nactive, B->rnorm, B->bnorm, B->outer_active, B->sys_active, B->R, B->P, B->AP,
-	              B->R32, B->P32, B->AP32, B->X32};
+	              B->tile0, B->part, B->inst, B->nactive, B->rnorm, B->bnorm, B->outer_active, B->sys_active, B->sys_slot,
+	              B->coef, B->R, B->P, B->AP, B->R32, B->P32, B->X32};
 	for (void *p : ps)
 		if (p) hipFree(p);
 }
@@ -816,33 +955,64 @@ static alp_rc_t bmalloc(T **p, size_t n) {
 	return ALP_SUCCESS;
 }
 
+// The direction slots: the vectors of the solver's own type first, then those of
+// the type that it does not iterate in.
+template <typename T>
+static Dirs<T> batch_slots(const alp_hip_batch_s *B) {
+	Dirs<T> d;
+	if constexpr (sizeof(T) == 4) {
+		d.p[0] = B->P32;
+		d.p[1] = reinterpret_cast<float *>(B->P);
+		d.p[2] = d.p[1] + B->pad;
+		d.p[3] = reinterpret_cast<float *>(B->AP);
+	} else {
+		d.p[0] = B->P;
+		d.p[1] = reinterpret_cast<double *>(B->P32);
+	}
+	return d;
+}
+
 // Iterate the inner CG on precision T until no instance is active.
 template <typename T>
-static alp_rc_t batch_iterate(alp_hip_batch_s *B, const T *val, T *X, T *R, T *P, T *AP, size_t max_iter,
-                              size_t *its, bool acc64 = false) {
+static alp_rc_t batch_iterate(alp_hip_batch_s *B, const T *val, T *X, T *R, T *AP, size_t max_iter, size_t *its,
+                              bool acc64 = false) {
 	hipStream_t s = stream();
 	const unsigned nsys = (unsigned)B->nsys;
 	const int nr = (int)B->nrhs;
 	const size_t g = B->ntiles < (size_t)fill_blocks(8) ? B->ntiles : fill_blocks(8);
-	auto iteration = [&](hipStream_t st) {
+	constexpr int V = 16 / (int)sizeof(T), D = batch_dirs<T>();
+	const Dirs<T> P = batch_slots<T>(B);
+	T *coef = reinterpret_cast<T *>(B->coef);
+	const size_t ninst = B->nsys * B->nrhs;
+	const bool wide = nr % V == 0;
+	auto iteration = [&](hipStream_t st, int slot) {
 		if (acc64)  // reliable updates: FP64 row sums of the FP32 data
-			launch_spmm<T, true, false, double>(B, B->W, val, P, nullptr, AP, st, B->sys_active);
+			launch_spmm<T, true, false, double>(B, B->W, val, P.p[slot], nullptr, AP, st, B->sys_active);
 		else
-			launch_spmm<T, true, false>(B, sizeof(T) == 8 ? B->W64 : B->W, val, P, nullptr, AP, st, B->sys_active);
-		hipLaunchKernelGGL(k_b_alpha, dim3(nsys), dim3(kBlock), 0, st, nr, (const double *)B->part,
-		                   (const uint32_t *)B->tile0, B->inst);
-		hipLaunchKernelGGL(k_b_update<T>, dim3(g), dim3(kBlock), 0, st, B->ntiles, (const uint32_t *)B->tile_row0,
-		                   (const uint32_t *)B->tile_row1, (const uint32_t *)B->tile_sys, nr, X, R, (const T *)P,
-		                   (const T *)AP, (const BatchInst *)B->inst, B->part, (const int *)B->sys_active);
-		hipLaunchKernelGGL(k_b_beta, dim3(nsys), dim3(kBlock), 0, st, nr, (const double *)B->part,
-		                   (const uint32_t *)B->tile0, B->inst, (unsigned long long)max_iter, B->nactive,
-		                   B->sys_active);
-		hipLaunchKernelGGL(k_b_dir<T>, dim3(g), dim3(kBlock), 0, st, B->ntiles, (const uint32_t *)B->tile_row0,
-		                   (const uint32_t *)B->tile_row1, (const uint32_t *)B->tile_sys, nr, P, (const T *)R,
-		                   (const BatchInst *)B->inst, (const int *)B->sys_active);
+			launch_spmm<T, true, false>(B, sizeof(T) == 8 ? B->W64 : B->W, val, P.p[slot], nullptr, AP, st,
+			                            B->sys_active);
+		hipLaunchKernelGGL(k_b_alpha<T>, dim3(nsys), dim3(kBlock), 0, st, nr, (const double *)B->part,
+		                   (const uint32_t *)B->tile0, B->inst, coef, ninst, slot, B->sys_active);
+		hipLaunchKernelGGL((wide ? k_b_update<T, V> : k_b_update<T, 1>), dim3(g), dim3(kBlock), 0, st, B->ntiles,
+		                   (const uint32_t *)B->tile_row0, (const uint32_t *)B->tile_row1,
+		                   (const uint32_t *)B->tile_sys, nr, R, (const T *)AP, (const T *)(coef + slot * ninst),
+		                   B->part, (const int *)B->sys_active);
+		hipLaunchKernelGGL(k_b_beta<T>, dim3(nsys), dim3(kBlock), 0, st, nr, (const double *)B->part,
+		                   (const uint32_t *)B->tile0, B->inst, (unsigned long long)max_iter, B->nactive, coef, ninst,
+		                   slot, B->sys_active, B->sys_slot);
+		auto dir = slot == 0 ? (wide ? k_b_dir<T, V, 0> : k_b_dir<T, 1, 0>)
+		                     : (wide ? k_b_dir<T, V, 1> : k_b_dir<T, 1, 1>);
+		if constexpr (D == 4) {
+			if (slot == 2) dir = wide ? k_b_dir<T, V, 2> : k_b_dir<T, 1, 2>;
+			if (slot == 3) dir = wide ? k_b_dir<T, V, 3> : k_b_dir<T, 1, 3>;
+		}
+		hipLaunchKernelGGL(dir, dim3(g), dim3(kBlock), 0, st, B->ntiles, (const uint32_t *)B->tile_row0,
+		                   (const uint32_t *)B->tile_row1, (const uint32_t *)B->tile_sys, nr, X, P, (const T *)R, coef,
+		                   ninst, (const int *)B->sys_active);
 	};
 	// capture `batch` iterations once; the active count of the last one is read back
 	const int batch = 8;
+	static_assert(8 % kBatchDirs == 0, "each batch starts at slot 0");
 	hipGraph_t graph = nullptr;
 	hipGraphExec_t exec = nullptr;
 	bool use_graph = false;
@@ -850,7 +1020,7 @@ static alp_rc_t batch_iterate(alp_hip_batch_s *B, const T *val, T *X, T *R, T *P
 		for (int i = 0; i < batch; ++i) {
 			// nactive counts the instances still active after each iteration
 			hipLaunchKernelGGL(k_b_zero, dim3(1), dim3(1), 0, s, B->nactive);
-			iteration(s);
+			iteration(s, i % D);
 		}
 		if (hipStreamEndCapture(s, &graph) == hipSuccess &&
 		    hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0) == hipSuccess)
@@ -868,7 +1038,7 @@ static alp_rc_t batch_iterate(alp_hip_batch_s *B, const T *val, T *X, T *R, T *P
 		} else {
 			for (int i = 0; i < batch; ++i) {
 				hipLaunchKernelGGL(k_b_zero, dim3(1), dim3(1), 0, s, B->nactive);
-				iteration(s);
+				iteration(s, i % D);
 			}
 		}
 		done_its += batch;
@@ -920,6 +1090,7 @@ static alp_rc_t batch_assemble(alp_hip_batch_s *B, Fill &&fill) {
 	B->nrows = B->row0[nsys];
 	B->ntiles = trow0.size();
 	const size_t ntot = B->nrows * nrhs, ninst = nsys * nrhs;
+	B->pad = (ntot + 3) / 4 * 4;
 	hipStream_t st = stream();
 	std::vector<uint32_t> rsys(B->nrows);
 	for (size_t s = 0; s < nsys; ++s)
@@ -932,10 +1103,11 @@ static alp_rc_t batch_assemble(alp_hip_batch_s *B, Fill &&fill) {
 	    (rc = bmalloc(&B->part, B->ntiles * nrhs)) || (rc = bmalloc(&B->inst, ninst)) ||
 	    (rc = bmalloc(&B->nactive, 1)) || (rc = bmalloc(&B->rnorm, ninst)) || (rc = bmalloc(&B->bnorm, ninst)) ||
 	    (rc = bmalloc(&B->outer_active, ninst)) || (rc = bmalloc(&B->sys_active, nsys)) ||
-	    (rc = bmalloc(&B->R, ntot)) || (rc = bmalloc(&B->P, ntot)) || (rc = bmalloc(&B->AP, ntot)) ||
-	    (rc = bmalloc(&B->R32, ntot)) || (rc = bmalloc(&B->P32, ntot)) || (rc = bmalloc(&B->AP32, ntot)) ||
-	    (rc = bmalloc(&B->X32, ntot)))
+	    (rc = bmalloc(&B->sys_slot, nsys)) || (rc = bmalloc(&B->coef, ninst * (kBatchDirs + 2))) ||
+	    (rc = bmalloc(&B->R, ntot)) || (rc = bmalloc(&B->P, B->pad)) || (rc = bmalloc(&B->AP, B->pad)) ||
+	    (rc = bmalloc(&B->R32, ntot)) || (rc = bmalloc(&B->P32, 2 * B->pad)) || (rc = bmalloc(&B->X32, ntot)))
 		return rc;
+	B->AP32 = B->P32 + B->pad;
 	if (copy_sync(B->row_sys, rsys.data(), 4 * B->nrows, hipMemcpyHostToDevice) != hipSuccess ||
 	    copy_sync(B->tile_row0, trow0.data(), 4 * B->ntiles, hipMemcpyHostToDevice) != hipSuccess ||
 	    copy_sync(B->tile_row1, trow1.data(), 4 * B->ntiles, hipMemcpyHostToDevice) != hipSuccess ||
@@ -1223,7 +1395,7 @@ ALP_EXPORT alp_rc_t alp_hip_batch_solve(alp_hip_batch_t B, const double *d_B, do
 		                   B->sys_active);
 		ALP_LAUNCH_CHECK();
 		size_t it = 0;
-		ALP_TRY(batch_iterate<double>(B, B->val, d_X, B->R, B->P, B->AP, max_iter, &it));
+		ALP_TRY(batch_iterate<double>(B, B->val, d_X, B->R, B->AP, max_iter, &it));
 		ALP_HIP_TRY(copy_sync(hin.data(), B->inst, sizeof(BatchInst) * ninst, hipMemcpyDeviceToHost));
 		for (int i = 0; i < ninst; ++i) its[i] = hin[i].iter;
 	} else if (precision == 1) {
@@ -1231,6 +1403,7 @@ ALP_EXPORT alp_rc_t alp_hip_batch_solve(alp_hip_batch_t B, const double *d_B, do
 		// passes instead of 7 for 435 rather than 410 iterations, 5% faster overall
 		const double delta = 0.01;
 		ALP_HIP_TRY(hipMemsetAsync(B->P32, 0, sizeof(float) * ntot, s));
+		ALP_HIP_TRY(hipMemsetAsync(B->sys_slot, 0, sizeof(int) * B->nsys, s));
 		for (int first = 1;; first = 0) {
 			// X += X32 (the last segment's update, accumulated in FP32: a group-wise
 			// update of the FP64 solution), X32 = 0; then the FP64 residual R = B - A X
@@ -1255,11 +1428,12 @@ ALP_EXPORT alp_rc_t alp_hip_batch_solve(alp_hip_batch_t B, const double *d_B, do
 			if (act == 0) break;  // every instance converged or ran out of iterations
 			if (!first) ++nouter;
 			// P = R32 + beta P for the active instances (beta = 0 on the first segment)
-			hipLaunchKernelGGL(k_b_dir<float>, dim3(g), dim3(kBlock), 0, s, B->ntiles, (const uint32_t *)B->tile_row0,
-			                   (const uint32_t *)B->tile_row1, (const uint32_t *)B->tile_sys, nr, B->P32,
-			                   (const float *)B->R32, (const BatchInst *)B->inst, (const int *)B->sys_active);
+			hipLaunchKernelGGL(k_b_restart<float>, dim3(g), dim3(kBlock), 0, s, B->ntiles,
+			                   (const uint32_t *)B->tile_row0, (const uint32_t *)B->tile_row1,
+			                   (const uint32_t *)B->tile_sys, nr, batch_slots<float>(B), (const float *)B->R32,
+			                   (const BatchInst *)B->inst, (const int *)B->sys_active, (const int *)B->sys_slot);
 			size_t it = 0;
-			ALP_TRY(batch_iterate<float>(B, B->val32, B->X32, B->R32, B->P32, B->AP32, max_iter, &it, true));
+			ALP_TRY(batch_iterate<float>(B, B->val32, B->X32, B->R32, B->AP32, max_iter, &it, true));
 		}
 		ALP_HIP_TRY(copy_sync(hin.data(), B->inst, sizeof(BatchInst) * ninst, hipMemcpyDeviceToHost));
 		for (int i = 0; i < ninst; ++i) its[i] = hin[i].iter;
@@ -1288,7 +1462,7 @@ ALP_EXPORT alp_rc_t alp_hip_batch_solve(alp_hip_batch_t B, const double *d_B, do
 			                   B->nactive, B->sys_active);
 			ALP_LAUNCH_CHECK();
 			size_t it = 0;
-			ALP_TRY(batch_iterate<float>(B, B->val32, B->X32, B->R32, B->P32, B->AP32, max_iter, &it));
+			ALP_TRY(batch_iterate<float>(B, B->val32, B->X32, B->R32, B->AP32, max_iter, &it));
 			ALP_HIP_TRY(copy_sync(hin.data(), B->inst, sizeof(BatchInst) * ninst, hipMemcpyDeviceToHost));
 			for (int i = 0; i < ninst; ++i) its[i] += hin[i].iter;
 			hipLaunchKernelGGL(k_b_up, dim3(fill_blocks(8)), dim3(kBlock), 0, s, ntot, nr, d_X, (const float *)B->X32,
