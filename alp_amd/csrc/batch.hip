@@ -10,11 +10,11 @@
 // per-instance dot product is a fixed-order fold of per-tile partials.
 //
 // One iteration for all (system, rhs) instances is five launches -- SpMM with the
-// p.Ap partials, per-instance alpha, x/r update with the r.r partials,
-// per-instance beta and convergence flags, direction update -- captured once in
-// a hipGraph and replayed; converged instances freeze (their scalars are 0 and
-// their flags stop updates), the host only reads the active count between
-// batches of iterations.
+// p.Ap partials, per-instance alpha, residual update with the r.r partials,
+// per-instance beta and convergence flags, direction update (with X's steps of the
+// last few directions) -- captured once in a hipGraph and replayed; converged
+// instances freeze (their scalars are 0 and their flags stop updates), the host only
+// reads the active count between batches of iterations.
 //
 // precision 0: FP64 CG. precision 1: FP32 SpMM (FP64 row sums) and CG iterations
 // with reliable FP64 residual updates (X kept in FP64). precision 2: FP32 SpMM and
@@ -23,6 +23,7 @@
 #include "spmv_device.hpp"
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -105,6 +106,15 @@ __global__ __launch_bounds__(kBlock) void k_lap_fill(size_t nrows, const SysDesc
 	});
 }
 
+// a system whose rows are all subsets of one list of (column - row, value) pairs
+struct BatchTemplate {
+	unsigned w;
+	int32_t dmin, dmax;  // of the offsets and 0
+	int32_t d[kDiaSlots];
+	float v32[kDiaSlots];
+	double v64[kDiaSlots];
+};
+
 // ---- SpMM with per-tile, per-rhs partial dots -----------------------------------------------
 // W lanes per row, each lane owns nrhs / W right-hand sides (RPL). With DOT, the
 // partial of sum_i p[i][r] * (A p)[i][r] over the tile goes to part[tile*nrhs + r].
@@ -149,6 +159,47 @@ struct RowChunk {
 	}
 };
 
+// v of the lane K places on in the same row of 16 lanes, cyclically
+template <int K>
+__device__ __forceinline__ double rotate16(double v) {
+	const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+	const unsigned lo = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)u, 0x120 + K, 0xF, 0xF, true);
+	const unsigned hi = (unsigned)__builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), 0x120 + K, 0xF, 0xF, true);
+	return __longlong_as_double((long long)((unsigned long long)hi << 32 | lo));
+}
+
+// The per-right-hand-side sums of a tile, from the sums of its lanes over their rows:
+// lanes with the same threadIdx.x % W own the same right-hand sides. Within 16 lanes
+// by register moves, the sixteen groups of a block through LDS: a whole tree of
+// ds_bpermute moves took 23 us of the 287 of k_spmm_const's FP32 product (10.3 M rows).
+constexpr int kGroups16 = kBlock / 16;
+template <int W, int RPL>
+__device__ __forceinline__ void tile_partials(const double (&acc)[RPL], double (&red)[kGroups16][W * RPL],
+                                              double *out) {
+	const int lane = threadIdx.x % W;
+	double v[RPL];
+#pragma unroll
+	for (int q = 0; q < RPL; ++q) {
+		v[q] = acc[q];
+		if constexpr (W <= 8) v[q] += rotate16<8>(v[q]);
+		if constexpr (W <= 4) v[q] += rotate16<4>(v[q]);
+		if constexpr (W <= 2) v[q] += rotate16<2>(v[q]);
+		if constexpr (W <= 1) v[q] += rotate16<1>(v[q]);
+	}
+	__syncthreads();
+	if ((threadIdx.x % 16) < W) {
+#pragma unroll
+		for (int q = 0; q < RPL; ++q) red[threadIdx.x / 16][lane * RPL + q] = v[q];
+	}
+	__syncthreads();
+	if (threadIdx.x < W * RPL) {
+		double s = 0.0;
+#pragma unroll
+		for (int w = 0; w < kGroups16; ++w) s += red[w][threadIdx.x];
+		out[threadIdx.x] = s;
+	}
+}
+
 template <typename T, int W, int RPL, bool DOT, bool RES, typename A = T, bool XCD = false>
 __global__ __launch_bounds__(kBlock) void k_spmm(size_t ntiles, const uint32_t *tile_row0, const uint32_t *tile_row1,
                                                  const uint64_t *__restrict__ off, const uint32_t *__restrict__ idx,
@@ -157,7 +208,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm(size_t ntiles, const uint32_t *
                                                  const int *sys_active, const uint32_t *tile_sys) {
 	constexpr int NR = W * RPL;
 	constexpr int kRows = kBlock / W;
-	__shared__ double red[kBlock / kWave][NR];
+	__shared__ double red[kGroups16][NR];
 	const int lane = threadIdx.x % W;
 	const unsigned grp = threadIdx.x / W;
 	// XCD: each XCD walks one contiguous range of tiles, so the X rows that
@@ -209,26 +260,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm(size_t ntiles, const uint32_t *
 				}
 			}
 		}
-		if (DOT || RES) {
-			// fold over the rows of the tile: lanes with the same `lane` own the same rhs
-#pragma unroll
-			for (int q = 0; q < RPL; ++q) {
-				double v = acc_dot[q];
-				for (int s = kWave / 2; s >= W; s >>= 1) v += __shfl_xor(v, s, kWave);
-				acc_dot[q] = v;
-			}
-			__syncthreads();
-			if ((threadIdx.x % kWave) < W) {
-#pragma unroll
-				for (int q = 0; q < RPL; ++q) red[threadIdx.x / kWave][lane * RPL + q] = acc_dot[q];
-			}
-			__syncthreads();
-			if (threadIdx.x < NR) {
-				double s = 0.0;
-				for (int w = 0; w < kBlock / kWave; ++w) s += red[w][threadIdx.x];
-				part[t * NR + threadIdx.x] = s;
-			}
-		}
+		if (DOT || RES) tile_partials<W, RPL>(acc_dot, red, part + t * NR);
 	}
 }
 
@@ -253,7 +285,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_dia(size_t ntiles, const uint32
 	constexpr int kRows = kBlock / W;     // rows per pass of the block
 	constexpr int kWaveRows = kWave / W;  // rows per wavefront, all in one slice
 	constexpr int U = 4;                  // slots in flight
-	__shared__ double red[kBlock / kWave][NR];
+	__shared__ double red[kGroups16][NR];
 	const int lane = threadIdx.x % W;
 	const unsigned grp = threadIdx.x / W;
 	const unsigned wl = threadIdx.x % kWave;
@@ -353,28 +385,200 @@ __global__ __launch_bounds__(kBlock) void k_spmm_dia(size_t ntiles, const uint32
 				}
 			}
 		}
-		if (DOT) {
+		if (DOT) tile_partials<W, RPL>(acc_dot, red, part + t * NR);
+	}
+}
+
+// The product (RES: the residual) over systems in constant form: every row of a
+// system is a subset of the system's (offset, value) template, and 4 bytes per row say
+// which entries it has. No values or column indices are read; a slot's X rows lie at
+// one uniform distance from the lane's own, so its address is a scalar base plus the
+// lane's offset, and the loads of eight slots are in flight together, with no branch
+// between them (a branch per slot: 380 us where this takes 264). A row that lacks an
+// entry reads what lies there (another system's row) and drops it by its mask; near the
+// ends of the batch the addresses are chosen per lane. The fold and the partials are
+// those of k_spmm, bit for bit. 10.3 M rows, 8 right-hand sides, 7 entries: FP32 data
+// with FP64 sums 430 us in diagonal form, 264 us here (0.7 GB: 2.7 TB/s; the wait is
+// for X lines on their way to L1, which the slots of a row share); FP64 690 -> 505 us.
+template <typename T, int W, int RPL, bool DOT, bool RES, typename A = T, bool XCD = false>
+__global__ __launch_bounds__(kBlock) void k_spmm_const(size_t ntiles, const uint32_t *tile_row0,
+                                                       const uint32_t *tile_row1,
+                                                       const uint32_t *__restrict__ tile_sl0,
+                                                       const uint32_t *__restrict__ mask,
+                                                       const BatchTemplate *__restrict__ tpl, size_t nrows,
+                                                       const T *__restrict__ X, const T *__restrict__ Bm,
+                                                       T *__restrict__ Y, double *part, const int *sys_active,
+                                                       const uint32_t *tile_sys) {
+	constexpr int NR = W * RPL;
+	constexpr int kRows = kBlock / W;                      // rows per pass of the block
+	constexpr int kWaveRows = kWave / W;                   // rows per wavefront, all in one slice
+	constexpr unsigned U = RPL * sizeof(T) <= 16 ? 8 : 4;  // slots in flight
+	__shared__ double red[kGroups16][NR];
+	const unsigned rl = threadIdx.x % kWave / W;           // the lane's row in the wavefront's rows
+	const unsigned lane_off = threadIdx.x % kWave * RPL;   // = rl * NR + (lane of the row) * RPL
+	const unsigned wave_row = (threadIdx.x / kWave) * kWaveRows;
+	const WorkSplit ws = XCD ? xcd_split(ntiles) : WorkSplit{blockIdx.x, ntiles, gridDim.x};
+	// a tile's description is read one tile ahead
+	uint32_t next_sys = 0, next_r0 = 0, next_r1 = 0, next_sl = 0;
+	if (ws.first < ws.last) {
+		next_sys = tile_sys[ws.first];
+		next_r0 = tile_row0[ws.first];
+		next_r1 = tile_row1[ws.first];
+		next_sl = tile_sl0[ws.first];
+	}
+	for (size_t t = ws.first; t < ws.last; t += ws.step) {
+		const uint32_t sys = next_sys, r0 = next_r0, r1 = next_r1, sl0 = next_sl;
+		const size_t tn = t + ws.step < ws.last ? t + ws.step : t;
+		next_sys = tile_sys[tn];
+		next_r0 = tile_row0[tn];
+		next_r1 = tile_row1[tn];
+		next_sl = tile_sl0[tn];
+		if (!RES && sys_active && sys_active[sys] != kRunning) continue;
+		const BatchTemplate &tp = tpl[sys];
+		const unsigned w = tp.w;
+		const uint32_t *tmask = mask + (size_t)sl0 * kSellRows;
+		double acc_dot[RPL];
 #pragma unroll
-			for (int q = 0; q < RPL; ++q) {
-				double v = acc_dot[q];
-				for (int sh = kWave / 2; sh >= W; sh >>= 1) v += __shfl_xor(v, sh, kWave);
-				acc_dot[q] = v;
-			}
-			__syncthreads();
-			if ((threadIdx.x % kWave) < W) {
+		for (int q = 0; q < RPL; ++q) acc_dot[q] = 0.0;
+		for (uint32_t rb = r0; rb < r1; rb += kRows) {
+			const uint32_t wr = (uint32_t)__builtin_amdgcn_readfirstlane(rb + wave_row);  // the wavefront's first row
+			if (wr >= r1) continue;
+			const uint32_t r = wr + rl;
+			const bool act = r < r1;
+			const uint32_t bits = act ? tmask[r - r0] : 0u;
+			const bool inside = (int64_t)wr + tp.dmin >= 0 && (int64_t)wr + kWaveRows - 1 + tp.dmax < (int64_t)nrows;
+			A acc[RPL];
 #pragma unroll
-				for (int q = 0; q < RPL; ++q) red[threadIdx.x / kWave][lane * RPL + q] = acc_dot[q];
+			for (int q = 0; q < RPL; ++q) acc[q] = A(0);
+			for (unsigned q0 = 0; q0 < w; q0 += U) {
+				T xv[U][RPL];
+				if (inside) {
+#pragma unroll
+					for (unsigned u = 0; u < U; ++u) {
+						const unsigned q = q0 + u < w ? q0 + u : w - 1;
+						const T *xb = X + ((int64_t)wr + tp.d[q]) * NR;
+						RowChunk<T, RPL>::load(xb + lane_off, xv[u]);
+					}
+				} else {
+#pragma unroll
+					for (unsigned u = 0; u < U; ++u) {
+						const unsigned q = q0 + u < w ? q0 + u : w - 1;
+						const int64_t j = (bits >> q) & 1u ? (int64_t)r + tp.d[q] : (int64_t)wr;
+						RowChunk<T, RPL>::load(X + j * NR + lane_off % NR, xv[u]);
+					}
+				}
+#pragma unroll
+				for (unsigned u = 0; u < U; ++u) {
+					// slots past the width have their bit clear
+					const unsigned q = q0 + u < w ? q0 + u : w - 1;
+					const A av = sizeof(T) == 8 ? (A)tp.v64[q] : (A)tp.v32[q];
+#pragma unroll
+					for (int j = 0; j < RPL; ++j) {
+						const A x = (A)keep_if(bits, q0 + u, xv[u][j]);
+						// FP32 products are exact in FP64: fused or not is the same sum
+						if constexpr (sizeof(A) > sizeof(T))
+							acc[j] = __builtin_fma(av, x, acc[j]);
+						else
+							acc[j] += av * x;
+					}
+				}
 			}
-			__syncthreads();
-			if (threadIdx.x < NR) {
-				double sum = 0.0;
-				for (int wv = 0; wv < kBlock / kWave; ++wv) sum += red[wv][threadIdx.x];
-				part[t * NR + threadIdx.x] = sum;
+			if (act) {
+				const size_t at = (size_t)wr * NR + lane_off;
+				T v[RPL];
+				if (RES) {
+					RowChunk<T, RPL>::load(Bm + at, v);
+#pragma unroll
+					for (int q = 0; q < RPL; ++q) {
+						v[q] = (T)(v[q] - acc[q]);
+						acc_dot[q] += (double)v[q] * (double)v[q];
+					}
+				} else {
+#pragma unroll
+					for (int q = 0; q < RPL; ++q) v[q] = (T)acc[q];
+					if (DOT) {
+						T pv[RPL];
+						RowChunk<T, RPL>::load(X + at, pv);
+#pragma unroll
+						for (int q = 0; q < RPL; ++q) acc_dot[q] += (double)v[q] * (double)pv[q];
+					}
+				}
+				RowChunk<T, RPL>::store(Y + at, v);
 			}
+		}
+		if (DOT || RES) tile_partials<W, RPL>(acc_dot, red, part + t * NR);
+	}
+}
+
+// A system's template: the entries of its first longest row, if they are distinct
+// and finite in both precisions (an absent entry folds v * 0); one block per system.
+__global__ __launch_bounds__(kBlock) void k_b_template(const uint64_t *row0, const uint64_t *off, const uint32_t *idx,
+                                                       const double *val, BatchTemplate *tpl, unsigned *bad) {
+	__shared__ unsigned long long s_best;
+	if (threadIdx.x == 0) s_best = 0;
+	__syncthreads();
+	const uint64_t a = row0[blockIdx.x], e = row0[blockIdx.x + 1];
+	unsigned long long best = 0;  // length in the high half, then the lowest row
+	for (uint64_t r = a + threadIdx.x; r < e; r += kBlock) {
+		const uint64_t len = off[r + 1] - off[r];
+		const unsigned long long k = (len < 0xFFFF ? len : 0xFFFFull) << 32 | (0xFFFFFFFFull - (r - a));
+		best = k > best ? k : best;
+	}
+	atomicMax(&s_best, best);
+	__syncthreads();
+	const uint64_t r = a + (0xFFFFFFFFull - (s_best & 0xFFFFFFFFull));
+	const uint64_t b = off[r];
+	const uint64_t w = off[r + 1] - b;
+	BatchTemplate &T = tpl[blockIdx.x];
+	if (w > kDiaSlots) {
+		if (threadIdx.x == 0) {
+			T.w = 0;
+			*bad = 1u;
+		}
+		return;
+	}
+	if (threadIdx.x == 0) {
+		T.w = (unsigned)w;
+		T.dmin = T.dmax = 0;
+		for (unsigned q = 0; q < w; ++q) {
+			const int64_t d = (int64_t)idx[b + q] - (int64_t)r;
+			const double v = val[b + q];
+			if (d < INT32_MIN || d > INT32_MAX || !(fabs(v) <= DBL_MAX) || !(fabsf((float)v) <= FLT_MAX)) *bad = 1u;
+			for (unsigned p = 0; p < q; ++p)
+				if (idx[b + p] == idx[b + q]) *bad = 1u;
+			T.d[q] = (int32_t)d;
+			T.v64[q] = v;
+			T.v32[q] = (float)v;
+			T.dmin = (int32_t)d < T.dmin ? (int32_t)d : T.dmin;
+			T.dmax = (int32_t)d > T.dmax ? (int32_t)d : T.dmax;
 		}
 	}
 }
 
+// One wavefront per slice: every row's entries against the system's template, in
+// order; *bad when a row is no subsequence of it.
+__global__ __launch_bounds__(kBlock) void k_b_match(size_t nslices, const uint32_t *srow, const uint32_t *row_sys,
+                                                    const uint64_t *off, const uint32_t *idx, const double *val,
+                                                    const BatchTemplate *tpl, uint32_t *mask, unsigned *bad) {
+	const size_t sl = (size_t)blockIdx.x * (kBlock / kSellRows) + threadIdx.x / kSellRows;
+	if (sl >= nslices) return;
+	const unsigned lane = threadIdx.x % kSellRows;
+	const uint32_t r = srow[sl] + lane;
+	const bool act = r < srow[sl + 1];
+	const BatchTemplate &T = tpl[row_sys[srow[sl]]];
+	const uint64_t b = act ? off[r] : 0;
+	const uint64_t len = act ? off[r + 1] - b : 0;
+	uint32_t bits = 0;
+	uint64_t j = 0;
+	for (unsigned q = 0; q < T.w && j < len; ++q)
+		if ((int64_t)idx[b + j] - (int64_t)r == T.d[q] &&
+		    __double_as_longlong(val[b + j]) == __double_as_longlong(T.v64[q])) {
+			bits |= 1u << q;
+			++j;
+		}
+	mask[sl * kSellRows + lane] = bits;
+	if (j != len) *bad = 1u;
+}
 // Per-system fold of the tile partials (tiles of system s: [tile0[s], tile0[s+1])),
 // one block per system: thread t folds tiles t, t + kBlock, ... for every
 // right-hand side, then a fixed tree over the block; sums[r] (LDS) gets the
@@ -857,6 +1061,11 @@ struct alp_hip_batch_s {
 	// fewer than half the slices qualify
 	DiaSlices dia;
 	size_t nslices = 0;
+	size_t ndiagonal = 0;             // slices that qualified, also where the constant form replaced theirs
+	// constant form: a template per system and a mask per row (slice by slice), when
+	// every system has one
+	BatchTemplate *tpl = nullptr;
+	uint32_t *cmask = nullptr;
 	uint32_t *srow = nullptr;         // first row of each slice (nslices + 1)
 	uint64_t *soff = nullptr;         // first entry of each slice's slot block (nslices + 1)
 	uint32_t *tile_sl0 = nullptr;     // first slice of each tile
@@ -895,7 +1104,13 @@ static void launch_spmm(alp_hip_batch_s *B, int cfg, const T *val, const T *X, c
 		if (sizeof(T) == 4 && (const void *)val == (const void *)B->val32) dval = (const T *)B->dia.val32;
 	}
 #define ALP_SPMM_X(WW, RPL, XX)                                                                                  \
-	if (dval)                                                                                                   \
+	if (B->tpl)                                                                                                 \
+		hipLaunchKernelGGL((k_spmm_const<T, WW, RPL, DOT, RES, A, XX>), dim3(grid), dim3(kBlock), 0, s,         \
+		                   B->ntiles, (const uint32_t *)B->tile_row0, (const uint32_t *)B->tile_row1,           \
+		                   (const uint32_t *)B->tile_sl0, (const uint32_t *)B->cmask,                           \
+		                   (const BatchTemplate *)B->tpl, B->nrows, X, Bm, Y, B->part, sys_active,              \
+		                   (const uint32_t *)B->tile_sys);                                                      \
+	else if (dval)                                                                                                   \
 		hipLaunchKernelGGL((k_spmm_dia<T, WW, RPL, DOT, A, XX>), dim3(grid), dim3(kBlock), 0, s, B->ntiles,     \
 		                   (const uint32_t *)B->tile_row0, (const uint32_t *)B->tile_row1,                      \
 		                   (const uint32_t *)B->tile_sl0, (const uint64_t *)B->soff,                            \
@@ -941,7 +1156,7 @@ static void launch_spmm(alp_hip_batch_s *B, int cfg, const T *val, const T *X, c
 
 static void free_batch(alp_hip_batch_s *B) {
 	dia_free(B->dia);
-	void *ps[] = {B->srow, B->soff, B->tile_sl0,
+	void *ps[] = {B->srow, B->soff, B->tile_sl0, B->tpl, B->cmask,
 	              B->off, B->idx, B->val, B->val32, B->row_sys, B->sys, B->tile_row0, B->tile_row1, B->tile_sys,
 	              B->tile0, B->part, B->inst, B->nactive, B->rnorm, B->bnorm, B->outer_active, B->sys_active, B->sys_slot,
 	              B->coef, B->R, B->P, B->AP, B->R32, B->P32, B->X32};
@@ -1069,6 +1284,51 @@ ALP_EXPORT alp_rc_t alp_hip_batch_destroy(alp_hip_batch_t B) {
 
 namespace alp {
 
+// The constant form, if every system qualifies: its products then read neither the
+// diagonal slices nor the CRS. Memory for it is optional: the other forms stay in use
+// where there is none.
+static alp_rc_t batch_const(alp_hip_batch_s *B) {
+	hipStream_t s = stream();
+	const size_t rows = B->nslices * kSellRows;
+	uint64_t *row0 = nullptr;
+	unsigned *bad = nullptr, h_bad = 0;
+	struct Free {
+		uint64_t *&a;
+		unsigned *&b;
+		~Free() {
+			if (a) hipFree(a);
+			if (b) hipFree(b);
+		}
+	} guard{row0, bad};
+	bool have = hipMalloc(&B->tpl, sizeof(BatchTemplate) * B->nsys) == hipSuccess &&
+	            hipMalloc(&B->cmask, sizeof(uint32_t) * rows) == hipSuccess &&
+	            hipMalloc(&row0, sizeof(uint64_t) * (B->nsys + 1)) == hipSuccess &&
+	            hipMalloc(&bad, sizeof(unsigned)) == hipSuccess;
+	if (have) {
+		ALP_HIP_TRY(copy_sync(row0, B->row0.data(), sizeof(uint64_t) * (B->nsys + 1), hipMemcpyHostToDevice));
+		ALP_HIP_TRY(hipMemsetAsync(bad, 0, sizeof(unsigned), s));
+		hipLaunchKernelGGL(k_b_template, dim3((unsigned)B->nsys), dim3(kBlock), 0, s, (const uint64_t *)row0,
+		                   (const uint64_t *)B->off, (const uint32_t *)B->idx, (const double *)B->val, B->tpl, bad);
+		hipLaunchKernelGGL(k_b_match, dim3((unsigned)((B->nslices + kBlock / kSellRows - 1) / (kBlock / kSellRows))),
+		                   dim3(kBlock), 0, s, B->nslices, (const uint32_t *)B->srow, (const uint32_t *)B->row_sys,
+		                   (const uint64_t *)B->off, (const uint32_t *)B->idx, (const double *)B->val,
+		                   (const BatchTemplate *)B->tpl, B->cmask, bad);
+		ALP_LAUNCH_CHECK();
+		ALP_HIP_TRY(copy_sync(&h_bad, bad, sizeof(unsigned), hipMemcpyDeviceToHost));
+	} else {
+		(void)hipGetLastError();  // the refusal is handled here
+	}
+	if (have && !h_bad) {
+		dia_free(B->dia);
+		return ALP_SUCCESS;
+	}
+	if (B->tpl) hipFree(B->tpl);
+	if (B->cmask) hipFree(B->cmask);
+	B->tpl = nullptr;
+	B->cmask = nullptr;
+	return ALP_SUCCESS;
+}
+
 // The part of a batch's construction that does not depend on where its rows come
 // from: the tiles (kRowsPerTile rows, never straddling two systems), the device
 // arrays and workspace, the FP32 value copy and the diagonal form. B->nsys,
@@ -1144,6 +1404,8 @@ static alp_rc_t batch_assemble(alp_hip_batch_s *B, Fill &&fill) {
 	    (rc = dia_build(B->dia, B->nslices, B->nrows, B->srow, B->soff, soff[B->nslices], B->off, B->idx,
 	                    ALP_VAL_F64, B->val, B->val32)))
 		return rc;
+	B->ndiagonal = B->dia.flag ? B->dia.n_dia : 0;
+	if (!(env && env[0] == '0') && const_dia_enabled() && (rc = batch_const(B))) return rc;
 	if (hipStreamSynchronize(st) != hipSuccess || hipGetLastError() != hipSuccess) return ALP_PANIC;
 	B->W = B->W64 = (int)std::min<size_t>(nrhs, 8);
 	return ALP_SUCCESS;
@@ -1283,7 +1545,7 @@ ALP_EXPORT alp_rc_t alp_hip_batch_info(alp_hip_batch_t B, size_t *nrows, size_t 
 ALP_EXPORT alp_rc_t alp_hip_batch_layout(alp_hip_batch_t B, size_t *nslices, size_t *ndiagonal) {
 	if (!B || !nslices || !ndiagonal) return ALP_ILLEGAL;
 	*nslices = B->nslices;
-	*ndiagonal = B->dia.flag ? B->dia.n_dia : 0;
+	*ndiagonal = B->ndiagonal;
 	return ALP_SUCCESS;
 }
 
