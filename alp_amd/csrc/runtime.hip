@@ -123,6 +123,43 @@ __global__ __launch_bounds__(kBlock) void k_dot(size_t n, const T *__restrict__ 
 	}
 }
 
+// The same for short vectors, in one block of sixteen wavefronts: no partials in
+// memory, no ticket and none of the fences around it, which are most of a short dot
+// product. From call to result, one block against the grid: 64 entries 8.6 us against
+// 10.7, 4096 9.3 against 12.1, 16384 11.9 against 12.8, 32768 15.7 against 12.6: the
+// line lies at 16384.
+constexpr int kSmallDotBlock = 1024;
+constexpr size_t kSmallDot = 16384;
+template <typename T>
+__global__ __launch_bounds__(kSmallDotBlock) void k_dot_small(size_t n, const T *__restrict__ x,
+                                                              const T *__restrict__ y, ScalarReport *rep,
+                                                              unsigned long long seq, double init) {
+	constexpr int U = 8;
+	__shared__ double lds[kSmallDotBlock / kWave];
+	double acc = 0.0;
+	for (size_t i0 = threadIdx.x; i0 < n; i0 += U * kSmallDotBlock) {
+		T a[U], b[U];
+#pragma unroll
+		for (int u = 0; u < U; ++u) {
+			const size_t i = i0 + (size_t)u * kSmallDotBlock;
+			a[u] = i < n ? x[i] : T(0);
+			b[u] = y ? (i < n ? y[i] : T(0)) : T(1);
+		}
+#pragma unroll
+		for (int u = 0; u < U; ++u) acc += (double)a[u] * (double)b[u];
+	}
+	acc = group_sum<kWave>(acc);
+	if (threadIdx.x % kWave == 0) lds[threadIdx.x / kWave] = acc;
+	__syncthreads();
+	if (threadIdx.x < kSmallDotBlock / kWave) {
+		const double s = group_sum<kSmallDotBlock / kWave>(lds[threadIdx.x]);
+		if (threadIdx.x == 0) {
+			rep->v[0] = init + s;
+			__hip_atomic_store(&rep->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+		}
+	}
+}
+
 static unsigned reduction_grid(size_t n) {
 	size_t g = (n + kBlock * 8 - 1) / (kBlock * 8);
 	if (g < 1) g = 1;
@@ -138,18 +175,27 @@ static unsigned stream_grid(size_t n) {
 	return static_cast<unsigned>(g);
 }
 
+// *h_z += x . y, or the sum of x (y null); n > 0
+template <typename T>
+static alp_rc_t dot_launch(size_t n, const T *x, const T *y, double *h_z) {
+	const unsigned long long seq = next_report();
+	if (n <= kSmallDot)
+		hipLaunchKernelGGL(k_dot_small<T>, dim3(1), dim3(kSmallDotBlock), 0, stream(), n, x, y, ctx().d_report, seq,
+		                   *h_z);
+	else
+		hipLaunchKernelGGL(k_dot<T>, dim3(reduction_grid(n)), dim3(kBlock), 0, stream(), n, x, y, ctx().d_partials,
+		                   ctx().d_tickets, ctx().d_report, seq, *h_z);
+	ALP_LAUNCH_CHECK();
+	return wait_report(h_z, seq, 1);
+}
+
 template <typename T>
 static alp_rc_t dot_impl(size_t n, const T *x, const T *y, double *h_z) {
 	ALP_TRY(ensure_init());
 	if (!h_z) return ALP_ILLEGAL;
 	if (n == 0) return ALP_SUCCESS;
 	if (!x || !y) return ALP_ILLEGAL;
-	const unsigned g = reduction_grid(n);
-	const unsigned long long seq = next_report();
-	hipLaunchKernelGGL(k_dot<T>, dim3(g), dim3(kBlock), 0, stream(), n, x, y, ctx().d_partials,
-	                   ctx().d_tickets, ctx().d_report, seq, *h_z);
-	ALP_LAUNCH_CHECK();
-	return wait_report(h_z, seq, 1);
+	return dot_launch(n, x, y, h_z);
 }
 
 // ---------------------------------------------------------------------------
@@ -1212,13 +1258,7 @@ ALP_EXPORT alp_rc_t alp_hip_sum_f64(size_t n, const double *x, double *h_z) {
 	ALP_TRY(ensure_init());
 	if (!h_z) return ALP_ILLEGAL;
 	if (n == 0) return ALP_SUCCESS;
-	const unsigned g = reduction_grid(n);
-	const unsigned long long seq = next_report();
-	hipLaunchKernelGGL(k_dot<double>, dim3(g), dim3(kBlock), 0, stream(), n, x,
-	                   (const double *)nullptr, ctx().d_partials, ctx().d_tickets,
-	                   ctx().d_report, seq, *h_z);
-	ALP_LAUNCH_CHECK();
-	return wait_report(h_z, seq, 1);
+	return dot_launch(n, x, (const double *)nullptr, h_z);
 }
 
 template <typename T>
