@@ -622,6 +622,62 @@ __global__ __launch_bounds__(kBlock) void k_const_step(ConstStep<T> a) {
 	}
 }
 
+// The coarsest level's sweep from z = 0, forward and backward over the colours, in one
+// workgroup with z, r and the masks in LDS: the same operations in the same order as
+// the steps above. A step of so few rows is its launch's chain (3.4 us) and little
+// else; here it is a barrier and 2.2 us, most of them the templates' scalar loads, 27 LDS
+// reads per row on one CU and the division. HPCG to 1e-10 in FP64: 88 x 56 x 40, three
+// levels, 15.0 -> 14.5 ms; 16^3, two levels, 2.97 -> 2.68 ms. With z alone in LDS and up
+// to 16384 rows a coarsest level of 24^3 was no faster (85.2 ms both at 192^3 in mixed
+// precision, 26.6 -> 27.0 at 96^3 in FP64), so the line lies where r and masks fit too.
+constexpr uint32_t kBottomRows = 7168;  // 20 bytes of LDS each in FP64
+constexpr int kBottomBlock = 1024, kBottomColours = 32;
+template <typename T>
+__global__ __launch_bounds__(kBottomBlock) void k_const_bottom(const ConstArg<T> *__restrict__ tab,
+                                                              const uint32_t *__restrict__ crow,
+                                                              const uint32_t *__restrict__ cslice,
+                                                              const uint32_t *__restrict__ mask, int ncolors,
+                                                              uint32_t n, T d, const T *__restrict__ r,
+                                                              T *__restrict__ z, const int *done) {
+	__shared__ T zs[kBottomRows], rs[kBottomRows];
+	__shared__ uint32_t ms[kBottomRows];
+	__shared__ uint32_t first[kBottomColours + 1];
+	if (done && *done) return;
+	for (uint32_t i = threadIdx.x; i < n; i += kBottomBlock) {
+		zs[i] = T(0);
+		rs[i] = r[i];
+	}
+	for (int c = 0; c < ncolors; ++c) {
+		const uint32_t r0 = crow[c], cnt = crow[c + 1] - r0;
+		const uint32_t *m = mask + (size_t)cslice[c] * kSellRows;  // a colour's slices are consecutive
+		for (uint32_t i = threadIdx.x; i < cnt; i += kBottomBlock) ms[r0 + i] = m[i];
+	}
+	if (threadIdx.x <= (unsigned)ncolors) first[threadIdx.x] = crow[threadIdx.x];
+	__syncthreads();
+	const unsigned lane = threadIdx.x % kSellRows;
+	for (int k = 0; k < 2 * ncolors; ++k) {
+		const int c = k < ncolors ? k : 2 * ncolors - 1 - k;
+		const uint32_t row1 = (uint32_t)__builtin_amdgcn_readfirstlane(first[c + 1]);
+		uint32_t r0 = (uint32_t)__builtin_amdgcn_readfirstlane(first[c] + threadIdx.x / kSellRows * kSellRows);
+		for (; r0 < row1; r0 += kBottomBlock) {
+			const uint32_t row = r0 + lane;
+			const bool act = row < row1;
+			const uint32_t at = act ? row : r0;
+			T zi;
+			if (k == 0) {
+				zi = rs[at] / d;
+			} else {
+				T xv[kDiaFullWidth];
+				gather27<T>(tab[c], (long long)r0, lane, (long long)n, zs, xv);
+				zi = ((rs[at] - sum27<T, T>(tab[c], ms[at], xv)) + zs[at] * d) / d;
+			}
+			if (act) zs[row] = zi;
+		}
+		__syncthreads();
+	}
+	for (uint32_t i = threadIdx.x; i < n; i += kBottomBlock) z[i] = zs[i];
+}
+
 // Row products over all colours: blockIdx.y is the colour; ep as in k_sell_rows.
 template <typename T, typename Ep>
 __global__ __launch_bounds__(kBlock) void k_const_rows(const ConstArg<T> *__restrict__ tab,
@@ -1543,6 +1599,14 @@ template <typename T>
 static void vcycle(alp_hip_hpcg_s *H, size_t l, hipStream_t s, const int *done) {
 	HpLevel &F = H->L[l];
 	if (l + 1 == H->L.size()) {
+		if (!F.cst.empty() && F.ncolors > 1 && F.ncolors <= kBottomColours && F.n <= kBottomRows) {
+			const ConstArg<T> *tab;
+			if constexpr (sizeof(T) == 8) tab = F.ctab; else tab = F.ctab32;
+			hipLaunchKernelGGL(k_const_bottom<T>, dim3(1), dim3(kBottomBlock), 0, s, tab, (const uint32_t *)F.crow,
+			                   (const uint32_t *)F.cslice, (const uint32_t *)F.cmask, F.ncolors, (uint32_t)F.n,
+			                   (T)F.cdiag, (const T *)Vec<T>::r(F), Vec<T>::z(F), done);
+			return;
+		}
 		rbgs<T>(F, s, done, true);
 		return;
 	}

@@ -167,6 +167,9 @@ def test_const_near_misses_keep_their_values(A, monkeypatch):
 
 @pytest.mark.parametrize("sizes,levels,pre,post", [((16, 16, 16), 2, 1, 1), ((24, 16, 40), 1, 2, 2), ((12, 20, 28), 1, 1, 1),
                                                   ((32, 16, 16), 2, 0, 1), ((16, 32, 16), 2, 1, 0), ((8, 12, 10), 0, 1, 1),
+                                                  # a coarsest level of one workgroup's most rows, and of more
+                                                  ((16, 16, 28), 0, 1, 1), ((16, 18, 26), 0, 1, 1),
+                                                  ((4, 4, 4), 1, 1, 1),
                                                   ((9, 11, 7), 0, 1, 1)])
 def test_const_hpcg_equals_kept_values(A, sizes, levels, pre, post, monkeypatch):
     """V-cycle and solves on levels in constant form (whose steps on one colour, and
