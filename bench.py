@@ -7,16 +7,20 @@ grb::mxv<dense>(y, A, x) under the FP64 plus-times semiring, i.e. y = y + A x
 (ALP's accumulate semantics, reference/blas2.hpp:1946).
 
 value = SpMV throughput in GB/s of the algorithmic bytes of the layout the timed
-kernel streams (format_bytes_per_launch) over the wall time per step. The default
-kernel streams the matrix as index-free diagonal slices:
-    8 E (values, E padded slot entries) + 393 S (per slice: a 4 B presence mask per
-    row, 32 slot offsets, a flag, the entry offset) + 8 n (x) + 16 n (y r+w)
-  = 1,731,557,376 B at 192^3.
+kernel streams (format_bytes_per_launch) over the wall time per step. The stencil's
+rows are subsets of one list of 27 (offset, value) pairs, which the default kernel
+takes as arguments; what it streams is a presence mask per row and the vectors:
+    256 S (4 B per row of the S 64-row slices) + 8 n (x) + 16 n (y r+w)
+  = 198,180,864 B at 192^3.
 roofline.achieved / roofline.frac are the same bytes over the kernel's HIP-event
 time per launch, so frac <= 1 is a fraction of the 8 TB/s HBM peak. The metric's
 CRS algorithmic bytes (12 nnz + 8 (n+1) + 8 n + 16 n = 2,495,923,112 B) over the
 same time are reported separately as crs_equivalent_gbs (they exceed what the
-hardware moves). crs_path times the CSR-stream kernel (kernel 2) forced on the same
+hardware moves). value_path times the same matrix built with a value per entry (the
+path of matrices whose slices share offsets but no one template), whose index-free
+diagonal slices stream 8 E (values, E padded slot entries) + 393 S (a 4 B mask per
+row, 32 slot offsets, a flag, the entry offset) + 8 n + 16 n = 1,731,557,376 B.
+crs_path times the CSR-stream kernel (kernel 2) forced on the same
 matrix, in CRS bytes. roofline.traffic is the measured HBM traffic per launch. The
 solve legs (FP64 and mixed-precision CG / HPCG to 1e-10 relative residual) are
 reported beside it (`solves`), and `configs` holds the other workloads: 50 CG
@@ -53,13 +57,24 @@ def spmv_bytes(n: int, nnz: int, accumulate: bool = True) -> int:
     return 12 * nnz + 8 * (n + 1) + 8 * n + (16 if accumulate else 8) * n
 
 
-def format_bytes(n: int, nnz: int, kernel: int, layout, accumulate: bool = True) -> int:
+def constant_form(kernel: int) -> bool:
+    """Whether the stencil's launches read its one (offset, value) template instead of
+    a value per entry (they do unless the build is told to keep the values, or kernel
+    4 to keep its sliced-ELL arrays)."""
+    return os.environ.get("ALP_HIP_CONST_DIA", "1")[:1] != "0" and (
+        kernel == 5 or kernel == 4 and os.environ.get("ALP_HIP_KEEP_SELL", "0")[:1] != "1")
+
+
+def format_bytes(n: int, nnz: int, kernel: int, layout, accumulate: bool = True, constant: bool = False) -> int:
     """Bytes one FP64 SpMV launch must move in the layout the kernel streams.
+    Constant form: a 4 B presence mask per row, x once and y as for CRS.
     Diagonal slices: values (8 B per padded entry), a 4 B presence mask per row,
     per slice its flag, 32 slot offsets and its entry offset; sliced-ELL slices add
     4 B column indices and read the row offsets; x once and y as for CRS."""
     slices, entries, dia = layout
     vec = 8 * n + (16 if accumulate else 8) * n
+    if constant and slices:
+        return 256 * slices + vec
     if kernel in (4, 5) and slices:
         share = dia / slices if kernel == 5 else 0.0
         per_slice = 8 + (share * (1 + 32 * 4 + 64 * 4))
@@ -126,13 +141,15 @@ def cpu_solve_reference(side: int, cg_iterations: int, hpcg_iterations: int):
     return out
 
 
-def measured_traffic(kernel: int, lanes: int, rows: int):
+def measured_traffic(kernel: int, lanes: int, rows: int, constant: bool = False):
     """HBM bytes per launch of this SpMV configuration from the committed rocprofv3
     FETCH_SIZE + WRITE_SIZE summaries (profiles/*_hbm_counters.md, calibrated on a
     copy kernel of known size), or None when none covers it."""
     import glob
     import re
-    pat = re.compile(r"traffic_bytes_per_launch:\s*(\d+)\s*\(kernel=(\d+) lanes=(\d+) rows=(\d+), accumulate\)")
+    form = "constant form, " if constant else ""
+    pat = re.compile(r"traffic_bytes_per_launch:\s*(\d+)\s*\(" + form +
+                     r"kernel=(\d+) lanes=(\d+) rows=(\d+), accumulate\)")
     for path in sorted(glob.glob(os.path.join(ROOT, "profiles", "*_hbm_counters.md"))):
         with open(path) as f:
             for m in pat.finditer(f.read()):
@@ -455,13 +472,39 @@ def main() -> int:
                   "max": round(single[-1], 2), "launches": 20, "unit": "us",
                   "note": "each launch between its own HIP events, after the timed region"}
     crs_bytes = spmv_bytes(n, nnz)
-    fbytes = format_bytes(n, nnz, kernel, layout)
+    constant = constant_form(kernel)
+    fbytes = format_bytes(n, nnz, kernel, layout, constant=constant)
     achieved = fbytes / (kern_ms * 1e-3) / 1e9
     crs_equiv = crs_bytes / (kern_ms * 1e-3) / 1e9
     value = fbytes / (ms_step * 1e-3) / 1e9
     log(f"[bench] mxv: {kern_ms * 1e3:.1f} us/launch (events), {ms_step * 1e3:.1f} us/step (wall), "
         f"{achieved:.0f} GB/s of the streamed layout ({fbytes} B; slices={layout[0]} entries={layout[1]} "
         f"diagonal={layout[2]}), {crs_equiv:.0f} GB/s CRS-equivalent")
+
+    # the same matrix with a value per entry
+    value_path = None
+    if constant and not args.kernel:
+        os.environ["ALP_HIP_CONST_DIA"] = "0"
+        V = alp.Matrix.stencil27(side, side, side)
+        del os.environ["ALP_HIP_CONST_DIA"]
+        vk = V.get_kernel()
+        for _ in range(max(2, args.warmup // 4)):
+            L.alp_hip_mxv(V.h, alp.PLUS_TIMES_F64, alp.DENSE, y.ptr, x.ptr, None)
+        v_steps = max(10, args.steps // 4)
+        alp.check(L.alp_hip_timer_start(), "timer_start")
+        for _ in range(v_steps):
+            L.alp_hip_mxv(V.h, alp.PLUS_TIMES_F64, alp.DENSE, y.ptr, x.ptr, None)
+        alp.check(L.alp_hip_timer_stop(ctypes.byref(ev)), "timer_stop")
+        v_ms, v_bytes = ev.value / v_steps, format_bytes(n, nnz, vk[0], V.layout(0))
+        v_gbs = v_bytes / (v_ms * 1e-3) / 1e9
+        value_path = {"kernel": KERNEL_NAMES.get(vk[0], str(vk[0])), "launches": v_steps,
+                      "us_per_launch": round(v_ms * 1e3, 2), "bytes_per_launch": v_bytes,
+                      "achieved_gbs": round(v_gbs, 1), "frac": round(v_gbs / HBM_PEAK_GBS, 4)}
+        trv = measured_traffic(*vk)
+        if trv is not None:
+            value_path["traffic"], value_path["traffic_source"] = trv
+        V.free()
+        log(f"[bench] mxv with a value per entry: {value_path['us_per_launch']} us/launch, {v_gbs:.0f} GB/s")
 
     # the CRS kernel any non-stencil matrix gets (CSR-stream), forced on the same matrix
     crs_path = None
@@ -599,8 +642,8 @@ def main() -> int:
         "dtype": "f64",
         "data": "synthetic",
         "config": {"workload": f"{side}^3 27-point stencil (n={n}, nnz={nnz}), FP64 plus-times "
-                               f"grb::mxv y += A x on device-resident storage (CRS and the diagonal-slice copy the kernel streams)",
-                   "kernel": KERNEL_NAMES.get(kernel, str(kernel)), "lanes": lanes, "rows": rows,
+                               f"grb::mxv y += A x on device-resident storage (CRS and the form the kernel streams)",
+                   "kernel": "constant-template" if constant else KERNEL_NAMES.get(kernel, str(kernel)), "lanes": lanes, "rows": rows,
                    "bytes_per_step": fbytes},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
@@ -613,15 +656,16 @@ def main() -> int:
         "crs_equivalent_gbs": round(crs_equiv, 1),
         "crs_equivalent_note": "the metric's CRS bytes (12 nnz + 8 (n+1) + 8 n + 16 n) over the same kernel time; "
                                "not a fraction of peak, since the layout streams no column indices or row offsets",
+        "value_path": value_path,
         "crs_path": crs_path,
         "layout": {"slices": layout[0], "padded_entries": layout[1], "diagonal_slices": layout[2]},
         "build_ms": {"stencil_crs_sell_diagonal_f32": round(build_ms, 1),
-                     "what": "generator, CRS, sliced ELL, diagonal slices and the FP32 copies, on the device"},
+                     "what": "generator, CRS, slices, the template and the FP32 copies, on the device"},
         "mxv_overwrite": {"us_per_launch": round(ow_ms * 1e3, 2), "gbs": round(ow_gbs, 1)},
         "solves": solves,
         "configs": configs,
     }
-    tr = measured_traffic(kernel, lanes, rows)
+    tr = measured_traffic(kernel, lanes, rows, constant)
     if tr is not None:
         out["roofline"]["traffic"] = tr[0]
         out["roofline"]["traffic_source"] = tr[1]

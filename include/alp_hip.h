@@ -148,7 +148,9 @@ alp_rc_t alp_hip_matrix_download(alp_hip_matrix_t A, int which, uint64_t *h_off,
  * one lane per row; `lanes` 0/1 = plain / XCD-contiguous slice order, `rows` 4, 8
  * or 16 entries in flight), 5 = the sliced ELL with its index-free diagonal slices
  * (same arguments). 4 and 5 exist only for matrices with regular rows, 5 only when
- * most slices share one column-offset pattern per slice (stencils). */
+ * most slices share one column-offset pattern per slice (stencils). Where every row
+ * is a subset of one list of (column - row, value) pairs, both run on that list and a
+ * mask per row instead of the slices' values, with the same results. */
 alp_rc_t alp_hip_matrix_set_kernel(alp_hip_matrix_t A, int kernel, int lanes, int rows);
 alp_rc_t alp_hip_matrix_get_kernel(alp_hip_matrix_t A, int *kernel, int *lanes, int *rows);
 /* time each candidate SpMV kernel on this matrix and keep the fastest */
