@@ -87,6 +87,17 @@ inline hipError_t copy_sync(void *dst, const void *src, size_t bytes, hipMemcpyK
 	return e != hipSuccess ? e : hipStreamSynchronize(stream());
 }
 
+// Device memory that its owner can do without: null, with no error left behind, where
+// there is none. ALP_HIP_OPTIONAL_BYTES=n refuses requests of more than n bytes (tests
+// of what runs then).
+void *optional_alloc(size_t bytes);
+// p stays as it is unless it is null; false when it still is
+template <typename T>
+inline bool optional_array(T *&p, size_t bytes) {
+	if (!p) p = static_cast<T *>(optional_alloc(bytes));
+	return p != nullptr;
+}
+
 // number of blocks that fill the chip `per_cu` deep with kBlock-thread blocks
 inline unsigned fill_blocks(int per_cu) {
 	return static_cast<unsigned>(ctx().num_cus > 0 ? ctx().num_cus * per_cu : 256 * per_cu);
@@ -360,8 +371,8 @@ namespace alp {
 
 alp_rc_t storage_finalize(Storage &S, int value_type, bool want_f32);
 alp_rc_t storage_refresh_values(Storage &S, int value_type);
-// gives an FP64 storage its FP32 value copy (and the sliced-ELL / diagonal-slice
-// copies of it) when it has none yet
+// gives an FP64 storage its FP32 value copy, and the layouts that hold values theirs,
+// when it has none yet; what the storage already holds stays as it is
 alp_rc_t storage_ensure_f32(Storage &S, size_t nnz);
 void storage_free(Storage &S);
 alp_rc_t build_ccs_from_crs(alp_hip_matrix_s *A);

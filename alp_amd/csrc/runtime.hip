@@ -64,6 +64,17 @@ alp_rc_t wait_report(double *h, unsigned long long seq, int count) {
 	return ALP_SUCCESS;
 }
 
+void *optional_alloc(size_t bytes) {
+	const char *e = std::getenv("ALP_HIP_OPTIONAL_BYTES");
+	void *p = nullptr;
+	if (e && bytes > std::strtoull(e, nullptr, 10)) return nullptr;
+	if (hipMalloc(&p, bytes ? bytes : 1) != hipSuccess) {
+		(void)hipGetLastError();
+		return nullptr;
+	}
+	return p;
+}
+
 // ---------------------------------------------------------------------------
 // kernels: fills, conversions, BLAS1
 // ---------------------------------------------------------------------------
@@ -343,7 +354,7 @@ __global__ __launch_bounds__(kBlock) void k_sell_fill(size_t nrows, size_t nslic
 		for (uint64_t q = 0; q < w; ++q) {
 			const uint64_t e = e0 + q * kSellRows + lane;
 			const bool in = q < len;
-			sidx[e] = in ? idx[b + q] : 0u;
+			if (sidx) sidx[e] = in ? idx[b + q] : 0u;
 			if (sval) sval[e] = in ? val[b + q] : V(0);
 			if (sval32) sval32[e] = in ? val32[b + q] : 0.0f;
 		}
@@ -497,17 +508,17 @@ alp_rc_t dia_detect(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *
 }
 
 // value arrays of D (val, and val32 when the matrix has an FP32 copy), allocated
-// where missing, then filled; without memory D is dropped
+// where missing, then filled; without memory for val D is dropped, without memory for
+// val32 FP32 products use the CRS kernels
 static alp_rc_t dia_values(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
                            size_t entries, const uint64_t *off, int value_type, const void *val, const float *val32) {
 	if (!D.flag) return ALP_SUCCESS;
 	const size_t vs = value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
-	if ((vs && !D.val && hipMalloc(&D.val, vs * entries) != hipSuccess) ||
-	    (val32 && !D.val32 && hipMalloc(&D.val32, sizeof(float) * entries) != hipSuccess)) {
-		(void)hipGetLastError();
+	if (vs && !optional_array(D.val, vs * entries)) {
 		dia_free(D);
 		return ALP_SUCCESS;
 	}
+	if (val32) optional_array(D.val32, sizeof(float) * entries);
 	const alp_rc_t rc = dia_refresh(D, nslices, nrows, srow, soff, off, value_type, val, val32);
 	if (rc != ALP_SUCCESS) dia_free(D);
 	return rc;
@@ -708,6 +719,25 @@ __global__ __launch_bounds__(kBlock) void k_run_fill(size_t nrows, size_t padded
 	});
 }
 
+// values of a template without them, padded to whole blocks of kRunRows rows
+static size_t run_entries(const Storage &S) {
+	return (S.nmajor + kRunRows - 1) / kRunRows * kRunRows * kDiaFullWidth;
+}
+
+static alp_rc_t run_fill(const Storage &S, int value_type, void *rval, float *rval32) {
+	const size_t padded = run_entries(S) / kDiaFullWidth;
+	if (value_type == ALP_VAL_F64)
+		hipLaunchKernelGGL(k_run_fill<double>, dim3(stream_grid(padded)), dim3(kBlock), 0, stream(), S.nmajor, padded,
+		                   (const uint64_t *)S.off, (const uint32_t *)S.cmask, (const double *)S.val,
+		                   (const float *)S.val32, (double *)rval, rval32);
+	else
+		hipLaunchKernelGGL(k_run_fill<float>, dim3(stream_grid(padded)), dim3(kBlock), 0, stream(), S.nmajor, padded,
+		                   (const uint64_t *)S.off, (const uint32_t *)S.cmask, (const float *)S.val,
+		                   (const float *)S.val32, (float *)rval, rval32);
+	ALP_LAUNCH_CHECK();
+	return ALP_SUCCESS;
+}
+
 static bool keep_sell() {
 	const char *keep = std::getenv("ALP_HIP_KEEP_SELL");  // "1": keep them (tests of the sliced-ELL path)
 	return keep && keep[0] == '1';
@@ -730,51 +760,33 @@ static alp_rc_t storage_const(Storage &S, int value_type) {
 	S.cst = ConstDia();
 	if (S.max_len == 0 || S.max_len > kDiaSlots || value_type == ALP_VAL_PATTERN || !const_dia_enabled()) return ALP_SUCCESS;
 	const size_t ns = (S.nmajor + kSellRows - 1) / kSellRows;
-	if (!S.cmask && hipMalloc(&S.cmask, sizeof(uint32_t) * ns * kSellRows) != hipSuccess) {
-		(void)hipGetLastError();
-		S.cmask = nullptr;
-		return ALP_SUCCESS;
-	}
+	if (!optional_array(S.cmask, sizeof(uint32_t) * ns * kSellRows)) return ALP_SUCCESS;
 	const alp_rc_t rc = const_detect(S.cst, 0, S.nmajor, 0, ns, nullptr, S.off, S.idx, value_type, S.val, S.cmask, true);
 	if (rc != ALP_SUCCESS || !S.cst.w) {
 		const_free(S);
 		return rc;
 	}
 	if (S.cst.uniform) return ALP_SUCCESS;
-	const size_t padded = (S.nmajor + kRunRows - 1) / kRunRows * kRunRows;
 	const size_t vs = value_type == ALP_VAL_F64 ? 8 : 4;
-	if ((!S.rval && hipMalloc(&S.rval, vs * kDiaFullWidth * padded) != hipSuccess) ||
-	    (S.val32 && !S.rval32 && hipMalloc(&S.rval32, sizeof(float) * kDiaFullWidth * padded) != hipSuccess)) {
-		(void)hipGetLastError();
+	if (!optional_array(S.rval, vs * run_entries(S))) {
 		const_free(S);
 		return ALP_SUCCESS;
 	}
-	if (value_type == ALP_VAL_F64)
-		hipLaunchKernelGGL(k_run_fill<double>, dim3(stream_grid(padded)), dim3(kBlock), 0, stream(), S.nmajor, padded,
-		                   (const uint64_t *)S.off, (const uint32_t *)S.cmask, (const double *)S.val,
-		                   (const float *)S.val32, (double *)S.rval, S.rval32);
-	else
-		hipLaunchKernelGGL(k_run_fill<float>, dim3(stream_grid(padded)), dim3(kBlock), 0, stream(), S.nmajor, padded,
-		                   (const uint64_t *)S.off, (const uint32_t *)S.cmask, (const float *)S.val,
-		                   (const float *)S.val32, (float *)S.rval, S.rval32);
-	ALP_LAUNCH_CHECK();
-	return ALP_SUCCESS;
+	if (S.val32) optional_array(S.rval32, sizeof(float) * run_entries(S));
+	return run_fill(S, value_type, S.rval, S.rval32);
 }
 
-// S's sliced-ELL arrays (those it has) from the CRS
-static alp_rc_t sell_fill(Storage &S, int value_type) {
-	if (!S.sell_idx) return ALP_SUCCESS;  // diagonal slices only
+// S's sliced-ELL arrays (those given) from the CRS
+static alp_rc_t sell_fill(const Storage &S, int value_type, uint32_t *sidx, void *sval, float *sval32) {
 	const unsigned g = stream_grid(S.n_slices * kSellRows);
 	if (value_type == ALP_VAL_F32)
 		hipLaunchKernelGGL(k_sell_fill<float>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, S.n_slices,
 		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const float *)S.val,
-		                   (const float *)S.val32, (const uint64_t *)S.sell_off, S.sell_idx, (float *)S.sell_val,
-		                   S.sell_val32);
+		                   (const float *)S.val32, (const uint64_t *)S.sell_off, sidx, (float *)sval, sval32);
 	else
 		hipLaunchKernelGGL(k_sell_fill<double>, dim3(g), dim3(kBlock), 0, stream(), S.nmajor, S.n_slices,
 		                   (const uint64_t *)S.off, (const uint32_t *)S.idx, (const double *)S.val,
-		                   (const float *)S.val32, (const uint64_t *)S.sell_off, S.sell_idx, (double *)S.sell_val,
-		                   S.sell_val32);
+		                   (const float *)S.val32, (const uint64_t *)S.sell_off, sidx, (double *)sval, sval32);
 	ALP_LAUNCH_CHECK();
 	return ALP_SUCCESS;
 }
@@ -828,14 +840,11 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 		uint32_t *sidx = nullptr;
 		void *sval = nullptr;
 		float *sval32 = nullptr;
-		if (hipMalloc(&sidx, sizeof(uint32_t) * total) != hipSuccess ||
-		    (vs && hipMalloc(&sval, vs * total) != hipSuccess) ||
-		    (values && S.val32 && hipMalloc(&sval32, sizeof(float) * total) != hipSuccess)) {
+		if (!optional_array(sidx, sizeof(uint32_t) * total) || (vs && !optional_array(sval, vs * total)) ||
+		    (values && S.val32 && !optional_array(sval32, sizeof(float) * total))) {
 			// not enough memory for the copy: keep the CRS kernels only
-			(void)hipGetLastError();
 			if (sidx) hipFree(sidx);
 			if (sval) hipFree(sval);
-			if (sval32) hipFree(sval32);
 			hipFree(soff);
 			dia_free(dia);
 			const_free(S);
@@ -849,7 +858,7 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 	S.n_slices = ns;
 	S.sell_entries = total;
 	S.dia = dia;
-	ALP_TRY(sell_fill(S, value_type));
+	if (S.sell_idx) ALP_TRY(sell_fill(S, value_type, S.sell_idx, S.sell_val, S.sell_val32));
 	if (S.cst.w) return ALP_SUCCESS;
 	return dia_values(S.dia, ns, S.nmajor, nullptr, S.sell_off, total, S.off, value_type, S.val, S.val32);
 }
@@ -862,16 +871,11 @@ alp_rc_t storage_refresh_values(Storage &S, int value_type) {
 	ALP_TRY(storage_const(S, value_type));
 	if (!S.cst.w && S.sell_idx) {
 		const size_t vs = value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
-		if (vs && !S.sell_val && hipMalloc(&S.sell_val, vs * S.sell_entries) != hipSuccess) {
-			(void)hipGetLastError();
-			S.sell_val = nullptr;  // the products then use the CRS kernels
-		}
-		if (S.val32 && !S.sell_val32 && hipMalloc(&S.sell_val32, sizeof(float) * S.sell_entries) != hipSuccess) {
-			(void)hipGetLastError();
-			S.sell_val32 = nullptr;
-		}
+		// without them the products use the CRS kernels
+		if (vs) optional_array(S.sell_val, vs * S.sell_entries);
+		if (S.val32) optional_array(S.sell_val32, sizeof(float) * S.sell_entries);
 	}
-	ALP_TRY(sell_fill(S, value_type));
+	if (S.sell_idx) ALP_TRY(sell_fill(S, value_type, S.sell_idx, S.sell_val, S.sell_val32));
 	if (S.cst.w) return ALP_SUCCESS;
 	return dia_values(S.dia, S.n_slices, S.nmajor, nullptr, S.sell_off, S.sell_entries, S.off, value_type, S.val,
 	                  S.val32);
@@ -885,8 +889,20 @@ alp_rc_t storage_ensure_f32(Storage &S, size_t nnz) {
 		hipLaunchKernelGGL((k_convert<double, float>), dim3(stream_grid(nnz)), dim3(kBlock), 0, stream(), nnz,
 		                   (const double *)S.val, S.val32);
 	ALP_LAUNCH_CHECK();
-	if (S.cst.uniform) return ALP_SUCCESS;  // the template holds both precisions
-	return storage_refresh_values(S, ALP_VAL_F64);
+	// Products and captured solver iterations already run on the layouts that are
+	// there: those keep their arrays, and each gets its FP32 values beside them (a
+	// uniform template holds both precisions). Where there is no memory for these, FP32
+	// products use the CRS kernels.
+	if (S.rval && optional_array(S.rval32, sizeof(float) * run_entries(S)))
+		ALP_TRY(run_fill(S, ALP_VAL_F64, nullptr, S.rval32));
+	if (S.sell_val && optional_array(S.sell_val32, sizeof(float) * S.sell_entries))
+		ALP_TRY(sell_fill(S, ALP_VAL_F64, nullptr, nullptr, S.sell_val32));
+	if (S.dia.val && optional_array(S.dia.val32, sizeof(float) * S.sell_entries)) {
+		DiaSlices d = S.dia;
+		d.val = nullptr;
+		ALP_TRY(dia_refresh(d, S.n_slices, S.nmajor, nullptr, S.sell_off, S.off, ALP_VAL_F64, S.val, S.val32));
+	}
+	return ALP_SUCCESS;
 }
 
 alp_rc_t storage_finalize(Storage &S, int value_type, bool want_f32) {
@@ -1347,9 +1363,8 @@ size_t storage_bytes(const Storage &S, int value_type, size_t nnz) {
 	if (S.sell_val32) b += sizeof(float) * S.sell_entries;
 	if (S.dia.flag) b += S.n_slices + sizeof(int32_t) * kDiaSlots * S.n_slices + sizeof(uint32_t) * S.n_slices * kSellRows;
 	if (S.cmask) b += sizeof(uint32_t) * S.n_slices * kSellRows;
-	const size_t padded = (S.nmajor + kRunRows - 1) / kRunRows * kRunRows;
-	if (S.rval) b += vs * kDiaFullWidth * padded;
-	if (S.rval32) b += sizeof(float) * kDiaFullWidth * padded;
+	if (S.rval) b += vs * run_entries(S);
+	if (S.rval32) b += sizeof(float) * run_entries(S);
 	if (S.dia.val) b += vs * S.sell_entries;
 	if (S.dia.val32) b += sizeof(float) * S.sell_entries;
 	b += S.n_long * 4 + (S.n_long + 1) * 8 + S.n_chunks * (4 + 8 + 8);

@@ -1,0 +1,92 @@
+"""Memory that layouts and solvers can do without, refused (ALP_HIP_OPTIONAL_BYTES): what
+already runs keeps its arrays and its captured iterations, and every call still
+gives its result."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def A():
+    import alp_amd
+    alp_amd.init(0)
+    return alp_amd
+
+
+def spd(n, offsets, rng, shuffle=False):
+    """A symmetric diagonally dominant matrix with entries at the offsets (of both signs),
+    the columns of a row in a random order with shuffle (no diagonal form then)."""
+    off, idx, val = [0], [], []
+    weight = {d: rng.uniform(0.1, 1.0, n) for d in offsets if d > 0}
+    for r in range(n):
+        row = [(r + d, -(weight[d][r] if d > 0 else weight[-d][r + d])) for d in offsets if d and 0 <= r + d < n]
+        row.append((r, 1.0 - sum(v for _, v in row)))
+        if shuffle:
+            rng.shuffle(row)
+        idx += [int(c) for c, _ in row]
+        val += [float(v) for _, v in row]
+        off.append(len(idx))
+    return np.array(off, np.uint64), np.array(idx, np.uint32), np.array(val)
+
+
+def make(A, kind, rng):
+    if kind == "runs":  # 27 points, a value per entry
+        s = 12
+        return A.Matrix.conductance27(s, s, s, A.Vector.from_numpy(rng.uniform(0.5, 2.0, 13 * s ** 3)), 1.0)
+    if kind == "constant":
+        return A.Matrix.stencil27(12, 12, 12)
+    n = 2000
+    off, idx, val = spd(n, [-40, -1, 1, 40], rng, kind == "sliced")
+    return A.Matrix.from_crs(n, n, off, idx, val)
+
+
+KINDS = ["runs", "diagonal", "sliced", "constant"]
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_fp32_copy_refused_between_two_solves(A, kind, monkeypatch):
+    """An FP64 solve, a mixed solve that gets no memory for the layout's FP32 values, and
+    the FP64 solve again on its captured iterations: the same bits, and the layout holds
+    what it held (beside the FP32 copy of the CRS values)."""
+    rng = np.random.default_rng(1)
+    M = make(A, kind, rng)
+    b, x = A.Vector.from_numpy(rng.standard_normal(M.nrows)), A.Vector(M.nrows)
+
+    def solve(precision, tol, limit):
+        x.set(0.0)
+        return A.cg(M, b, x, limit, tol, precision)[0], x.numpy()
+
+    first = solve(0, 1e-300, 20)[1]
+    held, layout, kernel = M.device_bytes(), M.layout(), M.get_kernel()
+    monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
+    mixed = [solve(p, 1e-10, 1000) for p in (1, 3)]
+    monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES")
+    assert M.device_bytes() == held + 4 * M.nnz
+    assert (M.layout(), M.get_kernel()) == (layout, kernel)
+    assert np.array_equal(solve(0, 1e-300, 20)[1], first)
+    rc, want = solve(0, 1e-12, 1000)
+    assert rc == A.SUCCESS
+    # residuals below 1e-10 of b on matrices of condition number below 1e3
+    for rc, got in mixed:
+        assert rc == A.SUCCESS
+        assert np.linalg.norm(got - want) <= 1e-7 * np.linalg.norm(want)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_layouts_refused_at_build(A, kind, monkeypatch):
+    """With no memory for any layout the products run on the CRS."""
+    full = make(A, kind, np.random.default_rng(2))
+    monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
+    bare = make(A, kind, np.random.default_rng(2))
+    monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES")
+    assert bare.device_bytes() < full.device_bytes()
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal(full.nrows)
+    got = []
+    for M in (full, bare):
+        y = A.Vector(M.nrows, fill=0.0)
+        assert A.mxv(y, M, A.Vector.from_numpy(x)) == A.SUCCESS
+        got.append(y.numpy())
+    # two orders of at most 27 products
+    assert np.max(np.abs(got[0] - got[1])) <= 28 * 2.0 ** -53 * 60 * np.max(np.abs(x))
