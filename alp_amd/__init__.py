@@ -42,6 +42,7 @@ OVERWRITE = 1 << 20
 
 VAL_F64, VAL_F32, VAL_PATTERN = 0, 1, 2
 MTX_PATTERN, MTX_SYMMETRIC = 1, 2
+FORM_CRS, FORM_SLICED, FORM_DIAGONAL, FORM_RUNS, FORM_CONSTANT = range(5)
 MAT_WITH_CCS, MAT_WITH_F32 = 1, 2
 GRAPH_SYMMETRIZE, GRAPH_DROP_SELF_LOOPS = 1, 2
 
@@ -99,6 +100,8 @@ SIGNATURES = {
                                ctypes.POINTER(_S), _P, _P, _P, ctypes.POINTER(_I)]),
     "alp_hip_matrix_read_mtx": (_RC, [ctypes.POINTER(_P), ctypes.c_char_p, _I, _U]),
     "alp_hip_matrix_layout": (_RC, [_P, _I, ctypes.POINTER(_S), ctypes.POINTER(_S), ctypes.POINTER(_S)]),
+    "alp_hip_matrix_form": (_RC, [_P, _I, ctypes.POINTER(_I)]),
+    "alp_hip_hpcg_constant_levels": (_RC, [_P, ctypes.POINTER(_S)]),
     "alp_hip_get_stream": (_RC, [ctypes.POINTER(_P)]),
     "alp_hip_matrix_storage": (_RC, [_P, _I, ctypes.POINTER(_P), ctypes.POINTER(_P), ctypes.POINTER(_P)]),
     "alp_hip_matrix_device_bytes": (_RC, [_P, ctypes.POINTER(_S)]),
@@ -363,6 +366,12 @@ class Matrix:
               "matrix_layout")
         return a.value, b.value, c.value
 
+    def form(self, which: int = 0) -> int:
+        """What an unmasked product streams: one of the FORM_* values."""
+        f = _I()
+        check(lib().alp_hip_matrix_form(self.h, which, ctypes.byref(f)), "matrix_form")
+        return f.value
+
     def device_bytes(self) -> int:
         """Device memory the matrix holds (CRS, CCS and every derived layout)."""
         b = _S()
@@ -460,6 +469,11 @@ class Hpcg:
         check(lib().alp_hip_hpcg_info(self.h, ctypes.byref(n), ctypes.byref(nnz), ctypes.byref(lv),
                                       ctypes.byref(pr)), "hpcg_info")
         self.n, self.nnz, self.levels, self.proper = n.value, nnz.value, lv.value, bool(pr.value)
+
+    def constant_levels(self) -> int:
+        n = _S()
+        check(lib().alp_hip_hpcg_constant_levels(self.h, ctypes.byref(n)), "hpcg_constant_levels")
+        return n.value
 
     def vcycle(self, r: Vector, z: Vector) -> None:
         check(lib().alp_hip_hpcg_vcycle(self.h, r.ptr, z.ptr), "hpcg_vcycle")

@@ -1903,6 +1903,13 @@ ALP_EXPORT alp_rc_t alp_hip_hpcg_create(alp_hip_hpcg_t *out, size_t nx, size_t n
 	return ALP_SUCCESS;
 }
 
+ALP_EXPORT alp_rc_t alp_hip_hpcg_constant_levels(alp_hip_hpcg_t H, size_t *levels) {
+	if (!H || !levels) return ALP_ILLEGAL;
+	*levels = 0;
+	for (const HpLevel &L : H->L) *levels += L.cst.empty() ? 0 : 1;
+	return ALP_SUCCESS;
+}
+
 ALP_EXPORT alp_rc_t alp_hip_hpcg_info(alp_hip_hpcg_t H, size_t *n, size_t *nnz, size_t *levels,
                                       int *proper) {
 	if (!H || H->L.empty()) return ALP_ILLEGAL;

@@ -1680,6 +1680,23 @@ ALP_EXPORT alp_rc_t alp_hip_matrix_layout(alp_hip_matrix_t A, int which, size_t 
 	return ALP_SUCCESS;
 }
 
+// as dispatch chooses for the storage's own values without a mask
+static int product_form(const Storage &S) {
+	const int k = S.kernel ? S.kernel : auto_kernel(S);
+	if (k != 4 && k != 5) return 0;
+	if (S.val && S.cst.w && (k == 5 || !S.sell_val)) return S.cst.uniform ? 4 : 3;
+	const void *v = nullptr;
+	const bool slices_only = S.sell_off && !S.sell_idx;
+	if ((k == 5 || slices_only) && dia_values(S, S.val, &v)) return 2;
+	return !slices_only && sell_values(S, S.val, &v) ? 1 : 0;
+}
+
+ALP_EXPORT alp_rc_t alp_hip_matrix_form(alp_hip_matrix_t A, int which, int *form) {
+	if (!A || !form || (which != 0 && which != 1)) return ALP_ILLEGAL;
+	*form = product_form(which == 0 ? A->crs : A->ccs);
+	return ALP_SUCCESS;
+}
+
 // Autotuner: times each candidate on this matrix's CRS with its natural semiring
 // (3 warm-up + 10 timed runs each, hipEvents on the library stream) and keeps
 // the fastest. Candidates: CSR-vector with G = 2..64 lanes per row and 1, 2 or 4

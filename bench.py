@@ -57,12 +57,8 @@ def spmv_bytes(n: int, nnz: int, accumulate: bool = True) -> int:
     return 12 * nnz + 8 * (n + 1) + 8 * n + (16 if accumulate else 8) * n
 
 
-def constant_form(kernel: int) -> bool:
-    """Whether the stencil's launches read its one (offset, value) template instead of
-    a value per entry (they do unless the build is told to keep the values, or kernel
-    4 to keep its sliced-ELL arrays)."""
-    return os.environ.get("ALP_HIP_CONST_DIA", "1")[:1] != "0" and (
-        kernel == 5 or kernel == 4 and os.environ.get("ALP_HIP_KEEP_SELL", "0")[:1] != "1")
+def kernel_name(kernel: int, form: int) -> str:
+    return {3: "offset-template", 4: "constant-template"}.get(form) or KERNEL_NAMES.get(kernel, str(kernel))
 
 
 def format_bytes(n: int, nnz: int, kernel: int, layout, accumulate: bool = True, constant: bool = False) -> int:
@@ -443,7 +439,7 @@ def main() -> int:
     else:
         kernel, lanes, rows = A.get_kernel()
     layout = A.layout(0)
-    log(f"[bench] n={n} nnz={nnz} kernel={KERNEL_NAMES.get(kernel, kernel)} lanes={lanes} rows={rows}")
+    log(f"[bench] n={n} nnz={nnz} kernel={kernel_name(kernel, A.form())} lanes={lanes} rows={rows}")
     x = alp.Vector.from_numpy(np.random.default_rng(0).random(n))
     y = alp.Vector(n, fill=0.0)
 
@@ -472,7 +468,7 @@ def main() -> int:
                   "max": round(single[-1], 2), "launches": 20, "unit": "us",
                   "note": "each launch between its own HIP events, after the timed region"}
     crs_bytes = spmv_bytes(n, nnz)
-    constant = constant_form(kernel)
+    constant = A.form() == alp.FORM_CONSTANT
     fbytes = format_bytes(n, nnz, kernel, layout, constant=constant)
     achieved = fbytes / (kern_ms * 1e-3) / 1e9
     crs_equiv = crs_bytes / (kern_ms * 1e-3) / 1e9
@@ -497,7 +493,7 @@ def main() -> int:
         alp.check(L.alp_hip_timer_stop(ctypes.byref(ev)), "timer_stop")
         v_ms, v_bytes = ev.value / v_steps, format_bytes(n, nnz, vk[0], V.layout(0))
         v_gbs = v_bytes / (v_ms * 1e-3) / 1e9
-        value_path = {"kernel": KERNEL_NAMES.get(vk[0], str(vk[0])), "launches": v_steps,
+        value_path = {"kernel": kernel_name(vk[0], V.form()), "launches": v_steps,
                       "us_per_launch": round(v_ms * 1e3, 2), "bytes_per_launch": v_bytes,
                       "achieved_gbs": round(v_gbs, 1), "frac": round(v_gbs / HBM_PEAK_GBS, 4)}
         trv = measured_traffic(*vk)
@@ -643,7 +639,7 @@ def main() -> int:
         "data": "synthetic",
         "config": {"workload": f"{side}^3 27-point stencil (n={n}, nnz={nnz}), FP64 plus-times "
                                f"grb::mxv y += A x on device-resident storage (CRS and the form the kernel streams)",
-                   "kernel": "constant-template" if constant else KERNEL_NAMES.get(kernel, str(kernel)), "lanes": lanes, "rows": rows,
+                   "kernel": kernel_name(kernel, A.form()), "lanes": lanes, "rows": rows,
                    "bytes_per_step": fbytes},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,

@@ -161,6 +161,11 @@ alp_rc_t alp_hip_matrix_autotune(alp_hip_matrix_t A);
  * reference stores CRS/CCS only; this reports what the kernels stream) */
 alp_rc_t alp_hip_matrix_layout(alp_hip_matrix_t A, int which, size_t *slices, size_t *entries,
                                size_t *dia_slices);
+/* what an unmasked product with A's own values streams under the kernel in use:
+ * 0 the CRS (which = 1: CCS); 1 the sliced ELL; 2 its diagonal slices; 3 a mask per
+ * row and values slot by slot, with one list of column - row offsets for the matrix;
+ * 4 a mask per row, with one list of (column - row, value) pairs */
+alp_rc_t alp_hip_matrix_form(alp_hip_matrix_t A, int which, int *form);
 
 /* ---- device storage, for callers that run kernels of their own on it ----
  * (the grb:: header layer instantiates its generic semiring kernels this way) */
@@ -308,6 +313,8 @@ alp_rc_t alp_hip_hpcg_destroy(alp_hip_hpcg_t H);
 /* n, nnz of the finest level, number of grids (finest included), and whether every
  * level's colouring is proper (then colour steps run fused) */
 alp_rc_t alp_hip_hpcg_info(alp_hip_hpcg_t H, size_t *n, size_t *nnz, size_t *levels, int *proper);
+/* the levels whose steps read a mask per row and one (offset, value) list per colour */
+alp_rc_t alp_hip_hpcg_constant_levels(alp_hip_hpcg_t H, size_t *levels);
 /* z = M r: one V-cycle of the preconditioner (FP64, original row numbering) */
 alp_rc_t alp_hip_hpcg_vcycle(alp_hip_hpcg_t H, const double *d_r, double *d_z);
 /* Solve A x = b from the given x: stop when ||r||/||r0|| <= tol or after max_iter

@@ -45,17 +45,22 @@ def products(A, M, x, y0, ring, mask):
     return out
 
 
-# widths around the compile-time ones (7 and 27) and the largest; rows around a slice,
-# wider and narrower than long, with NaN and infinities at entries of x
+# widths around the compile-time ones (7 and 27) and the largest; one slice, a last
+# slice of one (short) row, of 31 rows and of one full row; wider and narrower than
+# long, with NaN and infinities at entries of x
 @pytest.mark.parametrize("w", [1, 2, 6, 7, 8, 9, 26, 27, 28, 32])
-@pytest.mark.parametrize("n,m", [(64, 64), (65, 130), (1000, 1000), (3001, 2950)])
+@pytest.mark.parametrize("n,m", [(64, 64), (129, 400), (223, 215), (257, 1000), (1000, 1000), (3001, 2950)])
 def test_const_products_equal_kept_values(A, w, n, m, monkeypatch):
     rng = np.random.default_rng(1000 * w + n)
-    offs = rng.permutation(rng.choice(np.arange(-45, 46), size=w, replace=False))
+    reach = min(45, max((w + 1) // 2, n // 16))
+    offs = rng.permutation(rng.choice(np.arange(-reach, reach + 1), size=w, replace=False))
     vals = rng.standard_normal(w)
-    drop = rng.random(n * w) < 0.1
-    drop[np.arange(n // 2) * w + rng.integers(0, w, n // 2)] = False
-    off, idx, val = banded(n, m, offs, vals, drop if n > 64 else None)
+    drop = rng.random((n, w)) < (0.0 if n == 64 else 0.02 if n < 1000 else 0.1)
+    drop[n // 2] = False  # a row with the whole list
+    if n == 129:
+        drop[-1] = True
+        drop[-1, rng.integers(0, w)] = False
+    off, idx, val = banded(n, m, offs, vals, drop.ravel())
     x, y0 = rng.standard_normal(m), rng.standard_normal(n)
     if n == 1000:
         x[17], x[400], x[999] = np.nan, np.inf, -np.inf
@@ -68,8 +73,8 @@ def test_const_products_equal_kept_values(A, w, n, m, monkeypatch):
                                (F, P, A.PLUS_PATTERN_F64, x, y0)):
         # kernel 4 folds each row in storage order whatever the default is
         for k in (c, p):
-            if k.layout()[0]:
-                k.set_kernel(4)
+            k.set_kernel(4)
+        assert c.form() == A.FORM_CONSTANT and p.form() in (A.FORM_SLICED, A.FORM_DIAGONAL)
         for a, b in zip(products(A, c, xv, yv, ring, mask), products(A, p, xv, yv, ring, mask)):
             assert np.array_equal(a, b, equal_nan=True), (w, n, ring)
 
@@ -79,6 +84,7 @@ def test_const_stencil_takes_the_form(A, sides, monkeypatch):
     """27-point stencils, also where slices straddle lines and planes, hold fewer bytes
     than with values; products are the same bits through mxv and the transposed vxm."""
     C, P = both(A, monkeypatch, lambda: A.Matrix.stencil27(*sides, flags=A.MAT_WITH_CCS | A.MAT_WITH_F32))
+    assert C.form(0) == C.form(1) == (A.FORM_CRS if sides == (4, 4, 4) else A.FORM_CONSTANT)  # padding of 4^3: 1.7
     if P.layout()[0]:
         assert C.device_bytes() < P.device_bytes()
         P.set_kernel(4)
@@ -122,6 +128,7 @@ def test_run_values_equal_kept_values(A, sides, flip, monkeypatch):
         for k in (c, p):
             if k.layout()[0]:
                 k.set_kernel(4)
+        assert c.form() == (A.FORM_CRS if sides == (4, 4, 4) else A.FORM_RUNS)
         for a, b in zip(products(A, c, xv, yv, ring, mask), products(A, p, xv, yv, ring, mask)):
             assert np.array_equal(a, b, equal_nan=True), ring
     # the FP32 copy made by a mixed solve instead of at build time
@@ -155,6 +162,7 @@ def test_const_near_misses_keep_their_values(A, monkeypatch):
 
     for k in range(3):
         C, P = both(A, monkeypatch, lambda: variant(k))
+        assert C.form() == P.form() != A.FORM_CONSTANT
         assert C.device_bytes() == P.device_bytes(), k
         got = []
         for M in (C, P):
@@ -165,17 +173,19 @@ def test_const_near_misses_keep_their_values(A, monkeypatch):
         assert np.array_equal(got[0], got[1]), k
 
 
-@pytest.mark.parametrize("sizes,levels,pre,post", [((16, 16, 16), 2, 1, 1), ((24, 16, 40), 1, 2, 2), ((12, 20, 28), 1, 1, 1),
-                                                  ((32, 16, 16), 2, 0, 1), ((16, 32, 16), 2, 1, 0), ((8, 12, 10), 0, 1, 1),
-                                                  # a coarsest level of one workgroup's most rows, and of more
-                                                  ((16, 16, 28), 0, 1, 1), ((16, 18, 26), 0, 1, 1),
-                                                  ((4, 4, 4), 1, 1, 1),
-                                                  ((9, 11, 7), 0, 1, 1)])
-def test_const_hpcg_equals_kept_values(A, sizes, levels, pre, post, monkeypatch):
+@pytest.mark.parametrize("sizes,levels,pre,post,const", [
+    ((16, 16, 16), 2, 1, 1, 3), ((24, 16, 40), 1, 2, 2, 2), ((12, 20, 28), 1, 1, 1, 2),
+    ((32, 16, 16), 2, 0, 1, 3), ((16, 32, 16), 2, 1, 0, 3), ((8, 12, 10), 0, 1, 1, 1),
+    # a coarsest level of one workgroup's most rows, and of more
+    ((16, 16, 28), 0, 1, 1, 1), ((16, 18, 26), 0, 1, 1, 1),
+    ((4, 4, 4), 1, 1, 1, 1),  # 2^3 has no inner row
+    ((9, 11, 7), 0, 1, 1, 0)])
+def test_const_hpcg_equals_kept_values(A, sizes, levels, pre, post, const, monkeypatch):
     """V-cycle and solves on levels in constant form (whose steps on one colour, and
     transfers, run in one launch) equal the sliced layouts' bit for bit; odd sides
     (whose colours do not share offsets) keep those layouts."""
     C, P = both(A, monkeypatch, lambda: A.Hpcg(*sizes, max_levels=levels, colours=0, presmooth=pre, postsmooth=post))
+    assert (C.constant_levels(), P.constant_levels()) == (const, 0)
     rng = np.random.default_rng(11)
     r = A.Vector.from_numpy(rng.standard_normal(C.n))
     z = [A.Vector(C.n, fill=0.0) for _ in range(2)]

@@ -51,6 +51,7 @@ def test_fp32_copy_refused_between_two_solves(A, kind, monkeypatch):
     what it held (beside the FP32 copy of the CRS values)."""
     rng = np.random.default_rng(1)
     M = make(A, kind, rng)
+    assert M.form() == getattr(A, "FORM_" + kind.upper())
     b, x = A.Vector.from_numpy(rng.standard_normal(M.nrows)), A.Vector(M.nrows)
 
     def solve(precision, tol, limit):
@@ -58,12 +59,12 @@ def test_fp32_copy_refused_between_two_solves(A, kind, monkeypatch):
         return A.cg(M, b, x, limit, tol, precision)[0], x.numpy()
 
     first = solve(0, 1e-300, 20)[1]
-    held, layout, kernel = M.device_bytes(), M.layout(), M.get_kernel()
+    held, form = M.device_bytes(), (M.form(), M.layout(), M.get_kernel())
     monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
     mixed = [solve(p, 1e-10, 1000) for p in (1, 3)]
     monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES")
     assert M.device_bytes() == held + 4 * M.nnz
-    assert (M.layout(), M.get_kernel()) == (layout, kernel)
+    assert (M.form(), M.layout(), M.get_kernel()) == form
     assert np.array_equal(solve(0, 1e-300, 20)[1], first)
     rc, want = solve(0, 1e-12, 1000)
     assert rc == A.SUCCESS
@@ -80,7 +81,7 @@ def test_layouts_refused_at_build(A, kind, monkeypatch):
     monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
     bare = make(A, kind, np.random.default_rng(2))
     monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES")
-    assert bare.device_bytes() < full.device_bytes()
+    assert bare.form() == A.FORM_CRS and bare.device_bytes() < full.device_bytes()
     rng = np.random.default_rng(3)
     x = rng.standard_normal(full.nrows)
     got = []
