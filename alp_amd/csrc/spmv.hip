@@ -646,14 +646,14 @@ __global__ __launch_bounds__(kBlock) void k_spmv_const(size_t nrows, size_t ncol
 	}
 }
 
-// The product with several rows per lane (const_run_fold): RPL * 64 rows per wavefront.
+// The product with N rows per lane (const_run_fold): N * 64 rows per wavefront.
 // 192^3, y += A x in FP64: 93 -> 47 us (4.2 TB/s of its mask, x and y), FP32 y = A x
 // 33 -> 29 us, where the four operations per entry and row bind; staging x in LDS
 // windows instead took 83 and 62 us. VALUES: the rows' values are streamed 16 bytes per
 // lane from run_pos; against the diagonal slices' loads of one row per lane
 // (k_spmv_sell), FP64 accumulate at 64^3, 101x75x61, 128^3: 11.4, 22.4, 92.6 -> 9.3, 17.9,
 // 84 us; FP32 overwrite 7.5, 11.1, 45.9 -> 7.4, 10.3, 40.7 us (5.4 TB/s at 128^3).
-template <typename R, int MASK, bool OVERWRITE, int DIR, bool VALUES>
+template <typename R, int MASK, bool OVERWRITE, int DIR, bool VALUES, unsigned N>
 __global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols, ConstArg<typename R::V> T,
                                                      const typename R::V *__restrict__ rval,
                                                      const uint32_t *__restrict__ cmask,
@@ -662,7 +662,6 @@ __global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols
                                                      const uint8_t *__restrict__ mask, const int *__restrict__ skip) {
 	using A = typename R::A;
 	using Y = typename R::Y;
-	constexpr unsigned N = RowsPerLane<R>::N;
 	const unsigned bl = xcd_logical_block(blockIdx.x, gridDim.x);
 	const size_t r0 =
 	    (size_t)__builtin_amdgcn_readfirstlane(bl * (kBlock / kWave) + threadIdx.x / kWave) * (kSellRows * N);
@@ -686,7 +685,7 @@ __global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols
 	}
 	if (stop) return;  // a solver loop that has stopped
 	A acc[N];
-	const_run_fold<R, DIR, VALUES>(T, rval, (long long)r0, lane, bits, (long long)ncols, x, acc);
+	const_run_fold<R, DIR, VALUES, N>(T, rval, (long long)r0, lane, bits, (long long)ncols, x, acc);
 #pragma unroll
 	for (unsigned i = 0; i < N; ++i) {
 		if (OVERWRITE) yv[i] = bits[i] == 0 ? static_cast<Y>(R::zero()) : static_cast<Y>(acc[i]);
@@ -705,7 +704,7 @@ __global__ __launch_bounds__(kBlock) void k_const_run(size_t nrows, size_t ncols
 }
 
 // and with the partials of y.x (overwrite): wavefronts take several groups of rows
-template <typename R, int DIR, bool VALUES>
+template <typename R, int DIR, bool VALUES, unsigned N>
 __global__ __launch_bounds__(kBlock) void k_const_run_dot(size_t nrows, ConstArg<typename R::V> T,
                                                          const typename R::V *__restrict__ rval,
                                                          const uint32_t *__restrict__ cmask,
@@ -716,7 +715,6 @@ __global__ __launch_bounds__(kBlock) void k_const_run_dot(size_t nrows, ConstArg
 	using A = typename R::A;
 	using X = typename R::X;
 	using Y = typename R::Y;
-	constexpr unsigned N = RowsPerLane<R>::N;
 	constexpr size_t kRows = (size_t)kBlock * N;
 	const int stop = skip ? *skip : 0;
 	const unsigned lane = threadIdx.x % kWave;
@@ -742,7 +740,7 @@ __global__ __launch_bounds__(kBlock) void k_const_run_dot(size_t nrows, ConstArg
 		}
 		if (stop) return;  // uniform over the grid: no wavefront reaches the reduction
 		A acc[N];
-		const_run_fold<R, DIR, VALUES>(T, rval, (long long)r0, lane, bits, (long long)nrows, x, acc);
+		const_run_fold<R, DIR, VALUES, N>(T, rval, (long long)r0, lane, bits, (long long)nrows, x, acc);
 		Y yv[N];
 #pragma unroll
 		for (unsigned i = 0; i < N; ++i) {
@@ -1287,17 +1285,26 @@ static bool const_arg(const Storage &S, const void *val, ConstArg<typename R::V>
 	return true;
 }
 
-template <typename R, int MASK, bool OW, bool VALUES>
-static void launch_runs(const Storage &S, const ConstArg<typename R::V> &T, const void *rval, const void *x, void *y,
-                        const uint8_t *mask, hipStream_t s, const int *skip) {
-	const size_t rows = (size_t)kBlock * RowsPerLane<R>::N;
+template <typename R, int MASK, bool OW, bool VALUES, unsigned N>
+static void launch_runs_n(const Storage &S, const ConstArg<typename R::V> &T, const void *rval, const void *x, void *y,
+                          const uint8_t *mask, hipStream_t s, const int *skip) {
+	const size_t rows = (size_t)kBlock * N;
 #define ALP_CRUN(DD)                                                                                            \
-	hipLaunchKernelGGL((k_const_run<R, MASK, OW, DD, VALUES>), dim3((S.nmajor + rows - 1) / rows), dim3(kBlock), 0, \
-	                   s, S.nmajor, S.nminor, T, (const typename R::V *)rval, (const uint32_t *)S.cmask,            \
+	hipLaunchKernelGGL((k_const_run<R, MASK, OW, DD, VALUES, N>), dim3((S.nmajor + rows - 1) / rows), dim3(kBlock), \
+	                   0, s, S.nmajor, S.nminor, T, (const typename R::V *)rval, (const uint32_t *)S.cmask,         \
 	                   (const typename R::X *)x, (typename R::Y *)y, mask, skip)
 	if (S.cst.run > 0) ALP_CRUN(1);
 	else ALP_CRUN(-1);
 #undef ALP_CRUN
+}
+
+template <typename R, int MASK, bool OW, bool VALUES>
+static void launch_runs(const Storage &S, const ConstArg<typename R::V> &T, const void *rval, const void *x, void *y,
+                        const uint8_t *mask, hipStream_t s, const int *skip) {
+	if (S.nmajor < RowsPerLane<R>::kFewRows)
+		launch_runs_n<R, MASK, OW, VALUES, 1>(S, T, rval, x, y, mask, s, skip);
+	else
+		launch_runs_n<R, MASK, OW, VALUES, RowsPerLane<R>::N>(S, T, rval, x, y, mask, s, skip);
 }
 
 template <typename R, int MASK, bool OW>
@@ -1306,7 +1313,7 @@ static void launch_const(int xcd, const Storage &S, const ConstArg<typename R::V
 	const size_t per = kBlock / kSellRows;
 	const size_t grid = (S.n_slices + per - 1) / per;
 	if (grid == 0) return;
-	if (S.cst.run) {  // no slower than a row per lane at any size measured (16^3 to 192^3)
+	if (S.cst.run) {
 		launch_runs<R, MASK, OW, false>(S, T, nullptr, x, y, mask, s, skip);
 		return;
 	}
@@ -1454,6 +1461,30 @@ static void dispatch(const Storage &S, const void *val, unsigned descr, void *y,
 #undef ALP_GO
 }
 
+template <typename R, bool VALUES, unsigned N>
+static unsigned launch_run_dot_n(const Storage &S, const ConstArg<typename R::V> &T, const void *rval, const void *x,
+                                 void *y, double *partials, unsigned max_partials, const int *skip, hipStream_t s) {
+	const size_t rows = (size_t)kBlock * N;
+	const unsigned grid = (unsigned)std::min<size_t>((S.nmajor + rows - 1) / rows,
+	                                                 std::min<size_t>(max_partials, fill_blocks(8)));
+#define ALP_RDOT(DD)                                                                                           \
+	hipLaunchKernelGGL((k_const_run_dot<R, DD, VALUES, N>), dim3(grid), dim3(kBlock), 0, s, S.nmajor, T,       \
+	                   (const typename R::V *)rval, (const uint32_t *)S.cmask, (const typename R::X *)x,       \
+	                   (typename R::Y *)y, partials, skip)
+	if (S.cst.run > 0) ALP_RDOT(1);
+	else ALP_RDOT(-1);
+#undef ALP_RDOT
+	return grid;
+}
+
+template <typename R, bool VALUES>
+static void launch_run_dot(const Storage &S, const ConstArg<typename R::V> &T, const void *rval, const void *x, void *y,
+                           double *partials, unsigned max_partials, unsigned *nparts, const int *skip, hipStream_t s) {
+	*nparts = S.nmajor < RowsPerLane<R>::kFewRows
+	              ? launch_run_dot_n<R, VALUES, 1>(S, T, rval, x, y, partials, max_partials, skip, s)
+	              : launch_run_dot_n<R, VALUES, RowsPerLane<R>::N>(S, T, rval, x, y, partials, max_partials, skip, s);
+}
+
 template <typename R>
 static bool sell_dot_launch(const Storage &S, const void *val, const void *x, void *y, double *partials,
                             unsigned max_partials, unsigned *nparts, const int *skip, hipStream_t s) {
@@ -1465,17 +1496,8 @@ static bool sell_dot_launch(const Storage &S, const void *val, const void *x, vo
 		const size_t nb = (S.n_slices + kBlock / kSellRows - 1) / (kBlock / kSellRows);
 		const unsigned grid = (unsigned)std::min<size_t>(nb, std::min<size_t>(max_partials, fill_blocks(8)));
 		if (grid == 0) return false;
-		if (S.cst.run) {  // no slower than a row per lane at any size measured (16^3 to 192^3)
-			const size_t rows = (size_t)kBlock * RowsPerLane<RC>::N;
-			const unsigned gr = (unsigned)std::min<size_t>((S.nmajor + rows - 1) / rows,
-			                                               std::min<size_t>(max_partials, fill_blocks(8)));
-#define ALP_CRDOT(DD)                                                                                       \
-	hipLaunchKernelGGL((k_const_run_dot<RC, DD, false>), dim3(gr), dim3(kBlock), 0, s, S.nmajor, carg,         \
-	                   (const typename RC::V *)nullptr, (const uint32_t *)S.cmask, (const typename R::X *)x, (typename R::Y *)y, partials, skip)
-			if (S.cst.run > 0) ALP_CRDOT(1);
-			else ALP_CRDOT(-1);
-#undef ALP_CRDOT
-			*nparts = gr;
+		if (S.cst.run) {
+			launch_run_dot<RC, false>(S, carg, nullptr, x, y, partials, max_partials, nparts, skip, s);
 			return true;
 		}
 #define ALP_CDOT(WW)                                                                                         \
@@ -1492,16 +1514,8 @@ static bool sell_dot_launch(const Storage &S, const void *val, const void *x, vo
 	if ((k == 5 || !S.sell_val) && const_arg<R, false>(S, val, rarg)) {
 		const size_t rows = (size_t)kBlock * RowsPerLane<R>::N, nb = (S.nmajor + rows - 1) / rows;
 		if (nb > max_partials) return false;  // as below: larger matrices keep the separate dot
-		const unsigned gr = (unsigned)std::min<size_t>(nb, std::min<size_t>(max_partials, fill_blocks(8)));
-		const void *rv = val == S.val ? S.rval : (const void *)S.rval32;
-#define ALP_RDOT(DD)                                                                                        \
-	hipLaunchKernelGGL((k_const_run_dot<R, DD, true>), dim3(gr), dim3(kBlock), 0, s, S.nmajor, rarg,           \
-	                   (const typename R::V *)rv, (const uint32_t *)S.cmask, (const typename R::X *)x,          \
-	                   (typename R::Y *)y, partials, skip)
-		if (S.cst.run > 0) ALP_RDOT(1);
-		else ALP_RDOT(-1);
-#undef ALP_RDOT
-		*nparts = gr;
+		launch_run_dot<R, true>(S, rarg, val == S.val ? S.rval : (const void *)S.rval32, x, y, partials, max_partials,
+		                        nparts, skip, s);
 		return true;
 	}
 	const void *sval = nullptr, *dval = nullptr;

@@ -273,14 +273,25 @@ __device__ __forceinline__ typename R::A const_fold(const ConstArg<typename R::V
 }
 
 // Several rows per lane for templates that are nine runs of three consecutive
-// offsets (ConstDia::run; the 27-point stencil's order): a lane owns RPL = 16 /
-// sizeof(x) consecutive rows, whose slots of one run lie in RPL + 2 consecutive
+// offsets (ConstDia::run; the 27-point stencil's order): a lane owns N = 16 /
+// sizeof(x) consecutive rows, whose slots of one run lie in N + 2 consecutive
 // elements of x, read by one 16-byte load and one of the rest; so are its values. A wavefront's reads
 // then move 1.5 to 2 elements per row and run through L1 instead of 3, in a third
 // (FP64) or a sixth (FP32) of the load instructions. Each row's fold keeps its order.
+//
+// On few rows N = 1: the wide form then leaves most of the card's 256 CUs idle or with
+// one wavefront per SIMD. Its line (kFewRows) by the sums' type, where 1 and N rows per
+// lane take the same time; products with a value per entry, then constant ones:
+//   FP64 sums, with the dot, us per CG iteration of FP64 data: 32^3 16.8 against 17.2,
+//   40^3 17.9 and 18.3, 48^3 21.1 and 20.1 (16.3 and 16.4, 16.6 and 16.9, 18.4 and 17.9);
+//   of FP32 data: 32^3 18.2 and 20.4, 48^3 21.2 and 22.1, 56^3 23.7 and 23.5 (24.0 and
+//   25.5, 22.9 and 23.4, 25.0 and 24.4)
+//   FP32 sums, us per product: 32^3 5.9 and 7.6, 64^3 7.9 and 8.8, 80^3 12.2 and 11.7,
+//   100^3 21.2 and 20.6 (5.6 and 7.2, 5.8 and 6.6, 6.4 and 7.1, 9.0 and 8.1)
 template <typename R>
 struct RowsPerLane {
 	static constexpr unsigned N = 16 / sizeof(typename R::X);
+	static constexpr size_t kFewRows = sizeof(typename R::A) == 8 ? size_t(3) << 15 : size_t(1) << 19;
 };
 
 // n consecutive elements, whatever their alignment (global loads need only 4 bytes)
@@ -310,18 +321,16 @@ __device__ __forceinline__ void store_run(X *p, const X *in) {
 	*reinterpret_cast<V *>(p) = v;
 }
 
-// rows r0 + lane * RPL + i, i < RPL (r0 uniform), with masks bits[i]; DIR = the sign of
+// rows r0 + lane * N + i, i < N (r0 uniform), with masks bits[i]; DIR = the sign of
 // the runs. With VALUES the rows' values come from rval (run_pos), streamed once, not
 // from the template.
-template <typename R, int DIR, bool VALUES>
+template <typename R, int DIR, bool VALUES, unsigned N>
 __device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T,
                                                const typename R::V *__restrict__ rval, long long r0, unsigned lane,
-                                               const uint32_t (&bits)[RowsPerLane<R>::N], long long ncols,
-                                               const typename R::X *__restrict__ x,
-                                               typename R::A (&acc)[RowsPerLane<R>::N]) {
-	using A = typename R::A;
+                                               const uint32_t (&bits)[N], long long ncols,
+                                               const typename R::X *__restrict__ x, typename R::A (&acc)[N]) {
 	using X = typename R::X;
-	constexpr unsigned N = RowsPerLane<R>::N, kGroup = 3;  // runs in flight
+	constexpr unsigned kGroup = 3;  // runs in flight
 	constexpr uint32_t full = (1u << kDiaFullWidth) - 1u;
 	const bool inside = r0 + T.dmin >= 0 && r0 + (long long)(kSellRows * N) - 1 + T.dmax < ncols;
 	bool some = false;

@@ -141,6 +141,61 @@ def test_run_values_equal_kept_values(A, sides, flip, monkeypatch):
         assert np.array_equal(a, b)
 
 
+# both sides of the lines between one row per lane and several (98304 rows with FP64
+# sums, 524288 with FP32 ones), wider and narrower than long
+@pytest.mark.parametrize("n,m,f32", [(257, 300, False), (98303, 98290, False), (98305, 98400, False),
+                                     (524287, 524280, True), (524291, 524400, True)])
+@pytest.mark.parametrize("uniform", [True, False])
+def test_runs_at_each_row_count_per_lane(A, n, m, f32, uniform, monkeypatch):
+    """Nine runs of three offsets, constant and with a value per entry, on non-square
+    matrices: the bits of the kept values, also with NaN and infinities in x where a row
+    lacks the neighbour."""
+    rng = np.random.default_rng(n + uniform)
+    up = (n + m) % 2 == 0
+    base = np.array([-21, -17, -8, -4, 0, 4, 9, 13, 20])
+    offs = (base[:, None] + np.arange(-1, 2)[None, :]).ravel()
+    offs = offs if up else offs[::-1]
+    drop = rng.random((n, 27)) < 0.02
+    drop[n // 2] = False
+    off, idx, val = banded(n, m, offs, rng.standard_normal(27), drop.ravel())
+    if not uniform:
+        val = rng.standard_normal(val.size)
+    dt = np.float32 if f32 else np.float64
+    x, y0 = rng.standard_normal(m).astype(dt), rng.standard_normal(n).astype(dt)
+    x[rng.integers(0, m, 3)] = [np.nan, np.inf, -np.inf]
+    x[0], x[m - 1] = np.nan, np.inf
+    mask = (rng.random(n) < 0.5).astype(np.uint8)
+    C, P = both(A, monkeypatch, lambda: A.Matrix.from_crs(n, m, off, idx, val.astype(dt)))
+    C.set_kernel(4)
+    P.set_kernel(4)
+    assert C.form() == (A.FORM_CONSTANT if uniform else A.FORM_RUNS) and P.form() != C.form()
+    ring = A.PLUS_TIMES_F32 if f32 else A.PLUS_TIMES_F64
+    for a, b in zip(products(A, C, x, y0, ring, mask), products(A, P, x, y0, ring, mask)):
+        assert np.array_equal(a, b, equal_nan=True)
+
+
+@pytest.mark.parametrize("sides", [(46, 46, 46), (48, 46, 46)])
+@pytest.mark.parametrize("constant", [True, False])
+def test_solves_at_each_row_count_per_lane(A, sides, constant, monkeypatch):
+    """The product with its dot on both sides of 98304 rows: five iterations differ from
+    those on kept values by the order of the dot's partial sums alone (a relative 2^-53
+    or, in FP32 directions, 2^-24 per operation on systems of condition number below 1e3)."""
+    n = int(np.prod(sides))
+    rng = np.random.default_rng(n)
+    theta = A.Vector.from_numpy(rng.uniform(0.5, 2.0, 13 * n))
+    build = (lambda: A.Matrix.stencil27(*sides)) if constant else (lambda: A.Matrix.conductance27(*sides, theta, 1.0))
+    C, P = both(A, monkeypatch, build)
+    assert C.form() == (A.FORM_CONSTANT if constant else A.FORM_RUNS) and P.form() == A.FORM_DIAGONAL
+    b = A.Vector.from_numpy(rng.standard_normal(n))
+    for precision, bound in ((0, 1e3 * 2.0 ** -53), (1, 1e3 * 2.0 ** -24), (3, 1e3 * 2.0 ** -24)):
+        got = []
+        for M in (C, P):
+            x = A.Vector(n, fill=0.0)
+            A.cg(M, b, x, 5, 1e-300, precision)
+            got.append(x.numpy())
+        assert np.linalg.norm(got[0] - got[1]) <= bound * np.linalg.norm(got[1])
+
+
 def test_const_near_misses_keep_their_values(A, monkeypatch):
     """One value off by an ulp, one row in another order, one column stored twice: not
     one template, so the bytes held and the results are those without the form."""
