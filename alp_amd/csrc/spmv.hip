@@ -1411,7 +1411,14 @@ static void dispatch(const Storage &S, const void *val, unsigned descr, void *y,
 	int kernel = S.kernel;
 	int G = S.lanes ? S.lanes : default_lanes(S);
 	int RR = S.rows;  // CSR-stream: the launch variant
-	if (kernel == 0) kernel = auto_kernel(S);
+	if (kernel == 0) {
+		kernel = auto_kernel(S);
+		// CSR-vector reads the rows of the mask, a CSR-stream block its whole tile. Against
+		// row segments at 20 random entries per row in FP64, 1.2, 4 and 20 M nonzeros: 1 % of
+		// the rows 6.6, 16 and 67 us against 9.6, 29 and 209; half of them 8.2, 30 and 143
+		// against 10.2, 30 and 213; all but 1 % 9.5, 39 and 231 against 10.3, 30 and 213
+		if (mmode && kernel == 2 && !skewed(S)) kernel = 1;
+	}
 	// the constant form where the matrix has it (kernel 5, or 4 when no sliced-ELL
 	// values are kept: the same fold order); it reads neither indices nor values
 	bool cst = false, runs = false;

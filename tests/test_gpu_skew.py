@@ -82,3 +82,28 @@ def test_default_kernel_of_unstructured_matrices(A, rows, mean, sigma):
     assert A.vxm(z, A.Vector.from_numpy(x), M) == A.SUCCESS
     assert np.array_equal(y.numpy(), 1.0 + np.bincount(row, val * x[idx], minlength=rows))
     assert np.array_equal(z.numpy(), 1.0 + np.bincount(idx, val * x[row], minlength=rows))
+
+
+@pytest.mark.parametrize("sigma", [0.2, 1.4])
+def test_masked_products_read_the_rows_of_the_mask(A, sigma):
+    """Above the nonzero count from which row segments are the default, a masked product
+    on evenly long rows runs on CSR-vector, which reads the mask's rows alone: the bits of
+    that kernel's fold. Skewed rows keep row segments, masked or not."""
+    rng = np.random.default_rng(17)
+    rows = 60011
+    lengths = np.clip(np.round(20 * np.exp(sigma * rng.standard_normal(rows))), 1, 3000).astype(np.int64)
+    off = np.zeros(rows + 1, np.uint64)
+    np.cumsum(lengths, out=off[1:])
+    idx = rng.integers(0, rows, int(off[-1])).astype(np.uint32)
+    M = A.Matrix.from_crs(rows, rows, off, idx, rng.standard_normal(idx.size))
+    x, y0 = A.Vector.from_numpy(rng.standard_normal(rows)), rng.standard_normal(rows)
+    assert M.get_kernel()[::2] == (2, 64)
+    for mask in (None, (rng.random(rows) < 0.02).astype(np.uint8)):
+        got = {}
+        for kernel in ((0, 0, 0), (1, 0, 0), (2, 0, 64)):
+            M.set_kernel(*kernel)
+            y = A.Vector.from_numpy(y0)
+            assert A.mxv(y, M, x, mask=None if mask is None else A.Vector.from_numpy(mask)) == A.SUCCESS
+            got[kernel[0]] = y.numpy()
+        assert not np.array_equal(got[1], got[2])
+        assert np.array_equal(got[0], got[1 if mask is not None and sigma < 1 else 2])
