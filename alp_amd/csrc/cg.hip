@@ -7,8 +7,9 @@
 // round trip; all scalars live in a device state block:
 //   k_cg_spmv_dot  temp = A u and one partial sum of temp.u per block, in one pass
 //                  (CSR-vector matrices; on a sliced layout k_sell_dot does the same)
-//   k_cg_update    every block folds the temp.u partials into alpha = sigma / (temp.u);
-//                  r -= alpha temp and one partial of r.r per block
+//   k_cg_update    every block folds the temp.u partials into alpha = sigma / (temp.u),
+//                  which block 0 keeps for k_cg_dir; r -= alpha temp and one partial of
+//                  r.r per block
 //   k_cg_dir       every block folds r.r, applies the stopping test (||r|| < tol ||b||,
 //                  :378,437) and, unless done, u' = r + (r.r / sigma) u; every fourth
 //                  iteration, and the last, x += alpha u for the directions since
@@ -161,13 +162,17 @@ __device__ __forceinline__ void grid_for_pieces(size_t n, Load &&load, Use &&use
 }
 
 // alpha = sigma / p.Ap (folded from npap partials), r -= alpha temp and the partials
-// of r.r. X: also x += alpha u (the preconditioned loop); otherwise k_cg_dir adds it.
+// of r.r. X: also x += alpha u (the preconditioned loop); otherwise k_cg_dir adds it,
+// with the alpha of direction g that block 0 leaves in the state (folding p.Ap there
+// again in every block cost small systems 0.5 us per iteration).
 template <typename T, bool X>
-__global__ __launch_bounds__(kBlock) void k_cg_update(CgArgs<T> a, const CgScal *in, unsigned npap) {
+__global__ __launch_bounds__(kBlock) void k_cg_update(CgArgs<T> a, const CgScal *in, unsigned npap, int g) {
 	__shared__ double lds[kBlock / kWave];
 	if (in->done) return;
 	const double pAp = fold_partials(a.partials, npap, lds);
-	const T alpha = (T)(in->sigma / pAp);
+	const double alpha64 = in->sigma / pAp;
+	const T alpha = (T)alpha64;
+	if (!X && blockIdx.x == 0 && threadIdx.x == 0) a.st->alpha[g] = alpha64;
 	double part = 0.0;
 	if (X) {
 		grid_for_each<4>(a.n, [&](size_t i) {
@@ -217,8 +222,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CgArgs<T> a, const CgScal 
 // K: the group's size, kDirs or 1 (no room for more directions). XT: the solution's type
 // (double with T = float when CgArgs::x64 is set).
 template <typename T, typename XT, int G, int K>
-__global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in, CgScal *out, unsigned npap,
-                                                  unsigned nrr) {
+__global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in, CgScal *out, unsigned nrr) {
 	__shared__ double lds[kBlock / kWave];
 	if (in->done) {
 		if (blockIdx.x == 0 && threadIdx.x == 0) *out = *in;
@@ -226,9 +230,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in
 	}
 	XT *x;
 	if constexpr (std::is_same<XT, T>::value) x = a.x; else x = a.x64;
-	const double pAp = fold_partials(a.partials, npap, lds);
 	const double rr = fold_partials(a.partials + kHalfPartials, nrr, lds);
-	const double alpha64 = in->sigma / pAp;
 	const unsigned long long iter = in->iter + 1;
 	const bool conv = std::sqrt(rr) < a.st->tol_abs;
 	const bool done = conv || iter >= a.st->max_iter;
@@ -237,8 +239,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in
 	if (done || G == K - 1) {
 		XT alpha[G + 1];
 #pragma unroll
-		for (int g = 0; g < G; ++g) alpha[g] = (XT)a.st->alpha[g];
-		alpha[G] = (XT)alpha64;
+		for (int g = 0; g <= G; ++g) alpha[g] = (XT)a.st->alpha[g];
 		constexpr int U = sizeof(T) == 8 ? 2 : 1;
 		T w[U][G + 1][V], r[U][V];
 		XT xv[U][V];
@@ -293,7 +294,6 @@ __global__ __launch_bounds__(kBlock) void k_cg_dir(CgArgs<T> a, const CgScal *in
 		o.done = done ? 1 : 0;
 		o.converged = conv ? 1 : 0;
 		*out = o;
-		a.st->alpha[G] = alpha64;  // read by the group's later iterations only
 	}
 }
 
@@ -680,9 +680,8 @@ struct CgRunner {
 	CgScal *slot_out(int p) const { return &a.st->s[1 - p]; }
 
 	// the part of an iteration up to the stopping test, reading slot p: temp = A u[g],
-	// the partials of p.Ap (*np_out of them), alpha, r and the partials of r.r; with_x
-	// also x (then g = 0)
-	alp_rc_t step(hipStream_t s, int p, int g, bool with_x, unsigned *np_out = nullptr) {
+	// the partials of p.Ap, alpha, r and the partials of r.r; with_x also x (then g = 0)
+	alp_rc_t step(hipStream_t s, int p, int g, bool with_x) {
 		const CgScal *in = slot_in(p);
 		const T *u = a.u[g];
 		unsigned npap = gvec;
@@ -726,19 +725,17 @@ struct CgRunner {
 			}
 		}
 		if (with_x)
-			hipLaunchKernelGGL((k_cg_update<T, true>), dim3(gvec), dim3(kBlock), 0, s, a, in, npap);
+			hipLaunchKernelGGL((k_cg_update<T, true>), dim3(gvec), dim3(kBlock), 0, s, a, in, npap, g);
 		else
-			hipLaunchKernelGGL((k_cg_update<T, false>), dim3(gvec), dim3(kBlock), 0, s, a, in, npap);
+			hipLaunchKernelGGL((k_cg_update<T, false>), dim3(gvec), dim3(kBlock), 0, s, a, in, npap, g);
 		ALP_LAUNCH_CHECK();
-		if (np_out) *np_out = npap;
 		return ALP_SUCCESS;
 	}
 
 	template <typename XT>
-	void launch_dir(hipStream_t s, int p, int g, unsigned npap) {
+	void launch_dir(hipStream_t s, int p, int g) {
 #define ALP_CG_DIR_K(GG, KK)                                                                                   \
-	hipLaunchKernelGGL((k_cg_dir<T, XT, GG, KK>), dim3(gvec), dim3(kBlock), 0, s, a, slot_in(p), slot_out(p), npap, \
-	                   gvec)
+	hipLaunchKernelGGL((k_cg_dir<T, XT, GG, KK>), dim3(gvec), dim3(kBlock), 0, s, a, slot_in(p), slot_out(p), gvec)
 #define ALP_CG_DIR(GG)               \
 	case GG:                         \
 		ALP_CG_DIR_K(GG, kDirs);     \
@@ -762,11 +759,10 @@ struct CgRunner {
 	// iteration number i of a batch (whole): from slot i % 2 into the other one, with
 	// direction i % a.dirs
 	alp_rc_t iteration(hipStream_t s, int i) {
-		unsigned npap = 0;
 		const int g = i % a.dirs;
-		ALP_TRY(step(s, i % 2, g, false, &npap));
-		if (a.x64) launch_dir<double>(s, i % 2, g, npap);
-		else launch_dir<T>(s, i % 2, g, npap);
+		ALP_TRY(step(s, i % 2, g, false));
+		if (a.x64) launch_dir<double>(s, i % 2, g);
+		else launch_dir<T>(s, i % 2, g);
 		ALP_LAUNCH_CHECK();
 		return ALP_SUCCESS;
 	}
