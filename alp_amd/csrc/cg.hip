@@ -150,13 +150,20 @@ template <int V, int U, typename Load, typename Use, typename Tail>
 __device__ __forceinline__ void grid_for_pieces(size_t n, Load &&load, Use &&use, Tail &&tail) {
 	const size_t np = n / V, stride = (size_t)gridDim.x * kBlock;
 	const size_t t = (size_t)blockIdx.x * kBlock + threadIdx.x;
-	for (size_t i = t; i < np; i += U * stride) {
+	if (np <= stride) {  // one piece per thread: 0.2 us less per CG iteration than the loop's code
+		if (t < np) {
+			load(0, t * V);
+			use(0, t * V);
+		}
+	} else {
+		for (size_t i = t; i < np; i += U * stride) {
 #pragma unroll
-		for (int u = 0; u < U; ++u)
-			if (i + u * stride < np) load(u, (i + u * stride) * V);
+			for (int u = 0; u < U; ++u)
+				if (i + u * stride < np) load(u, (i + u * stride) * V);
 #pragma unroll
-		for (int u = 0; u < U; ++u)
-			if (i + u * stride < np) use(u, (i + u * stride) * V);
+			for (int u = 0; u < U; ++u)
+				if (i + u * stride < np) use(u, (i + u * stride) * V);
+		}
 	}
 	if (t < n - np * V) tail(np * V + t);
 }
