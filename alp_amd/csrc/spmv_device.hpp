@@ -330,7 +330,10 @@ __device__ __forceinline__ void const_run_fold(const ConstArg<typename R::V> &T,
                                                const uint32_t (&bits)[N], long long ncols,
                                                const typename R::X *__restrict__ x, typename R::A (&acc)[N]) {
 	using X = typename R::X;
-	constexpr unsigned kGroup = 3;  // runs in flight
+	// runs in flight; all nine where the registers allow it (us per CG iteration of FP32 data
+	// with one row per lane, three and nine: 25^3 16.5 and 16.1, 40^3 16.6 and 15.9; FP64
+	// data, where nine take 108 registers: 15.3 and 15.4, 16.1 both)
+	constexpr unsigned kGroup = VALUES && N == 1 && sizeof(X) == 4 ? 9 : 3;
 	constexpr uint32_t full = (1u << kDiaFullWidth) - 1u;
 	const bool inside = r0 + T.dmin >= 0 && r0 + (long long)(kSellRows * N) - 1 + T.dmax < ncols;
 	bool some = false;
