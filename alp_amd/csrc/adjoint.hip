@@ -119,18 +119,13 @@ ALP_EXPORT alp_rc_t alp_hip_matrix_conductance27(alp_hip_matrix_t *A, size_t nx,
                                                  const double *d_theta, double shift, unsigned flags) {
 	ALP_TRY(ensure_init());
 	if (!A || !d_theta) return ALP_ILLEGAL;
-	ALP_TRY(alp_hip_matrix_stencil27(A, nx, ny, nz, 0.0, 0.0, flags & ~ALP_MAT_WITH_CCS));
+	ALP_TRY(stencil27_crs(A, nx, ny, nz, 0.0, 0.0, flags));
 	alp_hip_matrix_t M = *A;
 	hipLaunchKernelGGL(k_cond_values, dim3(a_grid(M->nrows)), dim3(kBlock), 0, stream(), nx, ny, nz,
 	                   (const uint64_t *)M->crs.off, (const uint32_t *)M->crs.idx, d_theta, shift,
 	                   (double *)M->crs.val);
-	alp_rc_t rc = ALP_SUCCESS;
-	if (hipGetLastError() != hipSuccess) rc = ALP_PANIC;
-	if (!rc && M->crs.val32) rc = alp_hip_convert_f64_to_f32(M->nnz, (const double *)M->crs.val, M->crs.val32);
-	// the sliced-ELL copy was filled from the pattern's placeholder values
-	if (!rc) rc = storage_refresh_values(M->crs, M->value_type);
-	if (!rc && (flags & ALP_MAT_WITH_CCS)) rc = build_ccs_from_crs(M);
-	if (!rc && hipStreamSynchronize(stream()) != hipSuccess) rc = ALP_PANIC;
+	alp_rc_t rc = hipGetLastError() == hipSuccess ? ALP_SUCCESS : ALP_PANIC;
+	if (!rc) rc = finish_matrix(M);
 	if (rc) {
 		alp_hip_matrix_destroy(M);
 		*A = nullptr;

@@ -236,7 +236,7 @@ alp_rc_t dia_detect(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *
 alp_rc_t dia_build(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
                    size_t entries, const uint64_t *off, const uint32_t *idx, int value_type, const void *val,
                    const float *val32);
-// rewrites D's values from the CRS values (after an in-place value update)
+// fills D's value arrays (those it has) from the CRS values
 alp_rc_t dia_refresh(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *srow, const uint64_t *soff,
                      const uint64_t *off, int value_type, const void *val, const float *val32);
 void dia_free(DiaSlices &D);
@@ -370,13 +370,17 @@ struct alp_hip_matrix_s {
 namespace alp {
 
 alp_rc_t storage_finalize(Storage &S, int value_type, bool want_f32);
-alp_rc_t storage_refresh_values(Storage &S, int value_type);
 // gives an FP64 storage its FP32 value copy, and the layouts that hold values theirs,
 // when it has none yet; what the storage already holds stays as it is
 alp_rc_t storage_ensure_f32(Storage &S, size_t nnz);
 void storage_free(Storage &S);
 alp_rc_t build_ccs_from_crs(alp_hip_matrix_s *A);
 alp_rc_t build_ccs_from_crs(alp_hip_matrix_s *A, uint64_t *src);
+// the CRS of alp_hip_matrix_stencil27, for a caller that writes its values before
+// finish_matrix derives the layouts (and the FP32 copy and CCS of M's flags) from them
+alp_rc_t stencil27_crs(alp_hip_matrix_t *A, size_t nx, size_t ny, size_t nz, double diag, double offdiag,
+                       unsigned flags);
+alp_rc_t finish_matrix(alp_hip_matrix_s *M);
 // a new matrix handle with its sizes set and no storage yet
 alp_rc_t new_matrix(alp_hip_matrix_t *A, size_t nrows, size_t ncols, size_t nnz, int value_type, unsigned flags);
 // bytes of device memory a storage holds (all its layouts)

@@ -1176,7 +1176,8 @@ static ConstArg<T> const_level_arg(const ConstDia &D) {
 // rows have the same diagonal entry. Leaves L.cst empty when they do not.
 static alp_rc_t build_level_const(HpLevel &L) {
 	if (!L.proper || !const_dia_enabled() || L.nslices == 0) return ALP_SUCCESS;
-	ALP_TRY(dmalloc(&L.cmask, L.nslices * kSellRows));
+	// the form is optional (as in the other layouts' builds, where there is no memory)
+	if (!optional_array(L.cmask, sizeof(uint32_t) * L.nslices * kSellRows)) return ALP_SUCCESS;
 	std::vector<ConstDia> cst(L.ncolors);
 	std::vector<ConstArg<double>> tab(L.ncolors);
 	std::vector<ConstArg<float>> tab32(L.ncolors);

@@ -533,7 +533,7 @@ alp_rc_t dia_build(DiaSlices &D, size_t nslices, size_t nrows, const uint32_t *s
 
 // ---- constant form ----------------------------------------------------------------
 
-// *best = min(*best, first row in [row0, row1) with the most entries of that range):
+// *best = max(*best, the key of the first row in [row0, row1) with the most entries):
 // per-block (length, row) maxima, one 64-bit atomic per block (longest first, then
 // the lowest row)
 __global__ __launch_bounds__(kBlock) void k_const_longest(size_t row0, size_t row1, const uint64_t *off,
@@ -577,16 +577,20 @@ __global__ void k_const_template(size_t row0, const uint64_t *off, const uint32_
 	}
 }
 
-// One wavefront per slice: every row matches its (offset, value) pairs greedily
-// against the template's in order. The template's offsets are distinct (one row
-// stores a column once), so a row that is a subsequence is matched completely.
-// *bad is set when some row is not (it counts the slices seen before the rest left).
-template <typename V, bool VALUES>
+// One wavefront per slice: every row matches its offsets greedily against the
+// template's in order. The template's offsets are distinct (one row stores a column
+// once), so a row that is a subsequence is matched completely. bad[0] counts slices
+// with a row that is not, bad[1] those with a matched entry of another value (up to
+// where the rest left: once bad[0], or bad[1] with values_only, is set).
+template <typename V>
 __global__ __launch_bounds__(kBlock) void k_const_match(size_t s0, size_t s1, size_t row1, const uint32_t *srow,
                                                        const uint64_t *off, const uint32_t *idx, const V *val,
-                                                       const ConstTemplate *T, uint32_t *mask, unsigned *bad) {
+                                                       const ConstTemplate *T, uint32_t *mask, unsigned *bad,
+                                                       bool values_only) {
 	const size_t sl = s0 + (size_t)blockIdx.x * (kBlock / kSellRows) + threadIdx.x / kSellRows;
-	if (sl >= s1 || *bad) return;  // whole wavefronts leave together; a slice that failed decides
+	const unsigned w = T->w;
+	// whole wavefronts leave together
+	if (sl >= s1 || w > kDiaSlots || bad[0] || (values_only && bad[1])) return;
 	const unsigned lane = threadIdx.x % kSellRows;
 	size_t r0, r1;
 	dia_rows(sl, row1, srow, &r0, &r1);
@@ -594,24 +598,25 @@ __global__ __launch_bounds__(kBlock) void k_const_match(size_t s0, size_t s1, si
 	const bool act = r < r1;
 	const uint64_t b = act ? off[r] : 0;
 	const uint64_t len = act ? off[r + 1] - b : 0;
-	const unsigned w = T->w;
 	uint32_t bits = 0;
 	unsigned j = 0;
+	bool other = false;
 	for (unsigned q = 0; q < w; ++q) {
 		if (j >= len) break;
 		if ((long long)idx[b + j] - (long long)r != T->d[q]) continue;
 		unsigned long long u = 0;
-		if (VALUES) {
-			const V v = val[b + j];
-			__builtin_memcpy(&u, &v, sizeof(V));
-		}
-		if (!VALUES || u == T->bits[q]) {
-			bits |= 1u << q;
-			++j;
-		}
+		const V v = val[b + j];
+		__builtin_memcpy(&u, &v, sizeof(V));
+		other |= u != T->bits[q];
+		bits |= 1u << q;
+		++j;
 	}
 	mask[sl * kSellRows + lane] = bits;
-	if (__ballot(j != len) != 0 && lane == 0) atomicAdd(bad, 1u);
+	const bool misfit = __ballot(j != len) != 0, differs = __ballot(other) != 0;
+	if (lane == 0) {
+		if (misfit) atomicAdd(bad, 1u);
+		if (differs) atomicAdd(bad + 1, 1u);
+	}
 }
 
 // ALP_HIP_CONST_DIA=0 keeps the diagonal slices' own values (diagnostics, tests)
@@ -626,25 +631,29 @@ static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0,
                                bool offsets_only) {
 	struct Work {
 		unsigned long long best;
-		unsigned bad, pad;
+		unsigned bad[2];
 		ConstTemplate t;
-	} h{}, *d = nullptr;
-	ALP_HIP_TRY(hipMalloc(&d, sizeof(Work)));
+	} h{};
+	Work *d = nullptr;
+	if (!optional_array(d, sizeof(Work))) return ALP_SUCCESS;
 	struct Free {
 		void *p;
 		~Free() { hipFree(p); }
 	} guard{d};
 	hipStream_t s = stream();
+	const unsigned blocks = (unsigned)((s1 - s0 + kBlock / kSellRows - 1) / (kBlock / kSellRows));
 	ALP_HIP_TRY(hipMemsetAsync(d, 0, sizeof(Work), s));
 	hipLaunchKernelGGL(k_const_longest, dim3(stream_grid(row1 - row0)), dim3(kBlock), 0, s, row0, row1, off, &d->best);
 	hipLaunchKernelGGL(k_const_template<V>, dim3(1), dim3(kDiaSlots), 0, s, row0, off, idx, val,
 	                   (const unsigned long long *)&d->best, &d->t);
+	hipLaunchKernelGGL(k_const_match<V>, dim3(blocks), dim3(kBlock), 0, s, s0, s1, row1, srow, off, idx, val,
+	                   (const ConstTemplate *)&d->t, mask, d->bad, !offsets_only);
 	ALP_LAUNCH_CHECK();
 	ALP_HIP_TRY(copy_sync(&h, d, sizeof(Work), hipMemcpyDeviceToHost));
-	if (h.t.w == 0 || h.t.w > kDiaSlots) return ALP_SUCCESS;
+	if (h.t.w == 0 || h.t.w > kDiaSlots || h.bad[0]) return ALP_SUCCESS;
 	ConstDia N;
 	N.w = h.t.w;
-	N.uniform = true;
+	N.uniform = h.bad[1] == 0;
 	N.dmin = INT32_MAX;
 	N.dmax = INT32_MIN;
 	for (unsigned q = 0; q < N.w; ++q) {
@@ -669,23 +678,7 @@ static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0,
 				break;
 			}
 	}
-	const unsigned blocks = (unsigned)((s1 - s0 + kBlock / kSellRows - 1) / (kBlock / kSellRows));
-	for (int values : {1, 0}) {
-		if (values ? !N.uniform : !offsets_only || N.run == 0) continue;
-		if (!values) ALP_HIP_TRY(hipMemsetAsync(&d->bad, 0, sizeof(unsigned), s));
-		if (values)
-			hipLaunchKernelGGL((k_const_match<V, true>), dim3(blocks), dim3(kBlock), 0, s, s0, s1, row1, srow, off, idx,
-			                   val, (const ConstTemplate *)&d->t, mask, &d->bad);
-		else
-			hipLaunchKernelGGL((k_const_match<V, false>), dim3(blocks), dim3(kBlock), 0, s, s0, s1, row1, srow, off, idx,
-			                   val, (const ConstTemplate *)&d->t, mask, &d->bad);
-		ALP_LAUNCH_CHECK();
-		ALP_HIP_TRY(copy_sync(&h.bad, &d->bad, sizeof(unsigned), hipMemcpyDeviceToHost));
-		if (h.bad) continue;
-		N.uniform = values != 0;
-		C = N;
-		break;
-	}
+	if (N.uniform || (offsets_only && N.run != 0)) C = N;
 	return ALP_SUCCESS;
 }
 
@@ -861,24 +854,6 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 	if (S.sell_idx) ALP_TRY(sell_fill(S, value_type, S.sell_idx, S.sell_val, S.sell_val32));
 	if (S.cst.w) return ALP_SUCCESS;
 	return dia_values(S.dia, ns, S.nmajor, nullptr, S.sell_off, total, S.off, value_type, S.val, S.val32);
-}
-
-// Copies S's current CRS values (and FP32 copy) into its sliced layouts, after a
-// caller rewrote the values in place; the index layout is unchanged. Values that
-// leave the constant form get the arrays it did without.
-alp_rc_t storage_refresh_values(Storage &S, int value_type) {
-	if (!S.sell_off || S.n_slices == 0) return ALP_SUCCESS;
-	ALP_TRY(storage_const(S, value_type));
-	if (!S.cst.w && S.sell_idx) {
-		const size_t vs = value_type == ALP_VAL_F64 ? 8 : value_type == ALP_VAL_F32 ? 4 : 0;
-		// without them the products use the CRS kernels
-		if (vs) optional_array(S.sell_val, vs * S.sell_entries);
-		if (S.val32) optional_array(S.sell_val32, sizeof(float) * S.sell_entries);
-	}
-	if (S.sell_idx) ALP_TRY(sell_fill(S, value_type, S.sell_idx, S.sell_val, S.sell_val32));
-	if (S.cst.w) return ALP_SUCCESS;
-	return dia_values(S.dia, S.n_slices, S.nmajor, nullptr, S.sell_off, S.sell_entries, S.off, value_type, S.val,
-	                  S.val32);
 }
 
 alp_rc_t storage_ensure_f32(Storage &S, size_t nnz) {
@@ -1391,12 +1366,16 @@ alp_rc_t new_matrix(alp_hip_matrix_t *A, size_t nrows, size_t ncols, size_t nnz,
 
 }  // namespace alp
 
-static alp_rc_t finish_matrix(alp_hip_matrix_t M) {
+namespace alp {
+
+alp_rc_t finish_matrix(alp_hip_matrix_s *M) {
 	ALP_TRY(storage_finalize(M->crs, M->value_type, (M->flags & ALP_MAT_WITH_F32) != 0));
 	if (M->flags & ALP_MAT_WITH_CCS) ALP_TRY(build_ccs_from_crs(M));
 	ALP_HIP_TRY(hipStreamSynchronize(stream()));
 	return ALP_SUCCESS;
 }
+
+}  // namespace alp
 
 ALP_EXPORT alp_rc_t alp_hip_matrix_destroy(alp_hip_matrix_t A) {
 	if (!A) return ALP_SUCCESS;
@@ -1497,9 +1476,10 @@ ALP_EXPORT alp_rc_t alp_hip_matrix_create_coo(alp_hip_matrix_t *A, size_t nrows,
 	return rc;
 }
 
-ALP_EXPORT alp_rc_t alp_hip_matrix_stencil27(alp_hip_matrix_t *A, size_t nx, size_t ny,
-                                             size_t nz, double diag, double offdiag,
-                                             unsigned flags) {
+namespace alp {
+
+alp_rc_t stencil27_crs(alp_hip_matrix_t *A, size_t nx, size_t ny, size_t nz, double diag, double offdiag,
+                       unsigned flags) {
 	ALP_TRY(ensure_init());
 	// the reference's generator rejects sizes below 2*halo+1 (ndim_matrix_builders.hpp:229-233)
 	if (nx < 3 || ny < 3 || nz < 3) return ALP_ILLEGAL;
@@ -1538,13 +1518,26 @@ ALP_EXPORT alp_rc_t alp_hip_matrix_stencil27(alp_hip_matrix_t *A, size_t nx, siz
 			rc = ALP_PANIC;
 			break;
 		}
-		rc = finish_matrix(M);
 	} while (0);
 	hipStreamSynchronize(stream());
 	if (counts) hipFree(counts);
 	if (tmp) hipFree(tmp);
 	if (rc) {
 		alp_hip_matrix_destroy(M);
+		*A = nullptr;
+	}
+	return rc;
+}
+
+}  // namespace alp
+
+ALP_EXPORT alp_rc_t alp_hip_matrix_stencil27(alp_hip_matrix_t *A, size_t nx, size_t ny,
+                                             size_t nz, double diag, double offdiag,
+                                             unsigned flags) {
+	ALP_TRY(stencil27_crs(A, nx, ny, nz, diag, offdiag, flags));
+	const alp_rc_t rc = finish_matrix(*A);
+	if (rc) {
+		alp_hip_matrix_destroy(*A);
 		*A = nullptr;
 	}
 	return rc;
