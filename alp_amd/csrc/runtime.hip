@@ -746,10 +746,22 @@ static void const_free(Storage &S) {
 	S.cst = ConstDia();
 }
 
+// A template without values streams 27 of them per row whatever the row holds, a slice
+// its longest row's count. The form is faster while that is at most this many times
+// the slices' entries: 27-point rows on the lower part of a 128^3 box and identity rows
+// above, y += A x in FP64 at 1.01, 1.06, 1.11 and 1.41 times 84, 85, 87 and 86 us against
+// the slices' 92, 88, 84 and 71; in FP32 at 1.11, 1.18, 1.24 times 42.7 us against 45.2,
+// 43.4 and 41.3. Slices that are not diagonal stream 4 bytes of index beside each value.
+static double run_fill_limit(int value_type, bool diagonal) {
+	if (value_type == ALP_VAL_F64) return diagonal ? 1.085 : 1.085 * 12 / 8;
+	return diagonal ? 1.2 : 1.2 * 8 / 4;
+}
+
 // Tries one template for all of S's rows, with the values or (in runs) without; then
 // fills the values that a template without them needs. Without memory, or when the
-// rows do not fit, S keeps its other forms.
-static alp_rc_t storage_const(Storage &S, int value_type) {
+// rows do not fit, S keeps its other forms. entries: those of S's slices, diagonal: in
+// that form.
+static alp_rc_t storage_const(Storage &S, int value_type, uint64_t entries, bool diagonal) {
 	S.cst = ConstDia();
 	if (S.max_len == 0 || S.max_len > kDiaSlots || value_type == ALP_VAL_PATTERN || !const_dia_enabled()) return ALP_SUCCESS;
 	const size_t ns = (S.nmajor + kSellRows - 1) / kSellRows;
@@ -760,6 +772,10 @@ static alp_rc_t storage_const(Storage &S, int value_type) {
 		return rc;
 	}
 	if (S.cst.uniform) return ALP_SUCCESS;
+	if ((double)S.nmajor * kDiaFullWidth > run_fill_limit(value_type, diagonal) * (double)entries) {
+		const_free(S);
+		return ALP_SUCCESS;
+	}
 	const size_t vs = value_type == ALP_VAL_F64 ? 8 : 4;
 	if (!optional_array(S.rval, vs * run_entries(S))) {
 		const_free(S);
@@ -817,7 +833,7 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 	}
 	DiaSlices dia;
 	alp_rc_t rc = dia_detect(dia, ns, S.nmajor, nullptr, soff, total, S.off, S.idx);
-	if (rc == ALP_SUCCESS) rc = storage_const(S, value_type);
+	if (rc == ALP_SUCCESS) rc = storage_const(S, value_type, total, dia.flag != nullptr);
 	if (rc != ALP_SUCCESS) {
 		hipFree(soff);
 		dia_free(dia);

@@ -100,8 +100,18 @@ def test_const_stencil_takes_the_form(A, sides, monkeypatch):
         assert np.array_equal(got[0], got[1])
 
 
+def in_runs(n, layout, f32):
+    """Whether rows in runs of three with a value per entry take 27 values each: unless
+    the slices stream much less."""
+    slices, entries, diagonal = layout
+    limit = (1.2 if f32 else 1.085) * (1 if diagonal else 2 if f32 else 1.5)
+    return slices > 0 and 27 * n <= limit * entries
+
+
+# boxes with fills from 1.03 to 1.7; (64, 12, 10) takes the form in FP32 alone
 @pytest.mark.parametrize("flip", [False, True])
-@pytest.mark.parametrize("sides", [(4, 4, 4), (16, 5, 4), (65, 3, 5), (33, 17, 9), (64, 12, 10), (130, 20, 3)])
+@pytest.mark.parametrize("sides", [(4, 4, 4), (65, 3, 5), (33, 17, 13), (64, 12, 10), (130, 20, 3), (16, 16, 16),
+                                   (17, 19, 23), (65, 13, 21)])
 def test_run_values_equal_kept_values(A, sides, flip, monkeypatch):
     """27-point patterns with a value per entry take the template's offsets and keep their
     values slot by slot: the same bits as the sliced ELL's fold in every ring and mask
@@ -128,7 +138,7 @@ def test_run_values_equal_kept_values(A, sides, flip, monkeypatch):
         for k in (c, p):
             if k.layout()[0]:
                 k.set_kernel(4)
-        assert c.form() == (A.FORM_CRS if sides == (4, 4, 4) else A.FORM_RUNS)
+        assert (c.form() == A.FORM_RUNS) == in_runs(n, c.layout(), c is F32)
         for a, b in zip(products(A, c, xv, yv, ring, mask), products(A, p, xv, yv, ring, mask)):
             assert np.array_equal(a, b, equal_nan=True), ring
     # the FP32 copy made by a mixed solve instead of at build time
@@ -194,6 +204,24 @@ def test_solves_at_each_row_count_per_lane(A, sides, constant, monkeypatch):
             A.cg(M, b, x, 5, 1e-300, precision)
             got.append(x.numpy())
         assert np.linalg.norm(got[0] - got[1]) <= bound * np.linalg.norm(got[1])
+
+
+@pytest.mark.parametrize("part,f32,runs", [(1.0, False, True), (0.875, False, False), (0.875, True, True), (0.6, True, False)])
+def test_sparse_domains_keep_their_slices(A, part, f32, runs):
+    """27-point rows in the lower part of a box and identity rows above it: one list of 27
+    offsets fits all, but rows above would stream 27 values for one."""
+    s = 24
+    off, idx, _ = A.Matrix.stencil27(s, s, s).download(0)
+    n = off.size - 1
+    row = np.repeat(np.arange(n), np.diff(off).astype(int))
+    keep = (row < int(part * s) * s * s) | (idx == row)
+    noff = np.zeros(n + 1, np.uint64)
+    np.cumsum(np.bincount(row[keep], minlength=n), out=noff[1:])
+    rng = np.random.default_rng(5)
+    val = rng.standard_normal(int(keep.sum())).astype(np.float32 if f32 else np.float64)
+    M = A.Matrix.from_crs(n, n, noff, idx[keep], val)
+    assert in_runs(n, M.layout(), f32) == runs and M.form() == (A.FORM_RUNS if runs else A.FORM_DIAGONAL)
+    assert M.device_bytes() <= 2.5 * (12 if not f32 else 8) * int(noff[-1]) + 100 * n
 
 
 def test_const_near_misses_keep_their_values(A, monkeypatch):
