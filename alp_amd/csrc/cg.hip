@@ -225,7 +225,7 @@ __global__ __launch_bounds__(kBlock) void k_cg_update(CgArgs<T> a, const CgScal 
 // an update per iteration bit for bit. x costs 16 bytes of traffic per row and
 // iteration otherwise (FP64; the update and direction kernels run at the card's
 // rate): with 4 directions they move 31 instead of 44 bytes per row in mixed
-// precision, 58 instead of 72 in FP64 (dirs_for has the times).
+// precision, 58 instead of 72 in FP64 (dirs_fp64 has the times).
 // K: the group's size, kDirs or 1 (no room for more directions). XT: the solution's type
 // (double with T = float when CgArgs::x64 is set).
 template <typename T, typename XT, int G, int K>
@@ -590,17 +590,18 @@ struct CgSlot {
 	}
 };
 
-// How many directions an iteration's group keeps: kDirs, except where the vectors of
-// an iteration (n rows of `others` bytes for x, r and A u, 4 for the masks of a
-// constant form, and the directions of dir bytes) stay in the 256 MB Infinity Cache
-// with one direction but not with kDirs: the older directions then cost more than x.
-// FP64 at 176^3 and 192^3: 98 and 130 us per iteration with one, 100 and 135 with
-// four; 128^3 and 256^3: 50 and 360 with one, 48 and 336 with four. Mixed precision
-// at 128^3, 192^3, 256^3: 41.6, 102, 228 with one, 39.1, 94.3, 208 with four.
-static int dirs_for(size_t n, size_t others, size_t dir) {
+// How many directions an FP64 iteration's group keeps: kDirs, except where nothing but
+// vectors (n rows of 24 bytes for x, r and A u and 8 for each direction) and the masks of
+// a constant matrix go through the 256 MB Infinity Cache, and they fit with one direction
+// but not with kDirs: the older directions then cost more than x. us per iteration with
+// one and four on constant 27-point matrices: 160^3 78 and 75, 176^3 98 and 99, 192^3 133
+// and 137, 208^3 178 and 178, 256^3 360 and 336. A value stream empties the cache in
+// between anyway: 101^3 64.7 and 63.8, 176^3 309 and 305, 192^3 402 and 400. In FP32 the
+// older directions never cost more: 192^3 101 and 91, 208^3 123 and 114 (constant), 226 and
+// 218 at 192^3 with values.
+static int dirs_fp64(const Storage &S, size_t n) {
 	constexpr size_t kCache = size_t(256) << 20;
-	const size_t one = n * (others + 4 + dir), all = n * (others + 4 + kDirs * dir);
-	return one <= kCache && all > kCache ? 1 : kDirs;
+	return S.cst.uniform && n * (24 + 4 + 8) <= kCache && n * (24 + 4 + 8 * kDirs) > kCache ? 1 : kDirs;
 }
 
 // the buffers of sizes `fixed` and after them `dirs` direction vectors of dir bytes, or
@@ -851,7 +852,7 @@ static alp_rc_t cg_fp64(alp_hip_matrix_t A, Storage &S, const double *b, double 
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, &S == &A->ccs ? kSlotTransposed : kSlotFp64);
 	void *bp[3 + kDirs];
-	int dirs = dirs_for(n, 24, 8);
+	int dirs = dirs_fp64(S, n);
 	ALP_TRY(cg_buffers(slot, {8 * n, 8 * n, sizeof(CgState)}, 8 * n, bp, dirs));
 	double *r = (double *)bp[0], *temp = (double *)bp[1];
 	CgState *st = (CgState *)bp[2];
@@ -876,7 +877,7 @@ static alp_rc_t cg_mixed(alp_hip_matrix_t A, Storage &S, const double *b, double
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, &S == &A->ccs ? kSlotMixedInnerT : kSlotMixedInner);
 	void *bp[8 + kDirs];
-	int dirs = dirs_for(n, 12, 4);
+	int dirs = kDirs;
 	ALP_TRY(cg_buffers(slot, {8 * n, 8 * n, 4 * n, 4 * n, 4 * n, 4 * n, sizeof(CgState), sizeof(IrState)}, 4 * n, bp,
 	                   dirs));
 	double *r64 = (double *)bp[0], *t64 = (double *)bp[1];
@@ -935,7 +936,7 @@ static alp_rc_t cg_reliable(alp_hip_matrix_t A, Storage &S, const double *b, dou
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, &S == &A->ccs ? kSlotReliableT : kSlotReliable);
 	void *bp[5 + kDirs];
-	int dirs = dirs_for(n, x_fp64 ? 16 : 12, 4);
+	int dirs = kDirs;
 	ALP_TRY(cg_buffers(slot, {8 * n, 4 * n, 4 * n, 4 * n, sizeof(CgState)}, 4 * n, bp, dirs));
 	double *t64 = (double *)bp[0];
 	float *r32 = (float *)bp[1], *ap32 = (float *)bp[2], *x32 = (float *)bp[3];
@@ -994,7 +995,7 @@ alp_rc_t cg_native(alp_hip_matrix_s *A, const T *b, T *x, size_t max_iter, doubl
 	hipStream_t s = stream();
 	CgSlot &slot = cg_slot(A, std::is_same<T, float>::value ? kSlotNativeF32 : kSlotNativeF64);
 	void *bp[4 + kDirs];
-	int dirs = pc.fn ? 1 : dirs_for(n, 3 * sizeof(T), sizeof(T));
+	int dirs = pc.fn ? 1 : sizeof(T) == 8 ? dirs_fp64(S, n) : kDirs;
 	ALP_TRY(cg_buffers(slot, {sizeof(T) * n, sizeof(T) * n, sizeof(CgState), sizeof(T) * n}, sizeof(T) * n, bp, dirs));
 	T *r = (T *)bp[0], *temp = (T *)bp[1], *z = (T *)bp[3];
 	CgState *st = (CgState *)bp[2];
