@@ -556,6 +556,10 @@ struct CgSlot {
 	size_t n = 0;
 	std::vector<void *> bufs;
 	std::vector<size_t> sizes;
+	// the directions beside the first one, in one array: asked for once, after the
+	// buffers, for as long as those keep their sizes
+	void *more = nullptr;
+	bool refused = false;
 	hipGraph_t graph = nullptr;
 	hipGraphExec_t exec = nullptr;
 	const void *key[6] = {};
@@ -567,17 +571,23 @@ struct CgSlot {
 		exec = nullptr;
 		graph = nullptr;
 	}
+	void drop_buffers() {
+		for (void *p : bufs) hipFree(p);
+		bufs.clear();
+		sizes.clear();
+		if (more) hipFree(more);
+		more = nullptr;
+		refused = false;
+	}
 	~CgSlot() {
 		drop_graph();
-		for (void *p : bufs) hipFree(p);
+		drop_buffers();
 	}
 	// buffers of the given byte sizes; reallocated (and the graph dropped) when they change
 	alp_rc_t buffers(const std::vector<size_t> &w, void **out) {
 		if (w != sizes) {
 			drop_graph();
-			for (void *p : bufs) hipFree(p);
-			bufs.clear();
-			sizes.clear();
+			drop_buffers();
 			for (size_t b : w) {
 				void *q = nullptr;
 				ALP_HIP_TRY(hipMalloc(&q, b ? b : 1));
@@ -587,6 +597,14 @@ struct CgSlot {
 		}
 		for (size_t i = 0; i < bufs.size(); ++i) out[i] = bufs[i];
 		return ALP_SUCCESS;
+	}
+	// count - 1 more vectors of the given bytes; false where there is no memory for them
+	bool directions(size_t bytes, int count, void **out) {
+		const size_t each = (bytes + 255) / 256 * 256;
+		if (!more && !refused) refused = !optional_array(more, each * (count - 1));
+		if (!more) return false;
+		for (int g = 1; g < count; ++g) out[g - 1] = static_cast<char *>(more) + each * (g - 1);
+		return true;
 	}
 };
 
@@ -605,16 +623,14 @@ static int dirs_fp64(const Storage &S, size_t n) {
 }
 
 // the buffers of sizes `fixed` and after them `dirs` direction vectors of dir bytes, or
-// one where memory does not suffice (dirs then says so); out: all of them in that order
+// one where memory does not suffice (dirs then says so); out: all of them in that order.
+// A refusal is remembered, so that the next solve keeps its buffers and its graph.
 static alp_rc_t cg_buffers(CgSlot &slot, std::initializer_list<size_t> fixed, size_t dir, void **out, int &dirs) {
-	for (;;) {
-		std::vector<size_t> want(fixed);
-		want.insert(want.end(), (size_t)dirs, dir);
-		const alp_rc_t rc = slot.buffers(want, out);
-		if (rc != ALP_OUTOFMEM || dirs == 1) return rc;
-		(void)hipGetLastError();
-		dirs = 1;
-	}
+	std::vector<size_t> want(fixed);
+	want.push_back(dir);
+	ALP_TRY(slot.buffers(want, out));
+	if (dirs > 1 && !slot.directions(dir, dirs, out + want.size())) dirs = 1;
+	return ALP_SUCCESS;
 }
 
 enum CgSlotId {

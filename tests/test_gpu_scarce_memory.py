@@ -30,15 +30,15 @@ def spd(n, offsets, rng, shuffle=False):
     return np.array(off, np.uint64), np.array(idx, np.uint32), np.array(val)
 
 
-def make(A, kind, rng):
+def make(A, kind, rng, flags=0):
     if kind == "runs":  # 27 points, a value per entry
         s = 12
-        return A.Matrix.conductance27(s, s, s, A.Vector.from_numpy(rng.uniform(0.5, 2.0, 13 * s ** 3)), 1.0)
+        return A.Matrix.conductance27(s, s, s, A.Vector.from_numpy(rng.uniform(0.5, 2.0, 13 * s ** 3)), 1.0, flags)
     if kind == "constant":
-        return A.Matrix.stencil27(12, 12, 12)
+        return A.Matrix.stencil27(12, 12, 12, flags=flags)
     n = 2000
     off, idx, val = spd(n, [-40, -1, 1, 40], rng, kind == "sliced")
-    return A.Matrix.from_crs(n, n, off, idx, val)
+    return A.Matrix.from_crs(n, n, off, idx, val, flags=flags)
 
 
 KINDS = ["runs", "diagonal", "sliced", "constant"]
@@ -91,3 +91,74 @@ def test_layouts_refused_at_build(A, kind, monkeypatch):
         got.append(y.numpy())
     # two orders of at most 27 products
     assert np.max(np.abs(got[0] - got[1])) <= 28 * 2.0 ** -53 * 60 * np.max(np.abs(x))
+
+
+def cg_iterates(M, b, k):
+    x, r = np.zeros_like(b), b.copy()
+    p, rz = r.copy(), r @ r
+    out = []
+    for _ in range(k):
+        ap = M @ p
+        alpha = rz / (p @ ap)
+        x = x + alpha * p
+        r = r - alpha * ap
+        rr = r @ r
+        p, rz = r + rr / rz * p, rr
+        out.append(x)
+    return out
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("precision", [0, 1, 3])
+def test_cg_iterates_at_every_slot(A, precision, transpose, monkeypatch):
+    """x after 1 to 9 and 15 to 18 iterations, with four directions between the updates of
+    x and, where those are refused, with one: the same bits, and the iterates of an FP64
+    restatement. Rounding reaches x with a factor below 1e3 (the condition number)."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(4)
+    n = 1999
+    off, idx, val = spd(n, [-40, -7, -1, 1, 7, 40], rng)
+    S = sp.csr_matrix((val, idx.astype(np.int64), off.astype(np.int64)), shape=(n, n))
+    b = rng.standard_normal(n)
+    want = cg_iterates(S.T if transpose else S, b, 18)
+    four, one = (A.Matrix.from_crs(n, n, off, idx, val, flags=A.MAT_WITH_F32 | A.MAT_WITH_CCS) for _ in range(2))
+    rhs = A.Vector.from_numpy(b)
+    bound = 1e3 * 2.0 ** (-53 if precision == 0 else -24)
+    for k in list(range(1, 10)) + [15, 16, 17, 18]:
+        got = []
+        for M in (four, one):
+            if M is one:
+                monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
+            else:
+                monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES", raising=False)
+            x = A.Vector(n, fill=0.0)
+            rc, it, _ = A.cg(M, rhs, x, k, 1e-300, precision, transpose=transpose)
+            assert it == k
+            got.append(x.numpy())
+        assert np.array_equal(got[0], got[1]), k
+        assert np.max(np.abs(got[0] - want[k - 1])) <= bound * np.max(np.abs(want[k - 1])), k
+
+
+@pytest.mark.parametrize("kind", ["runs", "diagonal"])
+@pytest.mark.parametrize("precision", [0, 1, 3])
+def test_one_direction_equals_four(A, kind, precision, monkeypatch):
+    """Whole solves, whose reliable updates restart from whichever direction a segment ended
+    on, and again on the captured iterations after the refusal is over."""
+    four, one = (make(A, kind, np.random.default_rng(6), A.MAT_WITH_F32) for _ in range(2))
+    ends = set()
+    for t in range(7):
+        b = A.Vector.from_numpy(np.random.default_rng(t).standard_normal(four.nrows))
+        got = []
+        for M in (four, one):
+            if M is one and t < 6:
+                monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
+            else:
+                monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES", raising=False)
+            x = A.Vector(M.nrows, fill=0.0)
+            rc, it, res = A.cg(M, b, x, 2000, 10.0 ** -(6 + t % 6), precision)
+            assert rc == A.SUCCESS
+            got.append((it, res, x.numpy()))
+        assert got[0][:2] == got[1][:2]
+        assert np.array_equal(got[0][2], got[1][2])
+        ends.add(got[0][0] % 4)
+    assert len(ends) > 1  # not all on one slot
