@@ -763,8 +763,8 @@ __global__ __launch_bounds__(kBlock) void k_b_beta(int nrhs, const double *part,
 // The next direction, P' = R + beta P (P' = P for an instance that has stopped). X
 // is not read by the iteration, so it takes the steps of the last D directions at
 // once, in the order of the iterations, where slot SLOT is the last one or the
-// system freezes: per entry and iteration 3 + 1 + (D + 1) / D accesses with those
-// of k_b_update in place of 9 (64 systems x 8 right-hand sides, 72 M FP32 entries:
+// system freezes: per entry and iteration 3 accesses here, 3 in k_b_update and
+// (D + 1) / D of X, 7.25 for D = 4 in place of 9 (64 systems x 8 right-hand sides, 72 M FP32 entries:
 // both kernels 537 us before, see the rate above).
 template <typename T, int V, int SLOT>
 __global__ __launch_bounds__(kBlock) void k_b_dir(size_t ntiles, const uint32_t *tile_row0, const uint32_t *tile_row1,
@@ -1300,10 +1300,9 @@ static alp_rc_t batch_const(alp_hip_batch_s *B) {
 			if (b) hipFree(b);
 		}
 	} guard{row0, bad};
-	bool have = hipMalloc(&B->tpl, sizeof(BatchTemplate) * B->nsys) == hipSuccess &&
-	            hipMalloc(&B->cmask, sizeof(uint32_t) * rows) == hipSuccess &&
-	            hipMalloc(&row0, sizeof(uint64_t) * (B->nsys + 1)) == hipSuccess &&
-	            hipMalloc(&bad, sizeof(unsigned)) == hipSuccess;
+	const bool have = optional_array(B->tpl, sizeof(BatchTemplate) * B->nsys) &&
+	                  optional_array(B->cmask, sizeof(uint32_t) * rows) &&
+	                  optional_array(row0, sizeof(uint64_t) * (B->nsys + 1)) && optional_array(bad, sizeof(unsigned));
 	if (have) {
 		ALP_HIP_TRY(copy_sync(row0, B->row0.data(), sizeof(uint64_t) * (B->nsys + 1), hipMemcpyHostToDevice));
 		ALP_HIP_TRY(hipMemsetAsync(bad, 0, sizeof(unsigned), s));
@@ -1315,8 +1314,6 @@ static alp_rc_t batch_const(alp_hip_batch_s *B) {
 		                   (const BatchTemplate *)B->tpl, B->cmask, bad);
 		ALP_LAUNCH_CHECK();
 		ALP_HIP_TRY(copy_sync(&h_bad, bad, sizeof(unsigned), hipMemcpyDeviceToHost));
-	} else {
-		(void)hipGetLastError();  // the refusal is handled here
 	}
 	if (have && !h_bad) {
 		dia_free(B->dia);

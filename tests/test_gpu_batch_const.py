@@ -90,3 +90,20 @@ def test_infinities_reach_only_their_rows(A):  # noqa: F811
         want[130 + r, 2] = 0 in cols
         want[130 + r, 5] = 129 in cols
     assert np.array_equal(bad, want)
+
+
+def test_no_memory_for_the_form(A, monkeypatch):  # noqa: F811
+    """Without memory for the templates and masks a batch keeps its other forms."""
+    rng = np.random.default_rng(9)
+    systems = [banded(300, [-17, -1, 0, 1, 17], rng, 0.1), banded(190, [-3, 0, 3], rng, 0.1)]
+    C = A.Batch.from_crs(systems, 4)
+    monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
+    P = A.Batch.from_crs(systems, 4)
+    monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES")
+    x = A.Vector.from_numpy(rng.standard_normal(C.nrows * 4))
+    got = []
+    for B in (C, P):
+        y = A.Vector(B.nrows * 4)
+        B.spmm(x, y)
+        got.append(y.numpy())
+    assert np.array_equal(got[0], got[1])
