@@ -82,7 +82,7 @@ struct TileLong {
 };
 
 // the rows of the list: product(k) is entry k's product, row r's entries [off[r], off[r + 1])
-template <typename R, int MASK, bool OVERWRITE, typename Product>
+template <typename R, bool OVERWRITE, typename Product>
 __device__ __forceinline__ void fold_long_rows(const TileLong &ll, uint32_t r0, const uint64_t *__restrict__ off,
                                                typename R::Y *__restrict__ y, Product &&product) {
 	using A = typename R::A;
@@ -196,7 +196,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream(
 				}
 			}
 			if (__syncthreads_or(lng ? 1 : 0)) {
-				fold_long_rows<R, MASK, OVERWRITE>(ll, r0, off, y, [&](uint64_t k) { return tile[k - base]; });
+				fold_long_rows<R, OVERWRITE>(ll, r0, off, y, [&](uint64_t k) { return tile[k - base]; });
 				__syncthreads();
 			}
 		} else if (!skip_long) {
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_seg(
 				}
 			}
 			if (__syncthreads_or(lng ? 1 : 0)) {
-				fold_long_rows<R, MASK, OVERWRITE>(ll, r0, off, y, [&](uint64_t k) { return Val<R>::mul(R::kPattern ? VT(0) : sval[R::kPattern ? 0 : (unsigned)(k - base)], x[sidx[(unsigned)(k - base)]]); });
+				fold_long_rows<R, OVERWRITE>(ll, r0, off, y, [&](uint64_t k) { return Val<R>::mul(R::kPattern ? VT(0) : sval[R::kPattern ? 0 : (unsigned)(k - base)], x[sidx[(unsigned)(k - base)]]); });
 				__syncthreads();
 			}
 		} else if (!skip_long) {
@@ -914,7 +914,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream_pipe(
 				}
 			}
 			if (__syncthreads_or(lng ? 1 : 0)) {
-				fold_long_rows<R, MASK, OVERWRITE>(ll, c0, off, y, [&](uint64_t k) { return tile[k - cb]; });
+				fold_long_rows<R, OVERWRITE>(ll, c0, off, y, [&](uint64_t k) { return tile[k - cb]; });
 				__syncthreads();
 			}
 		} else {
@@ -1775,12 +1775,16 @@ ALP_EXPORT alp_rc_t alp_hip_matrix_autotune(alp_hip_matrix_t A) {
 	for (int t : {8, 16})
 		for (int v : {1, 2, 4, 8, 16, 32, 64}) cands.push_back({2, t, v});
 	cands.push_back({3, 0, 0});
-	if (A->crs.sell_idx)
+	for (int k : {4, 5}) {
+		if (!(k == 4 ? A->crs.sell_idx != nullptr : A->crs.dia.flag != nullptr)) continue;
+		// forms of one template ignore the entries in flight, runs of three the slice order
+		// too: one launch each, not six
+		A->crs.kernel = k;
+		const bool one = product_form(A->crs) >= 3;
 		for (int xcd : {0, 1})
-			for (int u : {4, 8, 16}) cands.push_back({4, xcd, u});
-	if (A->crs.dia.flag)
-		for (int xcd : {0, 1})
-			for (int u : {4, 8, 16}) cands.push_back({5, xcd, u});
+			for (int u : {4, 8, 16})
+				if (!one || (u == 8 && (xcd == 1 || !A->crs.cst.run))) cands.push_back({k, xcd, u});
+	}
 	float best = 1e30f;
 	Cand pick = {1, default_lanes(A->crs), 1};
 	for (const Cand &c : cands) {
