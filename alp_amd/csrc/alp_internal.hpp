@@ -284,10 +284,12 @@ struct ConstArg {
 // as in dia_build) and writes the slices' presence masks (indexed by slice and
 // lane) to mask; C.w stays 0 when some row does not fit. With offsets_only, rows that
 // fit in their offsets but not their values give a template that is not uniform,
-// provided it is in runs. Blocking.
+// provided it is in runs. work: kConstWork bytes of device memory (a detection of its
+// own allocation and release cost small matrices more than its kernels). Blocking.
+constexpr size_t kConstWork = 1024;
 alp_rc_t const_detect(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
                       const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask,
-                      bool offsets_only = false);
+                      void *work, bool offsets_only = false);
 bool const_dia_enabled();
 
 struct Storage {

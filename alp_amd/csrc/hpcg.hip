@@ -1190,7 +1190,8 @@ static alp_rc_t build_level_const(HpLevel &L) {
 	}
 	for (int c = 0; c < L.ncolors && ok; ++c) {
 		ALP_TRY(const_detect(cst[c], L.color_off[c], L.color_off[c + 1], L.colour_slice_off[c],
-		                     L.colour_slice_off[c + 1], L.srow, L.off, L.idx, ALP_VAL_F64, L.val, L.cmask));
+		                     L.colour_slice_off[c + 1], L.srow, L.off, L.idx, ALP_VAL_F64, L.val, L.cmask,
+		                     L.soff + L.nslices + 1));
 		ok = cst[c].w == kDiaFullWidth;
 		double v = 0.0;
 		bool self = false;
@@ -1253,7 +1254,7 @@ static alp_rc_t build_level_sell(HpLevel &L) {
 	void *tmp = nullptr;
 	alp_rc_t rc = ALP_SUCCESS;
 	do {
-		if ((rc = dmalloc(&L.srow, ns + 1)) || (rc = dmalloc(&L.soff, ns + 1)) || (rc = dmalloc(&sizes, ns + 1)))
+		if ((rc = dmalloc(&L.srow, ns + 1)) || (rc = dmalloc(&L.soff, ns + 1 + kConstWork / sizeof(uint64_t))) || (rc = dmalloc(&sizes, ns + 1)))
 			break;
 		if (copy_sync(L.srow, srow.data(), 4 * (ns + 1), hipMemcpyHostToDevice) != hipSuccess) {
 			rc = ALP_PANIC;
@@ -1308,7 +1309,7 @@ static alp_rc_t build_level(HpLevel &L, size_t nx, size_t ny, size_t nz, int col
 	L.n = nx * ny * nz;
 	const size_t n = L.n;
 	alp_hip_matrix_t A = nullptr;
-	ALP_TRY(alp_hip_matrix_stencil27(&A, nx, ny, nz, 26.0, -1.0, 0));
+	ALP_TRY(stencil27_crs(&A, nx, ny, nz, 26.0, -1.0, 0));  // its rows are permuted below: no layouts
 	L.nnz = A->nnz;
 	const size_t nnz = L.nnz;
 	L.ncolors = colours == 0 ? 8 : colours;

@@ -628,18 +628,14 @@ bool const_dia_enabled() {
 template <typename V>
 static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
                                const uint64_t *off, const uint32_t *idx, const V *val, uint32_t *mask,
-                               bool offsets_only) {
+                               void *work, bool offsets_only) {
 	struct Work {
 		unsigned long long best;
 		unsigned bad[2];
 		ConstTemplate t;
 	} h{};
-	Work *d = nullptr;
-	if (!optional_array(d, sizeof(Work))) return ALP_SUCCESS;
-	struct Free {
-		void *p;
-		~Free() { hipFree(p); }
-	} guard{d};
+	static_assert(sizeof(Work) <= kConstWork, "the record fits its room");
+	Work *d = static_cast<Work *>(work);
 	hipStream_t s = stream();
 	const unsigned blocks = (unsigned)((s1 - s0 + kBlock / kSellRows - 1) / (kBlock / kSellRows));
 	ALP_HIP_TRY(hipMemsetAsync(d, 0, sizeof(Work), s));
@@ -684,13 +680,14 @@ static alp_rc_t const_detect_t(ConstDia &C, size_t row0, size_t row1, size_t s0,
 
 alp_rc_t const_detect(ConstDia &C, size_t row0, size_t row1, size_t s0, size_t s1, const uint32_t *srow,
                       const uint64_t *off, const uint32_t *idx, int value_type, const void *val, uint32_t *mask,
-                      bool offsets_only) {
+                      void *work, bool offsets_only) {
 	C = ConstDia();
 	if (row1 <= row0 || s1 <= s0 || !val) return ALP_SUCCESS;
 	if (value_type == ALP_VAL_F64)
-		return const_detect_t<double>(C, row0, row1, s0, s1, srow, off, idx, (const double *)val, mask, offsets_only);
+		return const_detect_t<double>(C, row0, row1, s0, s1, srow, off, idx, (const double *)val, mask, work,
+		                              offsets_only);
 	if (value_type == ALP_VAL_F32)
-		return const_detect_t<float>(C, row0, row1, s0, s1, srow, off, idx, (const float *)val, mask, offsets_only);
+		return const_detect_t<float>(C, row0, row1, s0, s1, srow, off, idx, (const float *)val, mask, work, offsets_only);
 	return ALP_SUCCESS;
 }
 
@@ -760,13 +757,14 @@ static double run_fill_limit(int value_type, bool diagonal) {
 // Tries one template for all of S's rows, with the values or (in runs) without; then
 // fills the values that a template without them needs. Without memory, or when the
 // rows do not fit, S keeps its other forms. entries: those of S's slices, diagonal: in
-// that form.
-static alp_rc_t storage_const(Storage &S, int value_type, uint64_t entries, bool diagonal) {
+// that form; work: room for const_detect.
+static alp_rc_t storage_const(Storage &S, int value_type, uint64_t entries, bool diagonal, void *work) {
 	S.cst = ConstDia();
 	if (S.max_len == 0 || S.max_len > kDiaSlots || value_type == ALP_VAL_PATTERN || !const_dia_enabled()) return ALP_SUCCESS;
 	const size_t ns = (S.nmajor + kSellRows - 1) / kSellRows;
 	if (!optional_array(S.cmask, sizeof(uint32_t) * ns * kSellRows)) return ALP_SUCCESS;
-	const alp_rc_t rc = const_detect(S.cst, 0, S.nmajor, 0, ns, nullptr, S.off, S.idx, value_type, S.val, S.cmask, true);
+	const alp_rc_t rc = const_detect(S.cst, 0, S.nmajor, 0, ns, nullptr, S.off, S.idx, value_type, S.val, S.cmask, work,
+	                                 true);
 	if (rc != ALP_SUCCESS || !S.cst.w) {
 		const_free(S);
 		return rc;
@@ -806,7 +804,7 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 	if (S.nmajor == 0 || nnz == 0 || S.max_len > 4096) return ALP_SUCCESS;
 	const size_t ns = (S.nmajor + kSellRows - 1) / kSellRows;
 	uint64_t *soff = nullptr, *sizes = nullptr;
-	ALP_HIP_TRY(hipMalloc(&soff, sizeof(uint64_t) * (ns + 1)));
+	ALP_HIP_TRY(hipMalloc(&soff, sizeof(uint64_t) * (ns + 1) + kConstWork));
 	if (hipMalloc(&sizes, sizeof(uint64_t) * (ns + 1)) != hipSuccess) {
 		hipFree(soff);
 		return ALP_OUTOFMEM;
@@ -833,7 +831,7 @@ static alp_rc_t build_sell(Storage &S, int value_type, uint64_t nnz) {
 	}
 	DiaSlices dia;
 	alp_rc_t rc = dia_detect(dia, ns, S.nmajor, nullptr, soff, total, S.off, S.idx);
-	if (rc == ALP_SUCCESS) rc = storage_const(S, value_type, total, dia.flag != nullptr);
+	if (rc == ALP_SUCCESS) rc = storage_const(S, value_type, total, dia.flag != nullptr, soff + ns + 1);
 	if (rc != ALP_SUCCESS) {
 		hipFree(soff);
 		dia_free(dia);
@@ -1348,7 +1346,7 @@ size_t storage_bytes(const Storage &S, int value_type, size_t nnz) {
 	if (S.row_blocks) b += sizeof(uint32_t) * (S.n_row_blocks + 1) + sizeof(uint64_t) * (S.n_row_blocks + 1);
 	if (S.row_blocks_l) b += sizeof(uint32_t) * (S.n_row_blocks_l + 1) + sizeof(uint64_t) * (S.n_row_blocks_l + 1);
 	if (S.row_blocks_w) b += sizeof(uint32_t) * (S.n_row_blocks_w + 1) + sizeof(uint64_t) * (S.n_row_blocks_w + 1);
-	if (S.sell_off) b += sizeof(uint64_t) * (S.n_slices + 1);
+	if (S.sell_off) b += sizeof(uint64_t) * (S.n_slices + 1) + kConstWork;
 	if (S.sell_idx) b += sizeof(uint32_t) * S.sell_entries;
 	if (S.sell_val) b += vs * S.sell_entries;
 	if (S.sell_val32) b += sizeof(float) * S.sell_entries;
