@@ -138,6 +138,7 @@ SIGNATURES = {
     "alp_hip_batch_create_crs": (_RC, [ctypes.POINTER(_P), _S, _P, _P, _P, _P, _S]),
     "alp_hip_batch_destroy": (_RC, [_P]),
     "alp_hip_batch_info": (_RC, [_P, ctypes.POINTER(_S), ctypes.POINTER(_S), _P]),
+    "alp_hip_batch_constant": (_RC, [_P, ctypes.POINTER(_I)]),
     "alp_hip_batch_layout": (_RC, [_P, ctypes.POINTER(_S), ctypes.POINTER(_S)]),
     "alp_hip_batch_spmm": (_RC, [_P, _P, _P]),
     "alp_hip_batch_autotune": (_RC, [_P, ctypes.POINTER(_I)]),
@@ -610,6 +611,12 @@ class Batch:
         a, b = _S(), _S()
         check(lib().alp_hip_batch_layout(self.h, ctypes.byref(a), ctypes.byref(b)), "batch_layout")
         return a.value, b.value
+
+    def constant(self) -> bool:
+        """Whether every system is in constant form."""
+        c = _I()
+        check(lib().alp_hip_batch_constant(self.h, ctypes.byref(c)), "batch_constant")
+        return bool(c.value)
 
     def autotune(self) -> int:
         w = _I()

@@ -1539,6 +1539,12 @@ ALP_EXPORT alp_rc_t alp_hip_batch_info(alp_hip_batch_t B, size_t *nrows, size_t 
 
 // slices of the diagonal form and how many of them qualified (0 when the form
 // was not built: fewer than half qualified, or ALP_HIP_BATCH_DIA=0)
+ALP_EXPORT alp_rc_t alp_hip_batch_constant(alp_hip_batch_t B, int *constant) {
+	if (!B || !constant) return ALP_ILLEGAL;
+	*constant = B->tpl ? 1 : 0;
+	return ALP_SUCCESS;
+}
+
 ALP_EXPORT alp_rc_t alp_hip_batch_layout(alp_hip_batch_t B, size_t *nslices, size_t *ndiagonal) {
 	if (!B || !nslices || !ndiagonal) return ALP_ILLEGAL;
 	*nslices = B->nslices;

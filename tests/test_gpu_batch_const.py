@@ -11,12 +11,13 @@ pytestmark = pytest.mark.gpu
 
 
 def banded(n, offsets, rng, drop=0.3):
-    """Rows of one template with random entries missing; the diagonal stays."""
+    """Rows of one template with random entries missing; the diagonal stays, and the middle
+    row has the whole template."""
     off, idx, val = [0], [], []
     values = rng.uniform(0.1, 1.0, len(offsets)) * rng.choice([-1, 1], len(offsets))
     for r in range(n):
         for d, v in zip(offsets, values):
-            if 0 <= r + d < n and (d == 0 or rng.random() > drop):
+            if 0 <= r + d < n and (d == 0 or r == n // 2 or rng.random() > drop):
                 idx.append(r + d)
                 val.append(v if d else 40.0)
         off.append(len(idx))
@@ -42,13 +43,14 @@ def test_products_and_solves_equal_crs(A, monkeypatch, nrhs, breaks):  # noqa: F
     if 0 not in wide:
         wide = sorted(wide[:31] + [0])
     systems = [banded(1, [0], rng), banded(700, [-20, -1, 0, 1, 20], rng), banded(257, wide, rng),
-               banded(63, [-7, 0, 7], rng, 0.0), banded(256, [0], rng), banded(513, [-300, -1, 0, 1, 300], rng)]
+               banded(63, [-7, 0, 7], rng, 0.0), banded(256, [0], rng), banded(713, [-300, -1, 0, 1, 300], rng)]
     if breaks != "none":
         systems[1] = break_one(systems[1], breaks, rng)
     C = A.Batch.from_crs(systems, nrhs)
     monkeypatch.setenv("ALP_HIP_BATCH_DIA", "0")
     P = A.Batch.from_crs(systems, nrhs)
     monkeypatch.delenv("ALP_HIP_BATCH_DIA")
+    assert (C.constant(), P.constant()) == (breaks == "none", False)
     x = rng.standard_normal((C.nrows, nrhs))
     X = A.Vector.from_numpy(x.ravel())
     Yc, Yp = A.Vector(C.nrows * nrhs), A.Vector(C.nrows * nrhs)
@@ -77,6 +79,7 @@ def test_infinities_reach_only_their_rows(A):  # noqa: F811
     rng = np.random.default_rng(5)
     systems = [banded(130, [-9, -1, 0, 1, 9], rng) for _ in range(3)]
     B = A.Batch.from_crs(systems, 8)
+    assert B.constant()
     x = rng.standard_normal((B.nrows, 8))
     x[130, 2] = np.inf
     x[259, 5] = np.nan
@@ -100,6 +103,7 @@ def test_no_memory_for_the_form(A, monkeypatch):  # noqa: F811
     monkeypatch.setenv("ALP_HIP_OPTIONAL_BYTES", "0")
     P = A.Batch.from_crs(systems, 4)
     monkeypatch.delenv("ALP_HIP_OPTIONAL_BYTES")
+    assert (C.constant(), P.constant()) == (True, False)
     x = A.Vector.from_numpy(rng.standard_normal(C.nrows * 4))
     got = []
     for B in (C, P):
